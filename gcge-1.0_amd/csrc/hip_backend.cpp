@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdarg>
@@ -16,6 +17,7 @@
 #include <cstdlib>
 #include <cstddef>
 #include <cstring>
+#include <thread>
 #include <vector>
 
 #include "gcge_app_hip.h"
@@ -24,6 +26,8 @@
 namespace gh {
 void launch_rowidx(HIP_MAT *A);
 void launch_to_f32(int64_t n, const double *a, float *b);
+// rows of a lexicographically numbered box grid brick by brick (hip_order.cpp)
+bool grid_bricks(int n, const int *rowptr, const int *col, std::vector<int> &order, int dims[3]);
 
 // ------------------------------------------------------------ error latch
 static int g_err = 0;
@@ -398,6 +402,7 @@ static bool mat_ok(HIP_MAT *A, MV *x, const char *what)
 using namespace gh;
 
 // ====================================================================== matrices
+constexpr int kHaloRows = 256;  // rows of a staged block (the workgroup of k_spmm_halo)
 static int pick_gather_rows(int n, const int *rowptr, const int *col);
 static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col);
 
@@ -457,7 +462,8 @@ extern "C" HIP_MAT *HIP_MatCreateFromCSR(GCGE_INT nrows, GCGE_INT ncols, GCGE_IN
         ok = check(hipMalloc((void **)&A->long_rows, sizeof(int) * A->nlong), "hipMalloc long_rows") &&
              check(hipMemcpy(A->long_rows, longs.data(), sizeof(int) * A->nlong, hipMemcpyHostToDevice),
                    "H2D long_rows");
-    if (ok && !A->gather_rows) ok = build_halo(A, rowptr, col);
+    if (ok && A->gather_rows != 1) ok = build_halo(A, rowptr, col);
+    if (A->gather_rows == 2) A->gather_rows = A->halo ? 0 : 1;
     if (!ok) {
         HIP_MatDestroy(&A);
         return nullptr;
@@ -466,49 +472,175 @@ extern "C" HIP_MAT *HIP_MatCreateFromCSR(GCGE_INT nrows, GCGE_INT ncols, GCGE_IN
     return A;
 }
 
-// Staged row blocks of k_spmm_halo: for each 256-row block, the rows its
-// entries read besides its own (ascending), and every entry's LDS slot.
-// Chosen for the column-gather layout when the blocks are compact: on
-// average a block reads at most as many other rows as it owns, and no block
-// more than kHaloCap - 256 (a grid in tile order reads its surface, about
-// 0.9 times its rows; the natural order of a 3-D grid reads whole planes,
-// 2.4 times, where the direct gather of k_spmm is as fast).
-// GCGE_HIP_SPMM_GATHER=halo takes it whenever it fits, =columns or =rows
-// never.  Rows longer than kLongRow (k_spmm_long) are left out.
+// Rows of the staged blocks, 256 positions each: position i holds row
+// order[i] (-1: none) and row r sits at position pos[r]; both null: row =
+// position < n.
+struct BlockRows {
+    int n, nblk;
+    const int *order, *pos;
+    int row(int i) const { return order ? order[i] : i < n ? i : -1; }
+    int at(int r) const { return pos ? pos[r] : r; }
+};
+
+// The rows besides its own that block b reads, ascending, and (with lcol)
+// every entry's slot; false when they exceed the LDS slots.
+static bool block_extras(int b, const BlockRows &br, const int *rowptr, const int *col, std::vector<int> &ext,
+                         unsigned short *lcol)
+{
+    const int p0 = b * kHaloRows;
+    const auto slot = [&](int c) {
+        const int p = br.at(c) - p0;
+        return p >= 0 && p < kHaloRows ? p : -1;
+    };
+    const auto entries = [&](auto f) {
+        for (int i = p0; i < p0 + kHaloRows; i++) {
+            const int r = br.row(i);
+            if (r < 0 || rowptr[r + 1] - rowptr[r] > kLongRow) continue;
+            for (int q = rowptr[r]; q < rowptr[r + 1]; q++) f(q);
+        }
+    };
+    ext.clear();
+    entries([&](int q) {
+        if (slot(col[q]) < 0) ext.push_back(col[q]);
+    });
+    std::sort(ext.begin(), ext.end());
+    ext.erase(std::unique(ext.begin(), ext.end()), ext.end());
+    if ((int)ext.size() > kHaloCap - kHaloRows) return false;
+    if (!lcol) return true;
+    entries([&](int q) {
+        const int s = slot(col[q]);
+        lcol[q] = (unsigned short)(
+            s >= 0 ? s : kHaloRows + (int)(std::lower_bound(ext.begin(), ext.end(), col[q]) - ext.begin()));
+    });
+    return true;
+}
+
+// Other rows per own row over 48 blocks spread over the matrix by the golden
+// ratio, so that no grid's period meets them (infinite when one of them
+// exceeds the LDS slots).
+static double sampled_extras(const BlockRows &br, const int *rowptr, const int *col)
+{
+    std::vector<int> ext;
+    double rows = 0.0, extra = 0.0;
+    for (int i = 0; i < 48; i++) {
+        const double f = i * 0.6180339887498949;
+        const int b = std::min(br.nblk - 1, (int)((f - std::floor(f)) * br.nblk));
+        if (!block_extras(b, br, rowptr, col, ext, nullptr)) return INFINITY;
+        for (int i = b * kHaloRows; i < (b + 1) * kHaloRows; i++) rows += br.row(i) >= 0;
+        extra += (double)ext.size();
+    }
+    return extra / rows;
+}
+
+// Runs f(part, parts) for every part on its own host thread (at most 8; the
+// caller's thread alone when threads cannot be had).
+template <typename F>
+static void host_parallel(int parts, F f)
+{
+    std::vector<std::thread> th;
+    int started = 1;
+    try {
+        for (; started < parts; started++) th.emplace_back(f, started, parts);
+    } catch (...) {
+    }
+    f(0, parts);
+    for (int p = started; p < parts; p++) f(p, parts);
+    for (std::thread &x : th) x.join();
+}
+
+// Staged row blocks of k_spmm_halo: for each block of up to 256 rows, the
+// rows its entries read besides its own (ascending), and every entry's LDS
+// slot.  A block is 256 consecutive rows, or a brick of a box grid numbered
+// lexicographically, whose consecutive rows read whole neighbouring lines and
+// planes (2.0 other rows per row in 2-D, 2.3 to 3 in 3-D).  Bricks are taken
+// for 3-D grids whose lines start on 128-byte boundaries (16 cells) or that
+// are small; on others the bricks' runs share their cache lines with other
+// blocks, and writing Y in parts of lines costs the kernels that follow what
+// the SpMM saves.  2-D grids, where bricks gain least, keep consecutive rows
+// and with them the direct gather's summation order of the fused dots (an
+// FP64 solve takes the same course).  One block CG step (SpMM with dots,
+// residual, search; FP64, ms: direct gather k_spmm / consecutive rows /
+// bricks; 35 columns up to 112^3, then 30):
+//   70^3  0.239 0.220 0.217   101^3 0.691 0.656 0.707   112^3 0.941 0.899 0.870
+//   130^3 1.302 1.248 1.307   160^3 2.431 2.389 2.238   999^2 0.558 0.516 0.502
+// FP32 products keep the direct gather (halo_f32 = 0) where it is as fast:
+//   70^3  0.123 0.108 0.106   101^3 0.341 0.340 0.337   112^3 0.460 0.461 0.459
+//   150^3 0.981 1.012 0.978   160^3 1.176 1.215 1.108   999^2 0.267 0.263 0.249
+// Other rows per own row, over all blocks, that are accepted:
+// - 1.8 for rows of up to 8 entries on average: each costs about a third of
+//   an own row's time, and k_spmm breaks even near 1.9 in FP32 (101^3 in tile
+//   order, 35 columns, 1.25 other rows: 0.116 against 0.127 ms; 0.201 against
+//   0.284 in FP64); 3.2 on a grid, where they come in runs (FP64 above);
+// - avg / 4 for rows of 8 to 28 entries on average, which would gather from a
+//   row-major copy of X otherwise (gather_rows 2; 27-point matrix of a 96^3
+//   grid, 50 FP64 columns: 0.45 ms in tile order, 0.68 with the natural
+//   order's 3.1 other rows, 2.1 gathered).
+// No block's may exceed kHaloCap - 256.  GCGE_HIP_SPMM_GATHER=halo takes
+// consecutive rows whenever they fit, =columns or =rows never.  Rows longer
+// than kLongRow (k_spmm_long) are left out.
 static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col)
 {
     const char *e = getenv("GCGE_HIP_SPMM_GATHER");
     const bool forced = e && !strcmp(e, "halo");
     if (e && !forced) return true;
-    const int n = A->n, R = 256, nblk = (n + R - 1) / R;
-    std::vector<int> hptr((size_t)nblk + 1, 0), hcol, ext;
-    std::vector<unsigned short> lcol((size_t)std::max(1, A->nnz), 0);
-    int most = 0;
-    for (int b = 0; b < nblk; b++) {
-        const int r0 = b * R, r1 = std::min(n, r0 + R);
-        ext.clear();
-        for (int r = r0; r < r1; r++) {
-            if (rowptr[r + 1] - rowptr[r] > kLongRow) continue;
-            for (int q = rowptr[r]; q < rowptr[r + 1]; q++)
-                if (col[q] < r0 || col[q] >= r1) ext.push_back(col[q]);
-        }
-        std::sort(ext.begin(), ext.end());
-        ext.erase(std::unique(ext.begin(), ext.end()), ext.end());
-        if ((int)ext.size() > kHaloCap - R) return true;  // too wide for LDS: keep k_spmm
-        most = std::max(most, (int)ext.size());
-        for (int r = r0; r < r1; r++) {
-            if (rowptr[r + 1] - rowptr[r] > kLongRow) continue;
-            for (int q = rowptr[r]; q < rowptr[r + 1]; q++) {
-                const int c = col[q];
-                lcol[q] = (unsigned short)((c >= r0 && c < r1)
-                                               ? c - r0
-                                               : R + (int)(std::lower_bound(ext.begin(), ext.end(), c) - ext.begin()));
+    const int n = A->n;
+    const double avg = (double)A->nnz / n;
+    const bool longer = avg > 8.0;
+    double limit = !longer ? 1.8 : avg <= 28.0 ? avg / 4.0 : 0.0;
+    std::vector<int> order, pos;
+    BlockRows br{n, (n + kHaloRows - 1) / kHaloRows, nullptr, nullptr};
+    bool f32 = true;
+    if (!forced) {
+        if (limit == 0.0) return true;
+        double h = sampled_extras(br, rowptr, col);
+        if (h > 1.3 && grid_bricks(n, rowptr, col, order, A->brick_dims)) {
+            const int *d = A->brick_dims;
+            const bool flat = d[2] == 1, small = n < 500000;
+            if (!longer) limit = 3.2;
+            if (!flat && (small || d[0] % 16 == 0)) {
+                pos.resize((size_t)n);
+                for (size_t i = 0; i < order.size(); i++)
+                    if (order[i] >= 0) pos[order[i]] = (int)i;
+                br = {n, (int)(order.size() / kHaloRows), order.data(), pos.data()};
+                h = sampled_extras(br, rowptr, col);
+                f32 = longer || small || d[0] % 32 == 0;
+            } else {
+                f32 = longer || flat || h <= 1.8;
             }
         }
-        hcol.insert(hcol.end(), ext.begin(), ext.end());
-        hptr[b + 1] = (int)hcol.size();
-        if (!forced && (int64_t)hcol.size() > (int64_t)n) return true;  // not compact: keep k_spmm
+        if (h > 1.2 * limit) return true;
     }
+    const int nblk = br.nblk;
+    const int parts = std::max(1, std::min({8, nblk / 64, (int)std::thread::hardware_concurrency()}));
+    std::vector<int> hptr((size_t)nblk + 1, 0), most(parts, 0);
+    std::vector<std::vector<int>> lists(parts);
+    std::vector<unsigned short> lcol((size_t)std::max(1, A->nnz), 0);
+    std::atomic<bool> wide{false};
+    host_parallel(parts, [&](int part, int nparts) {
+        try {
+            std::vector<int> ext;
+            const int b1 = (int)((int64_t)nblk * (part + 1) / nparts);
+            for (int b = (int)((int64_t)nblk * part / nparts); b < b1 && !wide; b++) {
+                if (!block_extras(b, br, rowptr, col, ext, lcol.data())) wide = true;
+                most[part] = std::max(most[part], (int)ext.size());
+                lists[part].insert(lists[part].end(), ext.begin(), ext.end());
+                hptr[b + 1] = (int)ext.size();
+            }
+        } catch (...) {
+            wide = true;  // out of host memory: keep the other layouts
+        }
+    });
+    if (wide) return true;
+    int64_t total = 0;
+    for (int b = 0; b < nblk; b++) {
+        total += hptr[b + 1];
+        if (total > INT32_MAX) return true;
+        hptr[b + 1] = (int)total;
+    }
+    if (!forced && (double)total > limit * n) return true;
+    std::vector<int> hcol;
+    hcol.reserve((size_t)total);
+    for (const std::vector<int> &l : lists) hcol.insert(hcol.end(), l.begin(), l.end());
     const size_t nh = std::max<size_t>(1, hcol.size());
     bool ok = check(hipMalloc((void **)&A->halo_ptr, sizeof(int) * hptr.size()), "hipMalloc halo_ptr") &&
               check(hipMalloc((void **)&A->halo_col, sizeof(int) * nh), "hipMalloc halo_col") &&
@@ -520,18 +652,26 @@ static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col)
          check(hipMemcpy(A->lcol, lcol.data(), sizeof(unsigned short) * lcol.size(), hipMemcpyHostToDevice),
                "H2D lcol");
     if (!ok) return false;
+    if (br.order) {
+        ok = check(hipMalloc((void **)&A->brick_rows, sizeof(int) * order.size()), "hipMalloc brick_rows") &&
+             check(hipMemcpy(A->brick_rows, br.order, sizeof(int) * order.size(), hipMemcpyHostToDevice), "H2D bricks");
+        if (!ok) return false;
+    }
     A->halo = 1;
-    A->halo_cap = ((R + most + 31) / 32) * 32;
-    A->halo_bytes = 4.0 * (double)(hptr.size() + nh) + 2.0 * (double)lcol.size();
+    A->halo_f32 = f32;
+    A->halo_blocks = nblk;
+    A->halo_cap = ((kHaloRows + *std::max_element(most.begin(), most.end()) + 31) / 32) * 32;
+    A->halo_bytes = 4.0 * (double)(hptr.size() + nh + (br.order ? order.size() : 0)) + 2.0 * (double)lcol.size();
     g_ctx.dev_bytes += A->halo_bytes;
     return true;
 }
 
 // Gather layout of the SpMM.  The row-major path is used when
-// - the rows average more than 8 stored entries: the column-major kernel
-//   then cannot stage a 256-row workgroup's entries in LDS and each thread
-//   reads its own row's indices and values, 64 cache lines per load (the
-//   27-point mass matrix: 3-7x slower SpMM, 15-20x slower residual check);
+// - the rows average more than 8 stored entries and do not fit staged blocks
+//   (returns 2, build_halo decides): the column-major kernel then cannot
+//   stage a 256-row workgroup's entries in LDS and each thread reads its own
+//   row's indices and values, 64 cache lines per load (the 27-point mass
+//   matrix: 3-7x slower SpMM, 15-20x slower residual check);
 // - or the column indices scatter: a wavefront of the column-major kernel
 //   reads, per stored entry and column, the cache lines its 64 rows' column
 //   indices fall in; a stencil's rows share a few lines (about 0.03 distinct
@@ -545,7 +685,7 @@ static int pick_gather_rows(int n, const int *rowptr, const int *col)
     const char *e = getenv("GCGE_HIP_SPMM_GATHER");
     if (e && !strcmp(e, "rows")) return 1;
     if (e && (!strcmp(e, "columns") || !strcmp(e, "halo"))) return 0;
-    if ((double)rowptr[n] > 8.0 * n) return 1;
+    if ((double)rowptr[n] > 8.0 * n) return 2;
     const int nb = n / 64;
     if (nb == 0) return 0;
     const int step = std::max(1, nb / 2048);
@@ -807,6 +947,7 @@ extern "C" void HIP_MatDestroy(HIP_MAT **mat)
         if (A->halo_ptr) (void)hipFree(A->halo_ptr);
         if (A->halo_col) (void)hipFree(A->halo_col);
         if (A->lcol) (void)hipFree(A->lcol);
+        if (A->brick_rows) (void)hipFree(A->brick_rows);
         delete[] A->perm_h;
         delete[] A->iperm_h;
         delete[] A->nzmap_h;

@@ -69,13 +69,17 @@ struct HIP_MAT_ {
     int gather_rows;  // SpMM gathers from a row-major copy of X (scattered column indices)
     double row_abs_max;  // max_i sum_j |a_ij| (Gershgorin bound of ||A||_2)
     // staged-row-block SpMM (k_spmm_halo), chosen at creation when every
-    // 256-row block reads at most kHaloCap - 256 rows besides its own
+    // block of up to 256 rows reads at most kHaloCap - 256 rows besides its own
     int halo;                 // 1: SpMM by k_spmm_halo
+    int halo_f32;             // 1: FP32 products too (else k_spmm)
+    int halo_blocks;          // row blocks
     int halo_cap;             // LDS slots per column: 256 own rows + the most extras of any block (rounded)
-    int *halo_ptr;            // device, nblk+1: each block's extras in halo_col
+    int *halo_ptr;            // device, halo_blocks+1: each block's extras in halo_col
     int *halo_col;            // device: the other rows a block's entries read, ascending
-    unsigned short *lcol;     // device, nnz: each entry's slot (own row r0+i -> i, extra j -> 256+j)
-    double halo_bytes;        // device bytes of the three arrays
+    unsigned short *lcol;     // device, nnz: each entry's slot (i-th own row -> i, extra j -> 256+j)
+    int *brick_rows;          // device, 256 per block: its rows, -1 for none (null: 256 consecutive rows)
+    int brick_dims[3];        // box grid of brick_rows: matrices of equal dims have the same blocks
+    double halo_bytes;        // device bytes of these arrays
     // row order (HIP_MatCreateFromCSROrdered): the device matrix is
     // P A P^T; multivectors created from it hold rows in the same order and
     // are permuted at host transfers.  Host arrays, null when unordered.

@@ -379,63 +379,123 @@ __global__ __launch_bounds__(kSpmmRows) void k_spmm_long(const int *__restrict__
 // block at matrix creation, sorted) -- for KC columns into LDS, with
 // coalesced loads, and the rows then read their entries' values from LDS
 // through 16-bit local column indices (also built at creation).  Each row's
-// first kHaloMaxE entries (local indices and values) stay in registers for all
-// columns.  Every sum still runs over the row in CSR order from 0, so Y is
-// bit-identical to k_spmm's.  Rows longer than long_thr are left to
-// k_spmm_long.  Row blocks are numbered so that each XCD walks a contiguous
-// range of rows (a stencil's plane neighbours stay in its L2).
-constexpr int kHaloMaxE = 8;
+// first ME entries (local indices in pairs, and values) stay in registers for
+// all columns: 8 for stencils of up to 8 entries per row, 28 for the 27-point
+// matrices, whose products are then bound by LDS reads (27 x 8 bytes per row
+// and column) and not by re-reading 10 bytes per entry and pass.  With 28 in
+// FP64 the compiler's own choice is 207 registers and two wavefronts per
+// SIMD; three are asked for.  27-point matrix of a 96^3 grid, 50 columns:
+// 0.45 ms in FP64 and 0.25 in FP32, against 2.09 and 0.93 gathered from a
+// row-major copy of X (k_spmm_rows).  Every sum still runs over the row in CSR order from 0, so Y is bit-identical to
+// k_spmm's.  Rows longer than long_thr are left to k_spmm_long.  Row blocks
+// are numbered so that each XCD walks a contiguous range of rows (a stencil's
+// plane neighbours stay in its L2).
 
-// KC consecutive values of one LDS slot, moved as one vector
+// A slot holds KC consecutive columns of one X row.  Slots lie in planes of
+// 16 bytes (plane h: columns h * E .. h * E + E - 1 of every slot), so the
+// lanes of a wavefront that read neighbouring slots read consecutive 16-byte
+// words: with a slot's 32 bytes (FP64, KC = 4) side by side the 16-byte reads
+// step over every second word and each meets a bank twice.
 template <typename T, int KC>
-struct alignas(KC * sizeof(T) >= 16 ? 16 : KC * sizeof(T)) SlotVec {
-    T v[KC];
+struct Slots {
+    static constexpr int NP = KC * (int)sizeof(T) > 16 ? KC * (int)sizeof(T) / 16 : 1;
+    static constexpr int E = KC / NP;
+    struct alignas(E * sizeof(T)) Part {
+        T v[E];
+    };
+    struct Row {
+        T v[KC];
+    };
+    __device__ static __forceinline__ Row get(const Part *s, int cap, int slot)
+    {
+        Row x;
+#pragma unroll
+        for (int h = 0; h < NP; h++) {
+            const Part p = s[h * cap + slot];
+#pragma unroll
+            for (int e = 0; e < E; e++) x.v[h * E + e] = p.v[e];
+        }
+        return x;
+    }
+    __device__ static __forceinline__ void put(Part *s, int cap, int slot, const Row &x)
+    {
+#pragma unroll
+        for (int h = 0; h < NP; h++) {
+            Part p;
+#pragma unroll
+            for (int e = 0; e < E; e++) p.v[e] = x.v[h * E + e];
+            s[h * cap + slot] = p;
+        }
+    }
 };
 
-template <typename T, bool DOT, int KC>
-__global__ __launch_bounds__(kSpmmRows) void k_spmm_halo(int n, const int *__restrict__ rowptr,
+// The first ME entries of one row in registers: slots in pairs, values.
+template <typename T, int ME>
+struct RowHead {
+    unsigned lc[ME / 2];
+    T v[ME];
+    __device__ __forceinline__ void load(const unsigned short *__restrict__ lcol, const T *__restrict__ val, int s,
+                                         int cnt)
+    {
+#pragma unroll
+        for (int u = 0; u < ME; u += 2) {
+            const unsigned a = u < cnt ? lcol[s + u] : 0, b = u + 1 < cnt ? lcol[s + u + 1] : 0;
+            lc[u / 2] = a | (b << 16);
+            v[u] = u < cnt ? val[s + u] : T(0);
+            v[u + 1] = u + 1 < cnt ? val[s + u + 1] : T(0);
+        }
+    }
+    __device__ __forceinline__ int slot(int u) const
+    {
+        return (int)((u & 1) ? lc[u / 2] >> 16 : lc[u / 2] & 0xffffu);
+    }
+};
+
+// Extras of a block that each thread holds in registers one pass ahead; the
+// others load when their pass begins.
+template <int ME>
+constexpr int halo_prefetch = ME > 8 ? 2 : 1;
+
+template <typename T, bool DOT, int KC, int ME>
+__global__ __launch_bounds__(kSpmmRows, ME > 8 ? 3 : 1) void k_spmm_halo(int n, const int *__restrict__ rowptr,
                                                          const unsigned short *__restrict__ lcol,
-                                                         const T *__restrict__ val, const int *__restrict__ hptr,
-                                                         const int *__restrict__ hcol, const T *__restrict__ X,
-                                                         int64_t ldx, T *__restrict__ Y, int64_t ldy, int k,
-                                                         ColScalars g, double *__restrict__ partial, int nblk,
-                                                         int long_thr, int pstride, int hcap)
+                                                         const T *__restrict__ val, const int *__restrict__ brows,
+                                                         const int *__restrict__ hptr, const int *__restrict__ hcol,
+                                                         const T *__restrict__ X, int64_t ldx, T *__restrict__ Y,
+                                                         int64_t ldy, int k, ColScalars g,
+                                                         double *__restrict__ partial, int nblk, int long_thr,
+                                                         int pstride, int hcap)
 {
-    // s_x holds slot-major KC-column rows: slot j, column cc at s_x[j * KC + cc]
+    using S = Slots<T, KC>;
+    using Row = typename S::Row;
+    constexpr int NE = halo_prefetch<ME>;
     extern __shared__ __align__(16) unsigned char halo_smem[];
-    T *s_x = reinterpret_cast<T *>(halo_smem);                    // [hcap][KC]
-    int *s_h = reinterpret_cast<int *>(s_x + (size_t)KC * hcap);  // [hcap - kSpmmRows]
+    typename S::Part *sx = reinterpret_cast<typename S::Part *>(halo_smem);  // [NP][hcap]
     __shared__ double sdot[DOT ? kMaxCols : 1][4];
     const int per = (int)(gridDim.x >> 3);
     const int blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (blk >= nblk) return;  // uniform per workgroup (grid rounded up to 8)
-    const int tid = threadIdx.x, r0 = blk * kSpmmRows, r = r0 + tid;
-    const int nown = min(kSpmmRows, n - r0);
+    const int tid = threadIdx.x, p = blk * kSpmmRows + tid;
+    const int r = brows ? brows[p] : p < n ? p : -1;
     const int h0 = hptr[blk], nh = hptr[blk + 1] - h0;
-    for (int j = tid; j < nh; j += kSpmmRows) s_h[j] = hcol[h0 + j];
+    const int *hc = hcol + h0;
     int s = 0, t = 0;
-    if (r < n) {
+    if (r >= 0) {
         s = rowptr[r];
         t = rowptr[r + 1];
     }
-    const bool active = r < n && t - s <= long_thr;  // long rows: k_spmm_long
+    const bool active = r >= 0 && t - s <= long_thr;  // long rows: k_spmm_long
     const int cnt = active ? t - s : 0;
-    int lc[kHaloMaxE];
-    T v[kHaloMaxE];
-#pragma unroll
-    for (int u = 0; u < kHaloMaxE; u++) {
-        lc[u] = u < cnt ? (int)lcol[s + u] : 0;
-        v[u] = u < cnt ? val[s + u] : T(0);
-    }
+    RowHead<T, ME> row;
+    row.load(lcol, val, s, cnt);
     const int lane = tid & 63, wid = tid >> 6;
-    using SV = SlotVec<T, KC>;
-    SV *sv = reinterpret_cast<SV *>(s_x);
-    __syncthreads();
-    // the own row and the first extra slot of this thread for the next KC
+    // the own row and the first NE extras of this thread for the next KC
     // columns are loaded into registers while the current columns are
     // multiplied, so that a workgroup's loads overlap its own work
-    const int row1 = tid < nh ? s_h[tid] : 0;
-    SV pown, pext;
+    int erow[NE];
+#pragma unroll
+    for (int i = 0; i < NE; i++) erow[i] = tid + i * kSpmmRows < nh ? hc[tid + i * kSpmmRows] : 0;
+    Row pown, pext[NE];
     auto xcols = [&](int c0, const T *(&xc)[KC]) {
 #pragma unroll
         for (int cc = 0; cc < KC; cc++) {
@@ -446,49 +506,54 @@ __global__ __launch_bounds__(kSpmmRows) void k_spmm_halo(int n, const int *__res
     auto prefetch = [&](int c0) {
         const T *xc[KC];
         xcols(c0, xc);
-        if (tid < nown) {
+        if (r >= 0) {
 #pragma unroll
-            for (int cc = 0; cc < KC; cc++) pown.v[cc] = xc[cc][r0 + tid];
+            for (int cc = 0; cc < KC; cc++) pown.v[cc] = xc[cc][r];
         }
-        if (tid < nh) {
 #pragma unroll
-            for (int cc = 0; cc < KC; cc++) pext.v[cc] = xc[cc][row1];
-        }
+        for (int i = 0; i < NE; i++)
+            if (tid + i * kSpmmRows < nh) {
+#pragma unroll
+                for (int cc = 0; cc < KC; cc++) pext[i].v[cc] = xc[cc][erow[i]];
+            }
     };
     prefetch(0);
     for (int c0 = 0; c0 < k; c0 += KC) {
-        const T *xc[KC];
-        xcols(c0, xc);
-        if (tid < nown) sv[tid] = pown;
-        if (tid < nh) sv[kSpmmRows + tid] = pext;
-        // extras beyond one per thread (blocks with more than 256) load here
-        for (int j = tid + kSpmmRows; j < nh; j += kSpmmRows) {
-            const int row = s_h[j];
-            SV w;
+        if (r >= 0) S::put(sx, hcap, tid, pown);
 #pragma unroll
-            for (int cc = 0; cc < KC; cc++) w.v[cc] = xc[cc][row];
-            sv[kSpmmRows + j] = w;
+        for (int i = 0; i < NE; i++)
+            if (tid + i * kSpmmRows < nh) S::put(sx, hcap, kSpmmRows + tid + i * kSpmmRows, pext[i]);
+        if (nh > NE * kSpmmRows) {
+            const T *xc[KC];
+            xcols(c0, xc);
+            for (int j = tid + NE * kSpmmRows; j < nh; j += kSpmmRows) {
+                const int er = hc[j];
+                Row w;
+#pragma unroll
+                for (int cc = 0; cc < KC; cc++) w.v[cc] = xc[cc][er];
+                S::put(sx, hcap, kSpmmRows + j, w);
+            }
         }
+        const Row xo = pown;
         __syncthreads();
         if (c0 + KC < k) prefetch(c0 + KC);
         T acc[KC];
 #pragma unroll
         for (int cc = 0; cc < KC; cc++) acc[cc] = T(0);
 #pragma unroll
-        for (int u = 0; u < kHaloMaxE; u++)
+        for (int u = 0; u < ME; u++)
             if (u < cnt) {
-                const SV x = sv[lc[u]];
+                const Row x = S::get(sx, hcap, row.slot(u));
 #pragma unroll
-                for (int cc = 0; cc < KC; cc++) acc[cc] = acc[cc] + v[u] * x.v[cc];
+                for (int cc = 0; cc < KC; cc++) acc[cc] = acc[cc] + row.v[u] * x.v[cc];
             }
-        for (int e = s + kHaloMaxE; e < s + cnt; e++) {
-            const SV x = sv[lcol[e]];
+        for (int e = s + ME; e < s + cnt; e++) {
+            const Row x = S::get(sx, hcap, lcol[e]);
             const T ve = val[e];
 #pragma unroll
             for (int cc = 0; cc < KC; cc++) acc[cc] = acc[cc] + ve * x.v[cc];
         }
         double d[KC];
-        const SV xo = sv[tid];  // own row (written by this thread when active)
 #pragma unroll
         for (int cc = 0; cc < KC; cc++) {
             const int c = c0 + cc;
@@ -501,7 +566,7 @@ __global__ __launch_bounds__(kSpmmRows) void k_spmm_halo(int n, const int *__res
             const int c = c0 + (lane >> (6 - L));
             if ((lane & ((64 >> L) - 1)) == 0 && c < k) sdot[c][wid] = colsum;
         }
-        __syncthreads();  // the next chunk overwrites s_x
+        __syncthreads();  // the next chunk overwrites sx
     }
     if (DOT) {
         for (int c = tid; c < k; c += kSpmmRows)
@@ -804,6 +869,157 @@ __global__ __launch_bounds__(kSpmmRows) void k_residual(int n, const int *__rest
     const int nb = gridDim.x;
     for (int q = threadIdx.x; q < 3 * k; q += kSpmmRows)
         partial[(int64_t)q * nb + blk] = (sred[q][0] + sred[q][1]) + (sred[q][2] + sred[q][3]);
+}
+
+// r = A x - lambda B x (Bx = x when B is absent) for matrices in staged row
+// blocks: the X rows a 256-row block reads go through LDS as in k_spmm_halo
+// -- own rows, A's extras, then B's extras -- for KC columns at a time, and
+// both row sums are formed in FP64 from the staged values in CSR order from
+// 0, as in k_residual.  One pass over X and the matrices; as in k_spmm_halo
+// LDS reads and the staging of other rows bound it.  FP64, measured: 7-point
+// 160^3, B = I, 100 columns 1.37 ms (k_residual 2.97, X read once 0.55); 96^3
+// with the 27-point B, 50 columns 0.59 ms (k_residual_rows 2.69).
+template <typename TX, bool HASB, int KC, int MEA, int MEB>
+__global__ __launch_bounds__(kSpmmRows, HASB ? 2 : 3) void k_residual_halo(
+    int n, const int *__restrict__ arp, const unsigned short *__restrict__ alcol, const double *__restrict__ aval,
+    const int *__restrict__ brows, const int *__restrict__ ahptr, const int *__restrict__ ahcol,
+    const int *__restrict__ brp,
+    const unsigned short *__restrict__ blcol, const double *__restrict__ bval, const int *__restrict__ bhptr,
+    const int *__restrict__ bhcol, const TX *__restrict__ X, int64_t ldx, int k, ColScalars g,
+    double *__restrict__ partial, int nblk, int cap)
+{
+    using S = Slots<TX, KC>;
+    using Row = typename S::Row;
+    extern __shared__ __align__(16) unsigned char halo_smem[];
+    typename S::Part *sx = reinterpret_cast<typename S::Part *>(halo_smem);  // [NP][cap]
+    __shared__ double sred[3 * kMaxCols][4];
+    const int per = (int)(gridDim.x >> 3);
+    const int blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (blk >= nblk) return;  // uniform per workgroup (grid rounded up to 8)
+    const int tid = threadIdx.x, p = blk * kSpmmRows + tid;
+    const int r = brows ? brows[p] : p < n ? p : -1;
+    const int lane = tid & 63, wid = tid >> 6;
+    const bool active = r >= 0;
+    const int nha = ahptr[blk + 1] - ahptr[blk];
+    const int nhb = HASB ? bhptr[blk + 1] - bhptr[blk] : 0;
+    const int *hca = ahcol + ahptr[blk];
+    const int *hcb = HASB ? bhcol + bhptr[blk] : nullptr;
+    int as = 0, acnt = 0, bs = 0, bcnt = 0;
+    if (active) {
+        as = arp[r];
+        acnt = arp[r + 1] - as;
+        if (HASB) {
+            bs = brp[r];
+            bcnt = brp[r + 1] - bs;
+        }
+    }
+    RowHead<double, MEA> ra;
+    RowHead<double, HASB ? MEB : 2> rb;
+    ra.load(alcol, aval, as, acnt);
+    if (HASB) rb.load(blcol, bval, bs, bcnt);
+    // slot of a B entry: its extras follow A's
+    auto bslot = [&](int sl) { return sl < kSpmmRows ? sl : sl + nha; };
+    auto rowof = [&](int j) { return j < nha ? hca[j] : hcb[j - nha]; };
+    const int nh = nha + nhb;
+    constexpr int NE = HASB ? halo_prefetch<MEB> + 1 : halo_prefetch<MEA>;
+    int erow[NE];
+#pragma unroll
+    for (int i = 0; i < NE; i++) erow[i] = tid + i * kSpmmRows < nh ? rowof(tid + i * kSpmmRows) : 0;
+    Row pown, pext[NE];
+    auto xcols = [&](int c0, const TX *(&xc)[KC]) {
+#pragma unroll
+        for (int cc = 0; cc < KC; cc++) xc[cc] = X + (int64_t)g.idx[min(c0 + cc, k - 1)] * ldx;
+    };
+    auto prefetch = [&](int c0) {
+        const TX *xc[KC];
+        xcols(c0, xc);
+        if (active) {
+#pragma unroll
+            for (int cc = 0; cc < KC; cc++) pown.v[cc] = xc[cc][r];
+        }
+#pragma unroll
+        for (int i = 0; i < NE; i++)
+            if (tid + i * kSpmmRows < nh) {
+#pragma unroll
+                for (int cc = 0; cc < KC; cc++) pext[i].v[cc] = xc[cc][erow[i]];
+            }
+    };
+    prefetch(0);
+    for (int c0 = 0; c0 < k; c0 += KC) {
+        if (active) S::put(sx, cap, tid, pown);
+#pragma unroll
+        for (int i = 0; i < NE; i++)
+            if (tid + i * kSpmmRows < nh) S::put(sx, cap, kSpmmRows + tid + i * kSpmmRows, pext[i]);
+        if (nh > NE * kSpmmRows) {
+            const TX *xc[KC];
+            xcols(c0, xc);
+            for (int j = tid + NE * kSpmmRows; j < nh; j += kSpmmRows) {
+                const int er = rowof(j);
+                Row w;
+#pragma unroll
+                for (int cc = 0; cc < KC; cc++) w.v[cc] = xc[cc][er];
+                S::put(sx, cap, kSpmmRows + j, w);
+            }
+        }
+        const Row xo = pown;
+        __syncthreads();
+        if (c0 + KC < k) prefetch(c0 + KC);
+        double ax[KC], bx[KC];
+#pragma unroll
+        for (int cc = 0; cc < KC; cc++) ax[cc] = bx[cc] = 0.0;
+#pragma unroll
+        for (int u = 0; u < MEA; u++)
+            if (u < acnt) {
+                const Row x = S::get(sx, cap, ra.slot(u));
+#pragma unroll
+                for (int cc = 0; cc < KC; cc++) ax[cc] = ax[cc] + ra.v[u] * (double)x.v[cc];
+            }
+        for (int e = as + MEA; e < as + acnt; e++) {
+            const Row x = S::get(sx, cap, alcol[e]);
+            const double ve = aval[e];
+#pragma unroll
+            for (int cc = 0; cc < KC; cc++) ax[cc] = ax[cc] + ve * (double)x.v[cc];
+        }
+        if (HASB) {
+#pragma unroll
+            for (int u = 0; u < MEB; u++)
+                if (u < bcnt) {
+                    const Row x = S::get(sx, cap, bslot(rb.slot(u)));
+#pragma unroll
+                    for (int cc = 0; cc < KC; cc++) bx[cc] = bx[cc] + rb.v[u] * (double)x.v[cc];
+                }
+            for (int e = bs + MEB; e < bs + bcnt; e++) {
+                const Row x = S::get(sx, cap, bslot(blcol[e]));
+                const double ve = bval[e];
+#pragma unroll
+                for (int cc = 0; cc < KC; cc++) bx[cc] = bx[cc] + ve * (double)x.v[cc];
+            }
+        }
+        double drr[KC], dxx[KC], dbb[KC];
+#pragma unroll
+        for (int cc = 0; cc < KC; cc++) {
+            const int c = c0 + cc;
+            const bool live = active && c < k;
+            const double xr = live ? (double)xo.v[cc] : 0.0;
+            const double b = HASB ? bx[cc] : xr;
+            const double res = live ? axpby_el<double>(-g.a[min(c, k - 1)], b, 1.0, ax[cc]) : 0.0;
+            drr[cc] = res * res;
+            dxx[cc] = xr * xr;
+            dbb[cc] = live ? b * b : 0.0;
+        }
+        constexpr int L = KC == 1 ? 0 : KC == 2 ? 1 : 2;
+        const double srr = wave_colsum<KC>(drr, lane), sxx = wave_colsum<KC>(dxx, lane);
+        const double sbb = HASB ? wave_colsum<KC>(dbb, lane) : sxx;
+        const int c = c0 + (lane >> (6 - L));
+        if ((lane & ((64 >> L) - 1)) == 0 && c < k) {
+            sred[3 * c + 0][wid] = srr;
+            sred[3 * c + 1][wid] = sxx;
+            sred[3 * c + 2][wid] = sbb;
+        }
+        __syncthreads();  // the next chunk overwrites sx
+    }
+    for (int q = tid; q < 3 * k; q += kSpmmRows)
+        partial[(int64_t)q * nblk + blk] = (sred[q][0] + sred[q][1]) + (sred[q][2] + sred[q][3]);
 }
 
 // r = A x - lambda B x (Bx = x when B is absent) on the row-major gather
@@ -1279,25 +1495,35 @@ static int halo_kc(const HIP_MAT *A, size_t elem)
     if (env_kc != kc)
         while (kc > 1 && (size_t)kc * A->halo_cap * elem > (size_t)env_lds) kc /= 2;
     // never beyond 56 KiB of dynamic LDS (the kernel adds 4 KiB of its own)
-    while (kc > 1 && (size_t)kc * A->halo_cap * elem + (size_t)A->halo_cap * 4 > (size_t)56 * 1024) kc /= 2;
+    while (kc > 1 && (size_t)kc * A->halo_cap * elem > (size_t)56 * 1024) kc /= 2;
     return kc;
 }
+
+// More than 8 entries per row on average: 28 of them held in registers by
+// the staged kernels, 8 otherwise.
+static bool long_average(const HIP_MAT *A) { return A->nnz > 8.0 * A->n; }
 
 template <typename T, bool DOT, int KC>
 static void spmm_halo_kc(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColScalars g, T *Yc, int64_t ldy,
                          int kc, double *partial, int nblk, int long_thr, int pstride)
 {
-    const size_t lds = (size_t)KC * A->halo_cap * sizeof(T) + (size_t)(A->halo_cap - kSpmmRows) * sizeof(int);
-    k_spmm_halo<T, DOT, KC><<<((nblk + 7) / 8) * 8, kSpmmRows, lds, ctx().stream>>>(
-        A->n, A->rowptr, A->lcol, val, A->halo_ptr, A->halo_col, Xc, ldx, Yc, ldy, kc, g, partial, nblk, long_thr,
-        pstride, A->halo_cap);
+    const size_t lds = (size_t)KC * A->halo_cap * sizeof(T);
+    const int grid = ((nblk + 7) / 8) * 8;
+    if (long_average(A))
+        k_spmm_halo<T, DOT, KC, 28><<<grid, kSpmmRows, lds, ctx().stream>>>(
+            A->n, A->rowptr, A->lcol, val, A->brick_rows, A->halo_ptr, A->halo_col, Xc, ldx, Yc, ldy, kc, g, partial,
+            nblk, long_thr, pstride, A->halo_cap);
+    else
+        k_spmm_halo<T, DOT, KC, 8><<<grid, kSpmmRows, lds, ctx().stream>>>(
+            A->n, A->rowptr, A->lcol, val, A->brick_rows, A->halo_ptr, A->halo_col, Xc, ldx, Yc, ldy, kc, g, partial,
+            nblk, long_thr, pstride, A->halo_cap);
 }
 
 template <typename T, bool DOT>
 static bool spmm_halo(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColScalars g, T *Yc, int64_t ldy,
                       int kc, double *out)
 {
-    const int nblk = (A->n + kSpmmRows - 1) / kSpmmRows;
+    const int nblk = A->halo_blocks;
     const int nlong = A->nlong, long_thr = nlong > 0 ? kLongRow : INT_MAX;
     const int pstride = nblk + (DOT ? nlong : 0);
     double *partial = nullptr;
@@ -1340,7 +1566,7 @@ static bool spmm_t(HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy,
             if (!spmm_rows<T, DOT>(A, val, Xc, ldx, g, Yc, ldy, kc, DOT ? out + c0 : nullptr)) return false;
             continue;
         }
-        if (A->halo) {
+        if (A->halo && (sizeof(T) == 8 || A->halo_f32)) {
             if (!spmm_halo<T, DOT>(A, val, Xc, ldx, g, Yc, ldy, kc, DOT ? out + c0 : nullptr)) return false;
             continue;
         }
@@ -1440,17 +1666,66 @@ static bool residual_rows(HIP_MAT *A, HIP_MAT *B, const T *X, int64_t ldx, ColSc
     return residual_rows_g<T, 2>(A, B, X, ldx, g, kc, out);
 }
 
+// Slots per column of k_residual_halo for A and B (or A alone), and columns
+// per pass: 4, or 2 where the slots would exceed 56 KiB of LDS (the kernel
+// adds 12).  0 when that kernel does not take them: both in staged blocks of
+// the same rows, no row for k_spmm_long, the slots within the 56 KiB.
+static int residual_halo_cap(const HIP_MAT *A, const HIP_MAT *B, size_t elem, int *kc)
+{
+    if (!A->halo || A->nlong > 0 || (B && (!B->halo || B->nlong > 0))) return 0;
+    if (B && (!A->brick_rows != !B->brick_rows ||
+              (A->brick_rows && !std::equal(A->brick_dims, A->brick_dims + 3, B->brick_dims))))
+        return 0;
+    const int cap = A->halo_cap + (B ? B->halo_cap - kSpmmRows : 0);
+    const size_t room = (size_t)56 * 1024;
+    *kc = cap * 4 * elem <= room ? 4 : 2;
+    return cap * 2 * elem <= room ? cap : 0;
+}
+
+template <typename T, bool HASB, int MEA, int MEB>
+static void residual_halo_launch(HIP_MAT *A, HIP_MAT *B, const T *X, int64_t ldx, int k, const ColScalars &g,
+                                 double *partial, int cap, int kc)
+{
+    const int nblk = A->halo_blocks, grid = ((nblk + 7) / 8) * 8;
+    const size_t lds = (size_t)cap * kc * sizeof(T);
+#define GH_RES(KC_)                                                                                             \
+    k_residual_halo<T, HASB, KC_, MEA, MEB><<<grid, kSpmmRows, lds, ctx().stream>>>(                            \
+        A->n, A->rowptr, A->lcol, A->val64, A->brick_rows, A->halo_ptr, A->halo_col,                            \
+        HASB ? B->rowptr : nullptr, HASB ? B->lcol : nullptr, HASB ? B->val64 : nullptr,                        \
+        HASB ? B->halo_ptr : nullptr, HASB ? B->halo_col : nullptr, X, ldx, k, g, partial, nblk, cap)
+    if (kc == 4) GH_RES(4);
+    else GH_RES(2);
+#undef GH_RES
+}
+
+template <typename T>
+static void residual_halo(HIP_MAT *A, HIP_MAT *B, const T *X, int64_t ldx, int k, const ColScalars &g,
+                          double *partial, int cap, int kc)
+{
+    const bool a28 = long_average(A), b28 = B && long_average(B);
+    if (!B && !a28) residual_halo_launch<T, false, 8, 8>(A, B, X, ldx, k, g, partial, cap, kc);
+    else if (!B) residual_halo_launch<T, false, 28, 8>(A, B, X, ldx, k, g, partial, cap, kc);
+    else if (!a28 && !b28) residual_halo_launch<T, true, 8, 8>(A, B, X, ldx, k, g, partial, cap, kc);
+    else if (!a28) residual_halo_launch<T, true, 8, 28>(A, B, X, ldx, k, g, partial, cap, kc);
+    else if (!b28) residual_halo_launch<T, true, 28, 8>(A, B, X, ldx, k, g, partial, cap, kc);
+    else residual_halo_launch<T, true, 28, 28>(A, B, X, ldx, k, g, partial, cap, kc);
+}
+
 template <typename T>
 static bool residual_t(HIP_MAT *A, HIP_MAT *B, const void *X, int64_t ldx, const int *idx, int k,
                        const double *lambda, double *rnorm, double *xnorm, double *bxnorm)
 {
-    const int nblk = (A->n + kSpmmRows - 1) / kSpmmRows;
     std::vector<double> tmp(3 * kMaxCols);
+    int hkc = 4;
+    const int cap = residual_halo_cap(A, B, sizeof(T), &hkc);
+    const int nblk = cap ? A->halo_blocks : (A->n + kSpmmRows - 1) / kSpmmRows;
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars g = make_scalars(kc, lambda + c0, nullptr, idx + c0);
-        // row gather when either matrix prefers it (B's rows must all be short)
-        if ((A->gather_rows || (B && B->gather_rows)) && (!B || B->nlong == 0) && kc >= 2) {
+        // row gather for scattered or long rows that cannot be staged (B's
+        // rows must all be short)
+        const bool rows = A->gather_rows || long_average(A) || (B && (B->gather_rows || long_average(B)));
+        if (!cap && rows && (!B || B->nlong == 0) && kc >= 2) {
             if (!residual_rows<T>(A, B, (const T *)X, ldx, g, kc, tmp.data())) return false;
             for (int j = 0; j < kc; j++) {
                 rnorm[c0 + j] = std::sqrt(tmp[3 * j + 0]);
@@ -1465,7 +1740,9 @@ static bool residual_t(HIP_MAT *A, HIP_MAT *B, const void *X, int64_t ldx, const
                               (double)kc * A->n * sizeof(T);
         {
             ProfScope ps(K_RESIDUAL, rbytes, 2.0 * kc * (double)(A->nnz + (B ? B->nnz : 0)));
-            if (B)
+            if (cap)
+                residual_halo<T>(A, B, (const T *)X, ldx, kc, g, partial, cap, hkc);
+            else if (B)
                 k_residual<T, true><<<nblk, kSpmmRows, 0, ctx().stream>>>(
                     A->n, A->rowptr, A->col, A->val64, B->rowptr, B->col, B->val64, (const T *)X, ldx, kc, g,
                     partial);

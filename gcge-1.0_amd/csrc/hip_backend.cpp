@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <climits>
 #include <cmath>
 #include <cstdarg>
@@ -128,12 +129,34 @@ double *host_buf(size_t count)
         g_ctx.hbuf = nullptr;
     }
     size_t want = std::max(bytes, (size_t)(1u << 20));
-    if (!check(hipHostMalloc((void **)&g_ctx.hbuf, want, hipHostMallocDefault), "hipHostMalloc")) {
+    // coherent: what a kernel has written with system scope is seen by the host
+    // while the kernel's stream is still busy
+    if (!check(hipHostMalloc((void **)&g_ctx.hbuf, want, hipHostMallocCoherent), "hipHostMalloc")) {
+        g_ctx.hbuf = nullptr;
         g_ctx.hbuf_bytes = 0;
         return nullptr;
     }
     g_ctx.hbuf_bytes = want;
     return g_ctx.hbuf;
+}
+
+unsigned long long *host_seq(size_t count, unsigned long long *next)
+{
+    if (!ensure_ctx()) return nullptr;
+    if (count > g_ctx.hseq_count) {
+        if (!sync()) return nullptr;
+        if (g_ctx.hseq) (void)hipHostFree(g_ctx.hseq);
+        g_ctx.hseq = nullptr;
+        g_ctx.hseq_count = 0;
+        const size_t want = std::max(count, (size_t)4096);
+        if (!check(hipHostMalloc((void **)&g_ctx.hseq, sizeof(*g_ctx.hseq) * want, hipHostMallocCoherent),
+                   "hipHostMalloc"))
+            return nullptr;
+        std::memset(g_ctx.hseq, 0, sizeof(*g_ctx.hseq) * want);  // below every number to come
+        g_ctx.hseq_count = want;
+    }
+    *next = ++g_ctx.seq;
+    return g_ctx.hseq;
 }
 
 // ------------------------------------------------------------ profiler
@@ -227,6 +250,35 @@ bool sync()
     if (!g_pending.empty() && g_prof_open == 0) prof_resolve();
     g_ctx.stage_off = 0;  // every staged copy has completed
     return ok;
+}
+
+// Reading the numbers from host memory costs about 6 us less per reduction
+// than a copy to the host and a stream synchronization (a kernel of 1,280
+// workgroups, the reduction of its 20 columns and the wait: 17.9 us with copy
+// and synchronization, 15.9 with synchronization alone, 11.8 so).  After 20 ms
+// without them the stream is synchronized instead, which also reports errors.
+// The profiler's events have to be complete for the host, so it synchronizes.
+bool wait_seq(size_t count, unsigned long long want)
+{
+    size_t i = 0;
+    const auto arrived = [&] {
+        while (i < count && __atomic_load_n(g_ctx.hseq + i, __ATOMIC_ACQUIRE) == want) i++;
+        return i == count;
+    };
+    if (g_pending.empty()) {
+        const auto t0 = std::chrono::steady_clock::now();
+        for (unsigned spin = 1; !arrived(); spin++) {
+            __builtin_ia32_pause();
+            if (spin % 4096 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) break;
+        }
+        if (i == count) {
+            g_ctx.stage_off = 0;  // copies staged before the launch have completed
+            return true;
+        }
+    }
+    if (!sync()) return false;
+    if (!arrived()) latch(173, "reduction: its results did not arrive");
+    return i == count;
 }
 
 void *stage_to_device(const void *host, size_t bytes)

@@ -102,9 +102,15 @@ struct Ctx {
     size_t scratch_bytes = 0;
     void *rows = nullptr;  // row-major X staging of the SpMM gather path
     size_t rows_bytes = 0;
-    // pinned host buffer for results read back by the host
+    // pinned host buffer for results that kernels write and the host reads
     double *hbuf = nullptr;
     size_t hbuf_bytes = 0;
+    // numbers that kernels write beside their results: the host takes a result
+    // once its number is the launch's.  An array of its own, so that no other
+    // data can look like a number; it only grows, and the numbers with it.
+    unsigned long long *hseq = nullptr;
+    size_t hseq_count = 0;
+    unsigned long long seq = 0;  // the last launch's
     double dev_bytes = 0.0;
     int num_cu = 0;
     // host->device staging ring (pinned host side, device side)
@@ -121,7 +127,13 @@ bool ensure_ctx();
 bool noalloc_setup(int device);
 void *scratch(size_t bytes);           // device scratch of at least bytes
 void *row_stage(size_t bytes);         // device staging of row-major X copies (SpMM), at least bytes
-double *host_buf(size_t count);        // pinned host doubles
+double *host_buf(size_t count);        // pinned host doubles, writable by kernels
+// The first count numbers and the next launch's (one report at a time: the
+// launch, then wait_seq); null (latched) without memory.
+unsigned long long *host_seq(size_t count, unsigned long long *next);
+// Waits until the first count numbers are all `want`, written by kernels
+// queued on the stream; false (latched) when it has drained without them.
+bool wait_seq(size_t count, unsigned long long want);
 // Copy small host data (coefficients) to device memory without blocking:
 // the bytes go through a pinned ring whose slots are reused only after the
 // next stream synchronisation.  Returns the device address.

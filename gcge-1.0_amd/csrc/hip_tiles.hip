@@ -441,11 +441,17 @@ __global__ __launch_bounds__(kThreads) void k_gram_thin(int64_t n, const T *__re
     }
 }
 
-// G[e] = sum_c partial[c][e]: 64 entries per workgroup, the 4 wavefronts take
-// every 4th chunk, combined in a fixed order.  With upper_only, entries
-// below the diagonal (i > j, e = j * p + i) are skipped.
+// G[e] = sum_c partial[c][e] into host memory: 64 entries per workgroup, the 4
+// wavefronts take every 4th chunk, 8 loads in flight (a wavefront has up to
+// 128 chunks; one load at a time took 38 us on average in a mixed solve of
+// the 64^3 generalized problem, this 9), combined in a fixed order; then the
+// launch's number in seqs[workgroup].
+// With upper_only, entries below the diagonal (i > j, e = j * p + i) are
+// skipped.
 __global__ __launch_bounds__(kThreads) void k_sum_chunks(const double *__restrict__ partial, int nchunk, int p,
-                                                         int64_t pq, int upper_only, double *__restrict__ G)
+                                                         int64_t pq, int upper_only, double *__restrict__ G,
+                                                         unsigned long long *__restrict__ seqs,
+                                                         unsigned long long seq)
 {
     __shared__ double sh[4][64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -453,11 +459,23 @@ __global__ __launch_bounds__(kThreads) void k_sum_chunks(const double *__restric
     bool live = e < pq;
     if (live && upper_only) live = (e % p) <= (e / p);
     double acc = 0.0;
-    if (live)
-        for (int c = wave; c < nchunk; c += 4) acc += partial[(int64_t)c * pq + e];
+    if (live) {
+        int c = wave;
+        for (; c + 28 < nchunk; c += 32) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = partial[(int64_t)(c + 4 * u) * pq + e];
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc += v[u];
+        }
+        for (; c < nchunk; c += 4) acc += partial[(int64_t)c * pq + e];
+    }
     sh[wave][lane] = acc;
     __syncthreads();
     if (wave == 0 && e < pq) G[e] = live ? (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]) : 0.0;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(seqs + blockIdx.x, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- LinComb (MFMA)
@@ -841,7 +859,7 @@ bool gram(int prec, int64_t n, const void *V, int64_t ldv, int p, const void *W,
         rpc = ((rpc + unit - 1) / unit) * unit;
         nchunk = (int)((n + rpc - 1) / rpc);
     }
-    double *partial = (double *)scratch(sizeof(double) * ((size_t)nchunk * pq + pq));
+    double *partial = (double *)scratch(sizeof(double) * (size_t)nchunk * pq);
     if (!partial) return false;
     {
         ProfScope ps(thin ? K_GRAM_THIN : (prec == GCGE_HIP_FP64 ? K_GRAM_MFMA_F64 : K_GRAM_MFMA_F32),
@@ -877,16 +895,15 @@ bool gram(int prec, int64_t n, const void *V, int64_t ldv, int p, const void *W,
         }
     }
     if (!check(hipGetLastError(), "k_gram")) return false;
-    double *dG = partial + (int64_t)nchunk * pq;
     // the thin kernel writes every entry, so upper_only only prunes MFMA tiles
     const int up = (!thin && upper_only) ? 1 : 0;
-    k_sum_chunks<<<(int)((pq + 63) / 64), kThreads, 0, ctx().stream>>>(partial, nchunk, p, pq, up, dG);
-    if (!check(hipGetLastError(), "k_sum_chunks")) return false;
+    const int sums = (int)((pq + 63) / 64);
+    unsigned long long seq = 0, *seqs = host_seq(sums, &seq);
     double *h = host_buf((size_t)pq);
-    if (!h) return false;
-    if (!check(hipMemcpyAsync(h, dG, sizeof(double) * pq, hipMemcpyDeviceToHost, ctx().stream), "D2H gram"))
-        return false;
-    if (!sync()) return false;
+    if (!h || !seqs) return false;
+    k_sum_chunks<<<sums, kThreads, 0, ctx().stream>>>(partial, nchunk, p, pq, up, h, seqs, seq);
+    if (!check(hipGetLastError(), "k_sum_chunks")) return false;
+    if (!wait_seq(sums, seq)) return false;
     for (int j = 0; j < q; j++) std::memcpy(G + (int64_t)j * ldg, h + (int64_t)j * p, sizeof(double) * p);
     return true;
 }

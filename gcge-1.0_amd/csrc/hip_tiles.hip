@@ -21,12 +21,11 @@
 // Very thin products (p <= 4, q <= 8 or the transpose) take a vector kernel
 // that keeps the whole p x q block in registers and reads V and W once.
 //
-// LinComb: a wavefront owns 32 rows of Y (with more than 64 output columns,
-// two wavefronts share the rows and split the columns) and walks
-// its output columns in blocks of 16; X supplies the A operand straight from HBM (16 consecutive
-// rows per lane group), C the B operand from a copy packed on the host in
-// operand order.  Thin combinations (p, q <= 8) take a vector kernel with C
-// in the kernel arguments and 16-byte row vectors.
+// LinComb: a wavefront owns 32 (FP64) or 64 (FP32) rows of Y and all its
+// columns up to 128; X supplies the A operand straight from HBM, C the B
+// operand from a copy packed on the host in operand order and staged through
+// LDS for the workgroup.  Thin combinations (p, q <= 8) take a vector kernel
+// with C in the kernel arguments and 16-byte row vectors.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -61,6 +60,9 @@ struct MT<double> {
     }
     // result row of slot t in lane group g = l / 16
     __device__ static __forceinline__ int drow(int g, int t) { return 4 * t + g; }
+    // order of the 16 rows of an operand so that, slot by slot, the lane
+    // groups hold neighbouring result rows: operand row i is row spread(i)
+    __device__ static __forceinline__ int spread(int i) { return i; }
 };
 
 template <>
@@ -73,6 +75,7 @@ struct MT<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     __device__ static __forceinline__ int drow(int g, int t) { return 4 * g + t; }
+    __device__ static __forceinline__ int spread(int i) { return 4 * (i & 3) + (i >> 2); }
 };
 
 // R consecutive rows [row, row + R) of one column, zero past `end`
@@ -480,9 +483,170 @@ __global__ __launch_bounds__(kThreads) void k_sum_chunks(const double *__restric
 
 // ---------------------------------------------------------------- LinComb (MFMA)
 // Cp[((kb * nqb) + jb) * 64 + l] = C(4 kb + l / 16, 16 jb + l % 16), zero
-// past p and q.  A wavefront owns rows [rb, rb + 32) as two 16-row blocks and
-// walks the output in groups of RN 16-column blocks; slot t of lane l holds
-// row drow(l / 16, t) of its block and column l % 16.
+// past p and q.  A wavefront owns RB blocks of 16 rows, row i of block h being
+// row RB spread(i) + h of its 16 RB: a lane's A operands of the RB blocks are
+// RB consecutive rows of one column of X, one vector load, and slot t of the
+// lane groups 0 .. 3 are 4 RB consecutive rows of Y, 64 bytes for RB = 2 in
+// FP64 and 4 in FP32.  It forms RN blocks of 16
+// columns (all of them up to 128 columns, so X leaves memory once), RN fitted
+// to q: 100 columns are 7 blocks, not 8.  The four wavefronts share C, staged
+// in LDS in panels of 4 k blocks two deep (each reads 512 bytes per k block and
+// column block; from L2 these reads cost as much as the products); X is
+// loaded one panel ahead into registers.  Bound by the matrix cores for large
+// p and q (a large library product reaches 67 TF here in FP64, 153 in FP32).
+// Over 4.1M rows, 300 x 100: FP64 6.73 -> 5.03 ms (49 TF), FP32 3.44 -> 2.76
+// (89 TF); 100 x 100: 2.86 -> 2.10 and 1.45 -> 1.33; 300 x 130 (two passes of
+// 5 blocks): 12.5 -> 7.3 and 6.5 -> 3.9.  Every sum runs over k in ascending
+// blocks of 4, whatever RB and RN.
+
+// y[0..V) = beta y + alpha v with the branch rules of y = a x + b y, one
+// access of V elements
+template <typename T, int V>
+__device__ __forceinline__ void store_rows(T *y, const T (&v)[V], T al, T be, int64_t room)
+{
+    struct alignas(V * sizeof(T)) Vec {
+        T e[V];
+    };
+    if (room >= V) {
+        Vec out;
+        if (be == T(0)) {
+#pragma unroll
+            for (int t = 0; t < V; t++) out.e[t] = (al == T(1)) ? v[t] : al * v[t];
+        } else {
+            const Vec old = *reinterpret_cast<const Vec *>(y);
+#pragma unroll
+            for (int t = 0; t < V; t++) out.e[t] = be * old.e[t] + al * v[t];
+        }
+        *reinterpret_cast<Vec *>(y) = out;
+    } else {
+#pragma unroll
+        for (int t = 0; t < V; t++)
+            if (t < room) y[t] = (be == T(0)) ? ((al == T(1)) ? v[t] : al * v[t]) : be * y[t] + al * v[t];
+    }
+}
+
+// A wavefront's results to Y: slot t of lane group kk is operand row
+// drow(kk, t), column block r column 16 (g0 + r) + m
+template <typename T, int RN, int RB>
+__device__ __forceinline__ void store_tile(const typename MT<T>::acc_t (&acc)[RB][RN], T *__restrict__ Y,
+                                           int64_t ldy, int g0, int q, int64_t rw, int64_t n, T al, T be)
+{
+    const int m = threadIdx.x & 15, kk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int r = 0; r < RN; r++) {
+        const int j = (g0 + r) * 16 + m;
+        if (j >= q) continue;
+        T *yj = Y + (int64_t)j * ldy;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int64_t row = rw + MT<T>::spread(MT<T>::drow(kk, t)) * RB;
+            T v[RB];
+#pragma unroll
+            for (int h = 0; h < RB; h++) v[h] = (T)acc[h][r][t];
+            store_rows<T, RB>(yj + row, v, al, be, n - row);
+        }
+    }
+}
+
+template <typename T, int RN, int RB>
+__global__ __launch_bounds__(kThreads, RN <= 2 ? 4 : RN <= 4 ? 3 : 2) void k_lincomb_mfma(int64_t n, const T *__restrict__ X, int64_t ldx, int p,
+                                                              T *__restrict__ Y, int64_t ldy, int q,
+                                                              const T *__restrict__ Cp, int nkb, int nqb,
+                                                              double alpha, double beta)
+{
+    using acc_t = typename MT<T>::acc_t;
+    constexpr int KP = RB == 1 ? 8 : 4;          // k blocks per panel
+    constexpr int E = 16 / (int)sizeof(T);       // elements of a 16-byte copy unit
+    constexpr int UNITS = KP * RN * 64 / E;
+    constexpr int UPT = (UNITS + kThreads - 1) / kThreads;
+    typedef T u16 __attribute__((ext_vector_type(E)));
+    struct alignas(RB * sizeof(T)) Rows {
+        T e[RB];
+    };
+    __shared__ __attribute__((aligned(16))) T sc[2][KP * RN * 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int m = lane & 15, kk = lane >> 4;
+    // rows past n up to the next multiple of 64 RB <= 256 lie in the columns'
+    // padding: they feed only result rows that are not stored
+    const int64_t rw = ((int64_t)blockIdx.x * 4 + wave) * 16 * RB;
+    const T *xr = X + rw + MT<T>::spread(m) * RB;
+    const T al = (T)alpha, be = (T)beta;
+    const int npan = (nkb + KP - 1) / KP;
+    for (int g0 = 0; g0 < nqb; g0 += RN) {
+        u16 creg[UPT];
+        Rows a[KP], an[KP];
+        auto fetch = [&](int pan) {
+#pragma unroll
+            for (int i = 0; i < KP; i++) {
+                const int c = (pan * KP + i) * 4 + kk;
+                an[i] = *reinterpret_cast<const Rows *>(xr + (int64_t)min(c, p - 1) * ldx);
+            }
+#pragma unroll
+            for (int u = 0; u < UPT; u++) {
+                const int unit = min((int)threadIdx.x + u * kThreads, UNITS - 1);
+                const int kl = unit * E / (RN * 64), off = unit * E % (RN * 64);
+                const int kb = min(pan * KP + kl, nkb - 1);
+                creg[u] = *reinterpret_cast<const u16 *>(Cp + ((int64_t)kb * nqb + g0) * 64 + off);
+            }
+        };
+        // the fetched panel becomes the current one (here, not in fetch, is X
+        // looked at: its loads are in flight during the panel before)
+        auto park = [&](int pan) {
+#pragma unroll
+            for (int u = 0; u < UPT; u++) {
+                const int unit = threadIdx.x + u * kThreads;
+                if (UNITS % kThreads == 0 || unit < UNITS) *reinterpret_cast<u16 *>(&sc[pan & 1][unit * E]) = creg[u];
+            }
+            const bool whole = (pan + 1) * KP * 4 <= p;
+#pragma unroll
+            for (int i = 0; i < KP; i++)
+#pragma unroll
+                for (int h = 0; h < RB; h++)
+                    a[i].e[h] = (whole || (pan * KP + i) * 4 + kk < p) ? an[i].e[h] : T(0);
+        };
+        acc_t acc[RB][RN];
+#pragma unroll
+        for (int h = 0; h < RB; h++)
+#pragma unroll
+            for (int r = 0; r < RN; r++) acc[h][r] = acc_t{};
+        auto products = [&](int i, const T *c) {
+            T bb[RN];
+#pragma unroll
+            for (int r = 0; r < RN; r++) bb[r] = c[(i * RN + r) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < RN; r++)
+#pragma unroll
+                for (int h = 0; h < RB; h++) acc[h][r] = MT<T>::mma(a[i].e[h], bb[r], acc[h][r]);
+        };
+        fetch(0);
+        park(0);
+        __syncthreads();
+        for (int pan = 0; pan + 1 < npan; pan++) {
+            fetch(pan + 1);
+#pragma unroll
+            for (int i = 0; i < KP; i++) products(i, sc[pan & 1]);
+            park(pan + 1);
+            __syncthreads();
+        }
+        // the last panel: 1 .. KP k blocks
+#pragma unroll
+        for (int i = 0; i < KP; i++)
+            if ((npan - 1) * KP + i < nkb) products(i, sc[(npan - 1) & 1]);
+        __syncthreads();  // the next pass overwrites sc
+        store_tile<T, RN, RB>(acc, Y, ldy, g0, q, rw, n, al, be);
+    }
+}
+
+// The same products for few columns: a wavefront owns rows [rb, rb + 32) as
+// two 16-row blocks, walks the output in groups of RN 16-column blocks and
+// reads C from the caches; no LDS and no barriers, so more wavefronts are in
+// flight, which is what a memory-bound product needs.  FP32 over 4.1M rows,
+// this kernel against k_lincomb_mfma: 50 x 50 0.517 against 0.565 ms, 20 x 20
+// 0.228 against 0.250, but 150 x 50 1.087 against 0.999; FP64 20 x 20 0.419
+// against 0.433, but 50 x 50 1.080 against 0.840.  Over 16,384 rows, FP32:
+// 100 x 100 14.4 against 17.5 us, 200 x 100 23.5 against 25.5, but 300 x 100
+// 30.1 against 29.1.  slot t of lane l holds row drow(l / 16, t) of its block
+// and column l % 16.
 // Result rows of one lane after regrouping: lane (g = l / 16, m) returns
 // rows 4 g .. 4 g + 3 of column m of the 16 x 16 block.  For FP32 these are
 // already its four slots; for FP64 (slot t holds row 4 t + g) the four lanes
@@ -538,7 +702,7 @@ __device__ __forceinline__ void store_rows4(T *y, typename MT<T>::acc_t v, T al,
 }
 
 template <typename T, int RN, int WC>
-__global__ __launch_bounds__(kThreads) void k_lincomb_mfma(int64_t n, const T *__restrict__ X, int64_t ldx, int p,
+__global__ __launch_bounds__(kThreads) void k_lincomb_rows(int64_t n, const T *__restrict__ X, int64_t ldx, int p,
                                                            T *__restrict__ Y, int64_t ldy, int q,
                                                            const T *__restrict__ Cp, int nkb, int nqb, double alpha,
                                                            double beta)
@@ -637,6 +801,21 @@ __global__ __launch_bounds__(kThreads) void k_lincomb_mfma(int64_t n, const T *_
             }
         }
     }
+}
+
+template <typename T, int RB>
+void launch_lincomb_mfma(int rn, int64_t n, const void *X, int64_t ldx, int p, void *Y, int64_t ldy, int q,
+                         const void *Cp, int nkb, int nqb, double alpha, double beta)
+{
+    const int grid = (int)((n + 64 * RB - 1) / (64 * RB));
+#define GH_LC(RN_)                                                                                             \
+    if (rn == RN_) {                                                                                            \
+        k_lincomb_mfma<T, RN_, RB><<<grid, kThreads, 0, ctx().stream>>>(                                        \
+            n, (const T *)X, ldx, p, (T *)Y, ldy, q, (const T *)Cp, nkb, nqb, alpha, beta);                     \
+        return;                                                                                                 \
+    }
+    GH_LC(1) GH_LC(2) GH_LC(3) GH_LC(4) GH_LC(5) GH_LC(6) GH_LC(7) GH_LC(8)
+#undef GH_LC
 }
 
 // ---------------------------------------------------------------- LinComb (thin)
@@ -936,19 +1115,19 @@ bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, in
         else launch_lincomb_thin<float>(n, X, ldx, p, Y, ldy, q, cf, alpha, beta);
         return check(hipGetLastError(), "k_lincomb_thin");
     }
-    if (((uintptr_t)Y & 31u) || (ldy * elem_size(prec)) % 32) {
-        latch(171, "lincomb: output is not 32-byte aligned");
+    if (((uintptr_t)X & 15u) || (ldx * elem_size(prec)) % 16 || ((uintptr_t)Y & 31u) ||
+        (ldy * elem_size(prec)) % 32 || ldx < (n + 255) / 256 * 256) {
+        latch(171, "lincomb: operands are not aligned or padded");
         return false;
     }
-    // column blocks per wavefront pass (RN) and wavefronts per row block
-    // (WC): more than 4 column blocks are split over two wavefronts (4 blocks
-    // each), which keeps the accumulators small enough for two or more
-    // wavefronts per SIMD
+    // column blocks per pass (RN, at most 8) so that the passes are equal;
+    // k_lincomb_rows: 1, 2 or 4, beyond 4 by two wavefronts (WC)
     const int nkb = (p + 3) / 4, nqb0 = (q + 15) / 16;
-    const bool split = nqb0 > 4;
-    const int rn = split ? 4 : nqb0 <= 1 ? 1 : nqb0 <= 2 ? 2 : nqb0 <= 4 ? 4 : 8;
-    const int wc = split ? 2 : 1;
-    const int nqb = ((nqb0 + rn * wc - 1) / (rn * wc)) * rn * wc;  // zero blocks pad the last groups
+    const bool rows = prec == GCGE_HIP_FP64 ? q <= 32 && p < 64 : q <= 64 ? p < 128 : n < 65536 && p < 256;
+    const int wc = rows && nqb0 > 4 ? 2 : 1;
+    const int groups = (nqb0 + 7) / 8;
+    const int rn = rows ? (nqb0 <= 2 ? nqb0 : 4) : (nqb0 + groups - 1) / groups;
+    const int nqb = ((nqb0 + rn * wc - 1) / (rn * wc)) * rn * wc;  // zero blocks pad the last pass
     const size_t ncp = (size_t)nkb * nqb * 64;
     const void *dC = nullptr;
     if (prec == GCGE_HIP_FP64) {
@@ -971,27 +1150,31 @@ bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, in
         dC = stage_to_device(cp.data(), sizeof(float) * ncp);
     }
     if (!dC) return false;
-    const int grid = (int)((n + 128 / wc - 1) / (128 / wc));
     {
-        ProfScope ps(prec == GCGE_HIP_FP64 ? K_LINCOMB_MFMA_F64 : K_LINCOMB_MFMA_F32, (double)n * (p + q + (beta != 0.0 ? q : 0)) * elem_size(prec),
-                     2.0 * (double)n * p * q);
-#define GH_LC(T_, RN_) GH_LCW(T_, RN_, 1)
-#define GH_LCW(T_, RN_, WC_)                                                                                   \
-    k_lincomb_mfma<T_, RN_, WC_><<<grid, kThreads, 0, ctx().stream>>>(n, (const T_ *)X, ldx, p, (T_ *)Y, ldy,  \
-                                                                      q, (const T_ *)dC, nkb, nqb, alpha, beta)
-        if (prec == GCGE_HIP_FP64) {
-            if (wc == 2) GH_LCW(double, 4, 2);
-            else if (rn == 1) GH_LC(double, 1);
-            else if (rn == 2) GH_LC(double, 2);
-            else GH_LC(double, 4);
+        ProfScope ps(prec == GCGE_HIP_FP64 ? K_LINCOMB_MFMA_F64 : K_LINCOMB_MFMA_F32,
+                     (double)n * (p + q + (beta != 0.0 ? q : 0)) * elem_size(prec), 2.0 * (double)n * p * q);
+#define GH_LR(T_, RN_, WC_)                                                                                    \
+    k_lincomb_rows<T_, RN_, WC_><<<(int)((n + 128 / WC_ - 1) / (128 / WC_)), kThreads, 0, ctx().stream>>>(      \
+        n, (const T_ *)X, ldx, p, (T_ *)Y, ldy, q, (const T_ *)dC, nkb, nqb, alpha, beta)
+        // k_lincomb_mfma: as many 16-row blocks per wavefront as leave 512 workgroups
+        const int want = (int)std::min<int64_t>(4, n / (64 * 512));
+        if (rows && prec == GCGE_HIP_FP64) {
+            if (rn == 1) GH_LR(double, 1, 1);
+            else GH_LR(double, 2, 1);
+        } else if (rows) {
+            if (wc == 2) GH_LR(float, 4, 2);
+            else if (rn == 1) GH_LR(float, 1, 1);
+            else if (rn == 2) GH_LR(float, 2, 1);
+            else GH_LR(float, 4, 1);
+        } else if (prec == GCGE_HIP_FP64) {
+            if (want >= 2) launch_lincomb_mfma<double, 2>(rn, n, X, ldx, p, Y, ldy, q, dC, nkb, nqb, alpha, beta);
+            else launch_lincomb_mfma<double, 1>(rn, n, X, ldx, p, Y, ldy, q, dC, nkb, nqb, alpha, beta);
         } else {
-            if (wc == 2) GH_LCW(float, 4, 2);
-            else if (rn == 1) GH_LC(float, 1);
-            else if (rn == 2) GH_LC(float, 2);
-            else GH_LC(float, 4);
+            if (want >= 4) launch_lincomb_mfma<float, 4>(rn, n, X, ldx, p, Y, ldy, q, dC, nkb, nqb, alpha, beta);
+            else if (want >= 2) launch_lincomb_mfma<float, 2>(rn, n, X, ldx, p, Y, ldy, q, dC, nkb, nqb, alpha, beta);
+            else launch_lincomb_mfma<float, 1>(rn, n, X, ldx, p, Y, ldy, q, dC, nkb, nqb, alpha, beta);
         }
-#undef GH_LC
-#undef GH_LCW
+#undef GH_LR
     }
     return check(hipGetLastError(), "k_lincomb");
 }

@@ -13,11 +13,12 @@
 // (the FP64 result rows are interleaved; checked on the device).
 //
 // Gram: the n rows are cut into chunks; a workgroup owns one chunk and one
-// output tile, and the reduction index k of the MFMA runs over rows.  Each
-// lane loads R consecutive rows of one column as one aligned vector (32
-// bytes), so a superstep of the wavefront covers 4 R rows and MFMA step t
-// takes row  base + 4 R s + (l / 16) R + t  for both operands.  Partial
-// tiles go to a per-chunk buffer that a second kernel sums in a fixed order.
+// output block, and the reduction index k of the MFMA runs over rows.  Partial
+// blocks go to a per-chunk buffer that a second kernel sums in a fixed order.
+// Few columns (k_gram_mfma): each lane loads R consecutive rows of one column
+// as one aligned vector (32 bytes), so a superstep of the wavefront covers 4 R
+// rows and MFMA step t takes row  base + 4 R s + (l / 16) R + t  for both
+// operands.  Otherwise (k_gram_slab) V and W go through LDS.
 // Very thin products (p <= 4, q <= 8 or the transpose) take a vector kernel
 // that keeps the whole p x q block in registers and reads V and W once.
 //
@@ -30,6 +31,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "hip_common.h"
@@ -40,7 +42,9 @@ namespace {
 
 constexpr int kThreads = 256;       // 4 wavefronts per workgroup
 constexpr int kGramTargetWG = 2048; // workgroups a Gram launch aims for
-constexpr int kGramSlabWG = 512;    // workgroups of a slab Gram launch (two per CU)
+constexpr int kSlabThreads = 512;   // slab Gram: 8 wavefronts per workgroup
+constexpr int kSlabTiles = 28;      // most 16-column tiles of V and W together in its block (7 units per thread)
+constexpr int kSlabMaxNT = 17;      // most output tiles per wavefront
 
 typedef double dx4 __attribute__((ext_vector_type(4)));
 typedef float fx4 __attribute__((ext_vector_type(4)));
@@ -261,139 +265,187 @@ __global__ __launch_bounds__(kThreads) void k_gram_mfma(int64_t n, const T *__re
 }
 
 // ---------------------------------------------------------------- Gram (LDS slabs)
-// Workgroup output block (MB 16) x (NB 16), NB <= 8 at run time, over one
-// row chunk.  Every SLAB rows (128 bytes of each column) the 256 threads copy
-// the block's columns of V and W into LDS (column-major, 16-byte pad per
-// column: 144-byte column stride, so neither the 16-byte copies nor the
-// operand reads of 16 consecutive columns meet a bank twice), two buffers
-// deep; wavefront w runs the MFMAs of tile columns w and w + 4 for all MB
-// tile rows.  V and W thus leave memory once per block instead of once per
-// 64 x 64 tile, and p, q are padded to 16 rather than 64.
-template <typename T, int MB>
-__global__ __launch_bounds__(kThreads) void k_gram_slab(int64_t n, const T *__restrict__ V, int64_t ldv, int p,
-                                                        const T *__restrict__ W, int64_t ldw, int q, int NB,
-                                                        int blocks_p, int blocks_q, int nchunk,
-                                                        int64_t rows_per_chunk, int upper_only,
-                                                        double *__restrict__ partial)
+// Workgroup output block of MB x NB 16 x 16 tiles over one row chunk, eight
+// wavefronts.  Every SLAB rows (128 bytes of each column) the threads copy the
+// block's columns of V and W into LDS (column-major, 16-byte pad per column:
+// 144-byte column stride, so neither the 16-byte copies nor the operand
+// reads of 16 consecutive columns meet a bank twice), two buffers
+// deep.  The block's tiles, column by column, without those below the diagonal
+// when upper_only, are dealt out in equal runs of at most NT per wavefront,
+// whatever MB and NB: every SIMD has the same number of products.
+// UPT: 16-byte units that a thread copies per slab, at least (MB + NB) / 4.
+// Product t = 0 .. E - 1 of step 0 or 1, E = 16 / sizeof(T), takes row
+// 4 E step + 4 t + l / 16  of the slab for both operands, or with RUN (up to 64
+// x 64 columns, as in k_gram_mfma, and past 256)  2 E (l / 16) + E step + t,
+// which a lane reads at once: 4 % faster.
+// Bound by memory for few columns (4.0 - 4.6 TB/s: each visit of a column
+// reads 128 bytes of another page), by the matrix cores for many (67 TF in
+// FP64 and 153 in FP32 for a large library product here; 46 and 84 reached, 53
+// and 97 with the tiles' padding).  4.1M rows, ms, before (blocks of up to 8 x
+// 8 tiles dealt out by column, 4 wavefronts, loads and LDS reads waited for
+// one by one) and now, FP64 / FP32: 300 x 100 7.05 / 3.97 -> 5.31 / 2.91; 200
+// x 100 4.80 / 2.74 -> 4.20 / 2.33; 100 x 100, upper 1.87 / 1.12 -> 1.63 /
+// 0.86; 100 x 50 1.87 / 1.15 -> 1.73 / 0.90; 64 x 64 1.42 / 0.91 -> 1.06 /
+// 0.45 (without LDS).
+template <typename T, int NT, int UPT, bool RUN>
+__global__ __launch_bounds__(kSlabThreads, (UPT <= 4 ? 4 : 2)) void k_gram_slab(
+    int64_t n, const T *__restrict__ V, int64_t ldv, int p, const T *__restrict__ W, int64_t ldw, int q, int MB,
+    int NB, int blocks_p, int blocks_q, int nchunk, int64_t rows_per_chunk, int upper_only,
+    double *__restrict__ partial)
 {
-    constexpr int SLAB = 128 / (int)sizeof(T);     // rows per stage
-    constexpr int LD = SLAB + 16 / (int)sizeof(T);  // LDS column stride (elements)
-    constexpr int TP = MB * 16;
-    constexpr int COLS = TP + 128;                  // V block + up to 8 W tiles
-    constexpr int UPT = (COLS * 8 + kThreads - 1) / kThreads;  // 16-byte units per thread
-    constexpr int E = 16 / (int)sizeof(T);          // elements per unit
+    constexpr int E = 16 / (int)sizeof(T);     // elements of a 16-byte unit
+    constexpr int SLAB = 8 * E;                // rows per stage
+    constexpr int LD = SLAB + E;               // LDS column stride (elements)
+    constexpr int READS = RUN ? 2 : E;         // LDS reads of a tile's operands (two rows each unless RUN)
     using acc_t = typename MT<T>::acc_t;
     typedef T u16 __attribute__((ext_vector_type(E)));
-    __shared__ __attribute__((aligned(16))) T sbuf[2][COLS * LD];
+    extern __shared__ __attribute__((aligned(16))) unsigned char slab_smem[];
+    T *sbuf = reinterpret_cast<T *>(slab_smem);  // [2][(MB + NB) * 16 * LD]
 
     const int nblock = blocks_p * blocks_q;
     const int logical = xcd_logical_block();
     if (logical >= nblock * nchunk) return;
     const int chunk = logical / nblock, blk = logical % nblock;
-    const int i0 = (blk % blocks_p) * TP, j0 = (blk / blocks_p) * NB * 16;
+    const int i0 = (blk % blocks_p) * MB * 16, j0 = (blk / blocks_p) * NB * 16;
     const int64_t rb = (int64_t)chunk * rows_per_chunk;
     const int64_t re = min(n, rb + rows_per_chunk);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int m = lane & 15, kk = lane >> 4;
-    const int ncols = TP + NB * 16;
+    const int units = (MB + NB) * 128, bufsize = (MB + NB) * 16 * LD;
 
-    // this thread's copy units: column c (V for c < TP, else W), 16 bytes
+    // tiles of column y that are computed: x = 0 .. rows_of(y) - 1 (those that
+    // reach the matrix and, with upper_only, its diagonal)
+    const int xall = min(MB, (p - i0 + 15) / 16), yall = min(NB, (q - j0 + 15) / 16);
+    auto rows_of = [&](int y) { return upper_only ? max(0, min(xall, (j0 - i0) / 16 + y + 1)) : xall; };
+    int live = 0;
+    for (int y = 0; y < yall; y++) live += rows_of(y);
+    if (live == 0) return;  // a block below the diagonal
+    const int share = (live + 7) / 8, first = wave * share, mine = max(0, min(share, live - first));
+    // its i-th tile (uniform; the slots past `mine` repeat the last one and are
+    // not stored)
+    auto walk = [&](auto &&f) {
+        int y = 0, x = min(first, live - 1);
+        while (x >= rows_of(y)) x -= rows_of(y++);
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+            f(i, x, y);
+            if (i + 1 < mine && ++x >= rows_of(y)) {
+                x = 0;
+                do y++;
+                while (rows_of(y) == 0);
+            }
+        }
+    };
+    int ao[NT], bo[NT];  // LDS offsets of the tiles' operands
+    walk([&](int i, int x, int y) {
+        ao[i] = x * 16 * LD;
+        bo[i] = (MB + y) * 16 * LD;
+    });
+
+    // this thread's copy units: column c (V for c < 16 MB, else W), 16 bytes
     // at row offset E * seg of the slab; columns past p (q) repeat the last
     // one and feed only result entries that are never stored
+    const int seg = threadIdx.x & 7;
     const T *src[UPT];
-    int dst[UPT];
 #pragma unroll
     for (int u = 0; u < UPT; u++) {
-        const int unit = threadIdx.x + u * kThreads;
-        const int c = unit >> 3, seg = unit & 7;
-        if (c < ncols) {
-            src[u] = (c < TP ? V + (int64_t)min(i0 + c, p - 1) * ldv
-                             : W + (int64_t)min(j0 + c - TP, q - 1) * ldw) + seg * E;
-            dst[u] = c * LD + seg * E;
-        } else {
-            src[u] = nullptr;
-            dst[u] = -1;
-        }
+        const int c = min((int)threadIdx.x + u * kSlabThreads, units - 1) >> 3;
+        src[u] = (c < MB * 16 ? V + (int64_t)min(i0 + c, p - 1) * ldv
+                              : W + (int64_t)min(j0 + c - MB * 16, q - 1) * ldw) + seg * E;
     }
     u16 reg[UPT];
-    auto fetch = [&](int64_t r) {
-        if (r + SLAB <= re) {
+    auto park = [&](T *buf) {
 #pragma unroll
-            for (int u = 0; u < UPT; u++)
-                if (dst[u] >= 0) reg[u] = *reinterpret_cast<const u16 *>(src[u] + r);
-        } else {
-#pragma unroll
-            for (int u = 0; u < UPT; u++)
-                if (dst[u] >= 0) {
-                    const int64_t r0 = r + dst[u] % LD;  // row of the unit's first element
-#pragma unroll
-                    for (int e = 0; e < E; e++) reg[u][e] = (r0 + e < re) ? src[u][r + e] : T(0);
-                }
+        for (int u = 0; u < UPT; u++) {
+            const int unit = threadIdx.x + u * kSlabThreads;
+            if (unit < units) *reinterpret_cast<u16 *>(buf + (unit >> 3) * LD + seg * E) = reg[u];
         }
     };
-    auto park = [&](int b) {
+
+    acc_t acc[NT];
+#pragma unroll
+    for (int i = 0; i < NT; i++) acc[i] = acc_t{};
+    // Products of a parked slab, each tile's operands read while the products
+    // of the one before are issued (otherwise every read is waited for); with
+    // MORE, the slab at row `next` is loaded into the registers meanwhile, one
+    // load at a time among the first half of the products: a wavefront's loads
+    // meet 8 columns, thus 8 pages, each, and block its issue when they come
+    // together.  No branches: where paths meet, loads would be waited for.
+    auto products = [&](const T *buf, int64_t next, auto more) {
+        constexpr bool MORE = decltype(more)::value;
+        const T *s = buf + m * LD + kk * (RUN ? 2 * E : 1);
+        u16 a[2], b[2];
+        auto rows = [&](const T *c, int step) {
+            u16 v;
+            if constexpr (RUN) {
+                v = *reinterpret_cast<const u16 *>(c + step * E);
+            } else {
+#pragma unroll
+                for (int t = 0; t < E; t++) v[t] = c[step * 4 * E + 4 * t];
+            }
+            return v;
+        };
+        auto read = [&](int j) {
+            a[j & 1] = rows(s + ao[j % NT], j / NT);
+            b[j & 1] = rows(s + bo[j % NT], j / NT);
+        };
+        read(0);
+#pragma unroll
+        for (int j = 0; j < 2 * NT; j++) {
+            if (MORE && j < NT) {
+#pragma unroll
+                for (int u = j * UPT / NT; u < (j + 1) * UPT / NT; u++)
+                    reg[u] = *reinterpret_cast<const u16 *>(src[u] + next);
+            }
+            if (j + 1 < 2 * NT) read(j + 1);
+#pragma unroll
+            for (int t = 0; t < E; t++) acc[j % NT] = MT<T>::mma(a[j & 1][t], b[j & 1][t], acc[j % NT]);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);  // LDS reads of the first tile
+#pragma unroll
+        for (int j = 0; j < 2 * NT; j++) {
+            if (MORE && j < NT) {
+#pragma unroll
+                for (int u = j * UPT / NT; u < (j + 1) * UPT / NT; u++)
+                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
+            }
+            if (j + 1 < 2 * NT) __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, E, 0);  // products
+        }
+    };
+    const int nslab = (int)((re - rb) / SLAB);
+    const int64_t tail = rb + (int64_t)nslab * SLAB;
+    if (nslab > 0) {
+#pragma unroll
+        for (int u = 0; u < UPT; u++) reg[u] = *reinterpret_cast<const u16 *>(src[u] + rb);
+        park(sbuf);
+        __syncthreads();
+        for (int sl = 0; sl < nslab; sl++) {
+            // the last slab is loaded and parked once more
+            products(sbuf + (sl & 1) * bufsize, rb + (int64_t)min(sl + 1, nslab - 1) * SLAB, std::true_type{});
+            park(sbuf + ((sl + 1) & 1) * bufsize);
+            __syncthreads();
+        }
+    }
+    if (tail < re) {  // the chunk's partial slab, zero past its end
+        const int64_t r0 = tail + seg * E;
 #pragma unroll
         for (int u = 0; u < UPT; u++)
-            if (dst[u] >= 0) *reinterpret_cast<u16 *>(&sbuf[b][dst[u]]) = reg[u];
-    };
-
-    acc_t acc[MB][2];
 #pragma unroll
-    for (int x = 0; x < MB; x++) acc[x][0] = acc[x][1] = acc_t{};
-    // tiles this wavefront computes: column y = wave + 4 yy; with upper_only,
-    // tiles entirely below the diagonal are skipped
-    bool live[MB][2];
-#pragma unroll
-    for (int yy = 0; yy < 2; yy++) {
-        const int y = wave + 4 * yy;
-#pragma unroll
-        for (int x = 0; x < MB; x++)
-            live[x][yy] = y < NB && !(upper_only && i0 + x * 16 > j0 + y * 16 + 15);
-    }
-
-    const int nslab = (int)((re - rb + SLAB - 1) / SLAB);
-    if (nslab > 0) {
-        fetch(rb);
-        park(0);
-    }
-    __syncthreads();
-    for (int sl = 0; sl < nslab; sl++) {
-        const int b = sl & 1;
-        const bool more = sl + 1 < nslab;
-        if (more) fetch(rb + (int64_t)(sl + 1) * SLAB);
-        const T *sv = sbuf[b];
-        const T *sw = sbuf[b] + TP * LD;
-#pragma unroll
-        for (int ks = 0; ks < SLAB / 4; ks++) {
-            const int kr = ks * 4 + kk;
-            T a[MB], bq[2];
-#pragma unroll
-            for (int x = 0; x < MB; x++) a[x] = sv[(x * 16 + m) * LD + kr];
-#pragma unroll
-            for (int yy = 0; yy < 2; yy++) bq[yy] = sw[((wave + 4 * yy) * 16 + m) * LD + kr];
-#pragma unroll
-            for (int yy = 0; yy < 2; yy++)
-#pragma unroll
-                for (int x = 0; x < MB; x++)
-                    if (live[x][yy]) acc[x][yy] = MT<T>::mma(a[x], bq[yy], acc[x][yy]);
-        }
-        if (more) park(b ^ 1);
+            for (int e = 0; e < E; e++) reg[u][e] = (r0 + e < re) ? src[u][tail + e] : T(0);
+        park(sbuf);
         __syncthreads();
+        products(sbuf, tail, std::false_type{});
     }
 
     double *out = partial + (int64_t)chunk * p * q;
+    walk([&](int i, int x, int y) {
 #pragma unroll
-    for (int yy = 0; yy < 2; yy++) {
-        const int y = wave + 4 * yy;
-        if (y >= NB) continue;
-#pragma unroll
-        for (int x = 0; x < MB; x++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int i = i0 + x * 16 + MT<T>::drow(kk, t), j = j0 + y * 16 + m;
-                if (i < p && j < q) out[(int64_t)j * p + i] = (double)acc[x][yy][t];
-            }
-    }
+        for (int t = 0; t < 4; t++) {
+            const int r = i0 + x * 16 + MT<T>::drow(kk, t), j = j0 + y * 16 + m;
+            if (i < mine && r < p && j < q) out[(int64_t)j * p + r] = (double)acc[i][t];
+        }
+    });
 }
 
 // ---------------------------------------------------------------- Gram (thin)
@@ -962,17 +1014,73 @@ void launch_gram_mfma(const GramShape &g, int grid, int64_t n, const void *V, in
 #undef GH_GRAM
 }
 
-template <typename T>
-void launch_gram_slab(int MB, int grid, int64_t n, const void *V, int64_t ldv, int p, const void *W, int64_t ldw,
-                      int q, int NB, int bp, int bq, int nchunk, int64_t rpc, int upper, double *partial)
+// Blocks of a slab Gram launch: p16 x q16 tiles cut into bp x bq blocks of
+// MB x NB tiles, NT of them per wavefront
+struct SlabShape {
+    int bp, bq, MB, NB, NT;
+};
+
+// Most tiles that a block computes
+int slab_live(int p16, int q16, int MB, int NB, bool upper)
 {
-#define GH_SLAB(MB_)                                                                                            \
-    if (MB == MB_) {                                                                                            \
-        k_gram_slab<T, MB_><<<grid, kThreads, 0, ctx().stream>>>(n, (const T *)V, ldv, p, (const T *)W, ldw, q, \
-                                                                 NB, bp, bq, nchunk, rpc, upper, partial);      \
+    if (!upper) return std::min(MB, p16) * std::min(NB, q16);
+    int most = 0;
+    for (int i = 0; i < p16; i += MB)
+        for (int j = 0; j < q16; j += NB) {
+            int live = 0;
+            for (int y = j; y < std::min(q16, j + NB); y++)
+                live += std::max(0, std::min(std::min(MB, p16 - i), y - i + 1));
+            most = std::max(most, live);
+        }
+    return most;
+}
+
+// The cheapest cut: per row, a tile of products costs about 1, a tile's 16
+// columns 3.5 to load (67 TF and 5 TB/s in FP64, 153 TF in FP32).
+SlabShape slab_shape(int p16, int q16, bool upper)
+{
+    SlabShape best{0, 0, 0, 0, 0};
+    double least = 0.0;
+    for (int bp = 1; bp <= p16; bp++)
+        for (int bq = 1; bq <= q16; bq++) {
+            // many more blocks than some cut needs only load more
+            if (best.bp > 0 && bp * bq > 4 * best.bp * best.bq) break;
+            const int MB = (p16 + bp - 1) / bp, NB = (q16 + bq - 1) / bq;
+            const int NT = (slab_live(p16, q16, MB, NB, upper) + 7) / 8;
+            if (MB + NB > kSlabTiles || NT > kSlabMaxNT) continue;
+            const double cost = (double)bp * bq * (8.0 * NT + 3.5 * (MB + NB));
+            if (best.bp == 0 || cost < least) {
+                least = cost;
+                best = {(p16 + MB - 1) / MB, (q16 + NB - 1) / NB, MB, NB, NT};
+            }
+        }
+    return best;
+}
+
+// Blocks of up to 16 columns of tiles (74 KiB of LDS, at most 8 tiles per
+// wavefront, 128 registers): two workgroups per CU
+bool slab_narrow(const SlabShape &s) { return s.MB + s.NB <= 16; }
+
+size_t slab_lds(const SlabShape &s) { return (size_t)(s.MB + s.NB) * 16 * 144 * 2; }
+
+template <typename T>
+void launch_gram_slab(const SlabShape &s, int grid, int64_t n, const void *V, int64_t ldv, int p, const void *W,
+                      int64_t ldw, int q, int nchunk, int64_t rpc, int upper, double *partial)
+{
+    const bool small = p <= 64 && q <= 64, run = small || ((p > 256 || q > 256) && !slab_narrow(s));
+    const int upt = small ? 2 : slab_narrow(s) ? 4 : 7;
+#define GH_SLAB(NT_, UPT_, RUN_)                                                                                \
+    if (s.NT <= NT_ && upt == UPT_ && run == RUN_) {                                                            \
+        k_gram_slab<T, NT_, UPT_, RUN_><<<grid, kSlabThreads, slab_lds(s), ctx().stream>>>(                     \
+            n, (const T *)V, ldv, p, (const T *)W, ldw, q, s.MB, s.NB, s.bp, s.bq, nchunk, rpc, upper, partial); \
         return;                                                                                                 \
     }
-    GH_SLAB(1) GH_SLAB(2) GH_SLAB(3) GH_SLAB(4) GH_SLAB(5) GH_SLAB(6) GH_SLAB(7) GH_SLAB(8)
+    GH_SLAB(1, 2, true) GH_SLAB(2, 2, true)
+    GH_SLAB(1, 4, false) GH_SLAB(2, 4, false) GH_SLAB(3, 4, false) GH_SLAB(4, 4, false) GH_SLAB(5, 4, false)
+    GH_SLAB(6, 4, false) GH_SLAB(7, 4, false) GH_SLAB(8, 4, false)
+    GH_SLAB(2, 7, false) GH_SLAB(4, 7, false) GH_SLAB(6, 7, false) GH_SLAB(8, 7, false) GH_SLAB(10, 7, false)
+    GH_SLAB(12, 7, false) GH_SLAB(14, 7, false) GH_SLAB(17, 7, false)
+    GH_SLAB(3, 7, true) GH_SLAB(6, 7, true) GH_SLAB(10, 7, true) GH_SLAB(14, 7, true) GH_SLAB(17, 7, true)
 #undef GH_SLAB
 }
 
@@ -994,11 +1102,13 @@ bool gram(int prec, int64_t n, const void *V, int64_t ldv, int p, const void *W,
     int64_t rpc = 0;
     int tp = 1, tq = 1;
     GramShape g{1, 1, 1, 1};
-    // slab kernel beyond 64 columns on either side (blocks of up to 8 x 8
-    // tiles); up to 64 x 64 the single-tile workgroups with more chunks in
-    // flight move the data faster
-    const bool slab = !thin && (p > 64 || q > 64);
-    int MB = 0, NB = 0;
+    // slab kernel from 6 tiles of columns of V and W together; below, the
+    // kernel without LDS, with more workgroups in flight, moves the data
+    // faster.  4.1M rows, that one against the slabs, us: 60 x 16 FP64 556
+    // against 635 and FP32 292 against 321, 32 x 32 438 against 623 and 261
+    // against 318, but 40 x 40 1036 against 848 and 627 against 403
+    const bool slab = !thin && (p + 15) / 16 + (q + 15) / 16 >= 6;
+    SlabShape slab_sh{0, 0, 0, 0, 0};
     if (thin) {
         nchunk = (int)std::min<int64_t>(1024, std::max<int64_t>(1, (n + kThreads - 1) / kThreads));
     } else if (slab) {
@@ -1006,16 +1116,18 @@ bool gram(int prec, int64_t n, const void *V, int64_t ldv, int p, const void *W,
             latch(170, "gram: operands are not 32-byte aligned");
             return false;
         }
-        const int p16 = (p + 15) / 16, q16 = (q + 15) / 16;
-        tp = (p16 + 7) / 8;
-        tq = (q16 + 7) / 8;
-        MB = (p16 + tp - 1) / tp;
-        NB = (q16 + tq - 1) / tq;
+        slab_sh = slab_shape((p + 15) / 16, (q + 15) / 16, upper_only);
+        tp = slab_sh.bp;
+        tq = slab_sh.bq;
         const int64_t slab_rows = 128 / (int64_t)es;
         const int64_t max_chunks = std::max<int64_t>(1, (n + slab_rows - 1) / slab_rows);
-        // at most kGramSlabWG workgroups: all of them resident at once
-        nchunk = (int)std::min<int64_t>({(int64_t)kMaxChunks, max_chunks,
-                                         std::max<int64_t>(1, kGramSlabWG / (tp * tq))});
+        // Chunks: 512 for up to 128 x 128 columns, in inverse proportion
+        // beyond, but a workgroup for every CU (300 x 100, one block: 256
+        // chunks and not 170) and whole rounds of them where there are several
+        const int blocks = tp * tq;
+        nchunk = 512 / (((p + 127) / 128) * ((q + 127) / 128));
+        if (nchunk < 256) nchunk = (nchunk * blocks + 255) / 256 * 256 / blocks;
+        nchunk = (int)std::min<int64_t>({(int64_t)kMaxChunks, max_chunks, std::max(1, nchunk)});
         rpc = (n + nchunk - 1) / nchunk;
         rpc = ((rpc + slab_rows - 1) / slab_rows) * slab_rows;
         nchunk = (int)((n + rpc - 1) / rpc);
@@ -1057,11 +1169,11 @@ bool gram(int prec, int64_t n, const void *V, int64_t ldv, int p, const void *W,
             const int64_t blocks = (int64_t)tp * tq * nchunk;
             const int grid = (int)(((blocks + 7) / 8) * 8);
             if (prec == GCGE_HIP_FP64)
-                launch_gram_slab<double>(MB, grid, n, V, ldv, p, W, ldw, q, NB, tp, tq, nchunk, rpc,
-                                         upper_only ? 1 : 0, partial);
+                launch_gram_slab<double>(slab_sh, grid, n, V, ldv, p, W, ldw, q, nchunk, rpc, upper_only ? 1 : 0,
+                                         partial);
             else
-                launch_gram_slab<float>(MB, grid, n, V, ldv, p, W, ldw, q, NB, tp, tq, nchunk, rpc,
-                                        upper_only ? 1 : 0, partial);
+                launch_gram_slab<float>(slab_sh, grid, n, V, ldv, p, W, ldw, q, nchunk, rpc, upper_only ? 1 : 0,
+                                        partial);
         } else {
             const int64_t blocks = (int64_t)tp * tq * nchunk;
             const int grid = (int)(((blocks + 7) / 8) * 8);

@@ -65,3 +65,27 @@ def test_lincomb_edges(ops, mats, prec, n, p, q, alpha, beta):
     ref = alpha * (X @ cf) + (beta * Y if beta else 0.0)
     bound = (p + 3) * EPS[prec] * (abs(alpha) * (np.abs(X) @ np.abs(cf)) + abs(beta) * np.abs(Y))
     assert np.all(np.abs(y.get() - ref) <= bound)
+
+
+@pytest.mark.parametrize("prec", [F64, F32])
+@pytest.mark.parametrize("n", list(ROWS))
+@pytest.mark.parametrize("p,q,sym", [(33, 48, False), (16, 65, False), (81, 3, False), (300, 97, False),
+                                     (128, 128, False), (129, 130, False), (351, 100, False), (449, 17, False),
+                                     (33, 33, True), (49, 49, True), (100, 100, True), (129, 129, True),
+                                     (289, 289, True)])
+def test_gram_edges(ops, mats, prec, n, p, q, sym):
+    if n * (p + q) > 6.0e7:
+        pytest.skip("host reference too long")
+    g = np.random.default_rng(p * q + sym)
+    V = g.standard_normal((n, p))
+    W = V if sym else g.standard_normal((n, q))
+    v = nan_padded(mats[n], V, prec)
+    w = v if sym else nan_padded(mats[n], W, prec)
+    G = ops.gram(v, w, sym=sym)
+    V, W = stored(V, prec), stored(W, prec)
+    err = np.abs(G - V.T @ W)
+    # the device's sum of n terms, and the host's in FP64
+    bound = (n + 1) * (EPS[prec] + EPS[F64]) * (np.abs(V).T @ np.abs(W))
+    if sym:
+        err = np.triu(err)
+    assert np.all(err <= bound)

@@ -13,6 +13,8 @@
 #include <cmath>
 #include <cstring>
 #include <climits>
+#include <initializer_list>
+#include <type_traits>
 #include <vector>
 
 #include "hip_common.h"
@@ -68,33 +70,118 @@ int grid_1d(int64_t n, int cap)
     return (int)b;
 }
 
-// ---------------------------------------------------------------- axpby
+// ------------------------------------------------ element-wise streams
+// Kernels that read and write whole columns are bound by memory.  Two things
+// decide what they reach there (48 columns of 4.1M rows in FP32, 16 MB each,
+// GB/s): accesses of 16 bytes per lane, one per thread (copy 5230 with 4-byte
+// accesses, 6236), and, for blocks that no cache holds, loads and stores that
+// bypass them (copy 6794, search update 5390 -> 6380, residual update 5300 ->
+// 6540).  Blocks that the 256 MB cache holds are read back from it by the next
+// kernel: 252 MB of a search update take 53 us through it and 64 around it, 865
+// MB 263 and 244; kStreamBytes lies between.
+constexpr double kStreamBytes = 384e6;
+
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_axpby(int64_t n, const T *__restrict__ x, int64_t ldx,
-                                                  T *__restrict__ y, int64_t ldy, ColScalars s)
+constexpr int kWide = 16 / (int)sizeof(T);  // elements of a 16-byte access
+
+template <bool NT, typename V>
+__device__ __forceinline__ V load_as(const V *p)
 {
-    const int j = blockIdx.y;
-    const int64_t xc = s.use_idx ? (int64_t)s.idx[j] : (int64_t)j;
-    const T *xj = x + xc * ldx;
-    T *yj = y + (int64_t)j * ldy;
-    const T a = (T)s.a[j], b = (T)s.b[j];
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    if (a == T(0)) {
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) yj[i] = b * yj[i];
-    } else if (b == T(0)) {
-        if (a == T(1)) {
-            for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) yj[i] = xj[i];
-        } else {
-            for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) yj[i] = a * xj[i];
-        }
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
+template <bool NT, typename V>
+__device__ __forceinline__ void store_as(V *p, V v)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
+// V consecutive rows of a column from row i on, those below n
+template <typename T, int V, bool NT>
+__device__ __forceinline__ void load_run(const T *__restrict__ c, int64_t i, int64_t n, T (&v)[V])
+{
+    typedef T vec __attribute__((ext_vector_type(V)));
+    if (i + V <= n) {
+        const vec x = load_as<NT>(reinterpret_cast<const vec *>(c + i));
+#pragma unroll
+        for (int t = 0; t < V; t++) v[t] = x[t];
     } else {
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
-            yj[i] = a * xj[i] + b * yj[i];
+#pragma unroll
+        for (int t = 0; t < V; t++) v[t] = i + t < n ? c[i + t] : T(0);
     }
 }
 
+template <typename T, int V, bool NT>
+__device__ __forceinline__ void store_run(T *__restrict__ c, int64_t i, int64_t n, const T (&v)[V])
+{
+    typedef T vec __attribute__((ext_vector_type(V)));
+    if (i + V <= n) {
+        vec x;
+#pragma unroll
+        for (int t = 0; t < V; t++) x[t] = v[t];
+        store_as<NT>(reinterpret_cast<vec *>(c + i), x);
+    } else {
+#pragma unroll
+        for (int t = 0; t < V; t++)
+            if (i + t < n) c[i + t] = v[t];
+    }
+}
+
+// Row of this thread's run; the grid covers the n rows
+template <int V>
+__device__ __forceinline__ int64_t run_row()
+{
+    return ((int64_t)blockIdx.x * kBlock + threadIdx.x) * V;
+}
+
+// ---------------------------------------------------------------- axpby
+template <typename T, int V, bool NT>
+__global__ __launch_bounds__(kBlock) void k_axpby(int64_t n, const T *x, int64_t ldx, T *y, int64_t ldy,
+                                                  ColScalars s)
+{
+    const int j = blockIdx.y;
+    const int64_t i = run_row<V>();
+    if (i >= n) return;
+    const T *xj = x + (s.use_idx ? (int64_t)s.idx[j] : (int64_t)j) * ldx;
+    T *yj = y + (int64_t)j * ldy;
+    const T a = (T)s.a[j], b = (T)s.b[j];
+    T xv[V], yv[V];
+    if (a != T(0)) load_run<T, V, NT>(xj, i, n, xv);
+    if (a == T(0) || b != T(0)) load_run<T, V, NT>(yj, i, n, yv);
+#pragma unroll
+    for (int t = 0; t < V; t++) yv[t] = axpby_el<T>(a, xv[t], b, yv[t]);
+    store_run<T, V, NT>(yj, i, n, yv);
+}
+
 // ---------------------------------------------------------------- dots
+// Thread t of block b adds the rows 256 b + t + 256 gridDim.x m, m = 0, 1, ...
+// in turn, U of them loaded at a time (the order of the sums does not depend
+// on U); f(row, loaded) for each.
+template <int U, typename LD, typename F>
+__device__ __forceinline__ void strided_rows(int64_t n, LD load, F f)
+{
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if constexpr (U > 1) {
+        for (; i + (U - 1) * stride < n; i += U * stride) {
+            decltype(load(i)) v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = load(i + u * stride);
+#pragma unroll
+            for (int u = 0; u < U; u++) f(i + u * stride, v[u]);
+        }
+    }
+    for (; i < n; i += stride) f(i, load(i));
+}
+
 template <typename T>
+struct Pair {
+    T a, b;
+};
+
+template <typename T, int U, bool NT>
 __global__ __launch_bounds__(kBlock) void k_dots(int64_t n, const T *__restrict__ x, int64_t ldx,
                                                  const T *__restrict__ y, int64_t ldy,
                                                  double *__restrict__ partial)
@@ -104,9 +191,9 @@ __global__ __launch_bounds__(kBlock) void k_dots(int64_t n, const T *__restrict_
     const T *xj = x + (int64_t)j * ldx;
     const T *yj = y + (int64_t)j * ldy;
     double acc = 0.0;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
-        acc = fma((double)xj[i], (double)yj[i], acc);
+    strided_rows<U>(
+        n, [&](int64_t i) { return Pair<T>{load_as<NT>(xj + i), load_as<NT>(yj + i)}; },
+        [&](int64_t, const Pair<T> &v) { acc = fma((double)v.a, (double)v.b, acc); });
     const double s = block_sum(acc, sh);
     if (threadIdx.x == 0) partial[(int64_t)j * gridDim.x + blockIdx.x] = s;
 }
@@ -155,14 +242,18 @@ __global__ __launch_bounds__(kBlock) void k_reduce_rows_host(const double *__res
 }
 
 // ---------------------------------------------------------------- copy / swap / rows
-template <typename TX, typename TY>
+template <typename TX, typename TY, int V, bool NT>
 __global__ __launch_bounds__(kBlock) void k_copy(int64_t n, const TX *__restrict__ x, int64_t ldx,
                                                  TY *__restrict__ y, int64_t ldy)
 {
-    const int j = blockIdx.y;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
-        y[(int64_t)j * ldy + i] = (TY)x[(int64_t)j * ldx + i];
+    const int64_t i = run_row<V>();
+    if (i >= n) return;
+    TX xv[V];
+    TY yv[V];
+    load_run<TX, V, NT>(x + (int64_t)blockIdx.y * ldx, i, n, xv);
+#pragma unroll
+    for (int t = 0; t < V; t++) yv[t] = (TY)xv[t];
+    store_run<TY, V, NT>(y + (int64_t)blockIdx.y * ldy, i, n, yv);
 }
 
 template <typename T>
@@ -417,7 +508,11 @@ __global__ __launch_bounds__(kSpmmRows) void k_spmm_long(const int *__restrict__
 // FP64 the compiler's own choice is 207 registers and two wavefronts per
 // SIMD; three are asked for.  27-point matrix of a 96^3 grid, 50 columns:
 // 0.45 ms in FP64 and 0.25 in FP32, against 2.09 and 0.93 gathered from a
-// row-major copy of X (k_spmm_rows).  Every sum still runs over the row in CSR order from 0, so Y is bit-identical to
+// row-major copy of X (k_spmm_rows).  Y bypasses the caches at every size, which
+// leaves them to X's faces (us, FP32 48 columns of 160^3 502 -> 481, FP64 40
+// columns of a 1024^2 grid 168 -> 156, FP32 60 columns of 700^2 53 -> 45; the
+// matrix that way: 160^3 502 -> 557, its lines serve several loads).  Every sum
+// still runs over the row in CSR order from 0, so Y is bit-identical to
 // k_spmm's.  Rows longer than long_thr are left to k_spmm_long.  Row blocks
 // are numbered so that each XCD walks a contiguous range of rows (a stencil's
 // plane neighbours stay in its L2).
@@ -589,7 +684,7 @@ __global__ __launch_bounds__(kSpmmRows, ME > 8 ? 3 : 1) void k_spmm_halo(int n, 
 #pragma unroll
         for (int cc = 0; cc < KC; cc++) {
             const int c = c0 + cc;
-            if (active && c < k) Y[(int64_t)c * ldy + r] = acc[cc];
+            if (active && c < k) store_as<true>(Y + (int64_t)c * ldy + r, acc[cc]);
             if (DOT) d[cc] = (active && c < k) ? (double)xo.v[cc] * (double)acc[cc] : 0.0;
         }
         if (DOT) {
@@ -1180,7 +1275,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(int64_t n, T *__restrict__
 
 // ---------------------------------------------------------------- split CG steps
 // r -= alpha w (VecAxpby(-alpha, w, 1.0, r)); partial r.r  (gcge_cg.c:250-276)
-template <typename T>
+template <typename T, int U, bool NT>
 __global__ __launch_bounds__(kBlock) void k_cg_resid(int64_t n, const T *__restrict__ w, int64_t ldw,
                                                      T *__restrict__ r, int64_t ldr, ColScalars s,
                                                      double *__restrict__ partial)
@@ -1191,12 +1286,13 @@ __global__ __launch_bounds__(kBlock) void k_cg_resid(int64_t n, const T *__restr
     const T *wj = w + (int64_t)j * ldw;
     T *rj = r + (int64_t)j * ldr;
     double acc = 0.0;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
-        const T rn = axpby_el<T>(-al, wj[i], T(1), rj[i]);
-        rj[i] = rn;
-        acc = fma((double)rn, (double)rn, acc);
-    }
+    strided_rows<U>(
+        n, [&](int64_t i) { return Pair<T>{load_as<NT>(wj + i), load_as<NT>(rj + i)}; },
+        [&](int64_t i, const Pair<T> &v) {
+            const T rn = axpby_el<T>(-al, v.a, T(1), v.b);
+            store_as<NT>(rj + i, rn);
+            acc = fma((double)rn, (double)rn, acc);
+        });
     const double bs = block_sum(acc, sh);
     if (threadIdx.x == 0) partial[(int64_t)j * gridDim.x + blockIdx.x] = bs;
 }
@@ -1205,6 +1301,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_resid(int64_t n, const T *__restr
 // k_cg_resid), partial r.z (row 2j) and r.r (row 2j + 1) with z = dinv .* r
 // rounded as k_cg_search<T, true> forms it
 template <typename T>
+struct Triple {
+    T a, b, c;
+};
+
+template <typename T, int U, bool NT>
 __global__ __launch_bounds__(kBlock) void k_pcg_resid(int64_t n, const T *__restrict__ w, int64_t ldw,
                                                       T *__restrict__ r, int64_t ldr, const T *__restrict__ dinv,
                                                       ColScalars s, double *__restrict__ partial)
@@ -1215,14 +1316,15 @@ __global__ __launch_bounds__(kBlock) void k_pcg_resid(int64_t n, const T *__rest
     const T *wj = w + (int64_t)j * ldw;
     T *rj = r + (int64_t)j * ldr;
     double arz = 0.0, arr = 0.0;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
-        const T rn = axpby_el<T>(-al, wj[i], T(1), rj[i]);
-        const T zn = rn * dinv[i];
-        rj[i] = rn;
-        arz = fma((double)rn, (double)zn, arz);
-        arr = fma((double)rn, (double)rn, arr);
-    }
+    strided_rows<U>(
+        n, [&](int64_t i) { return Triple<T>{load_as<NT>(wj + i), load_as<NT>(rj + i), dinv[i]}; },
+        [&](int64_t i, const Triple<T> &v) {
+            const T rn = axpby_el<T>(-al, v.a, T(1), v.b);
+            const T zn = rn * v.c;
+            store_as<NT>(rj + i, rn);
+            arz = fma((double)rn, (double)zn, arz);
+            arr = fma((double)rn, (double)rn, arr);
+        });
     const double brz = block_sum(arz, sh);
     const double brr = block_sum(arr, sh);
     if (threadIdx.x == 0) {
@@ -1250,31 +1352,34 @@ __global__ __launch_bounds__(kBlock) void k_diag_inv(int n, const int *__restric
 // p = r + beta p (MultiVecAxpbyDiag(1, r, beta, p)) for the columns j < kp
 // With PRE, the search direction is built from z = dinv .* r (the Jacobi-
 // preconditioned residual, formed here rather than stored).
-template <typename T, bool PRE>
+template <typename T, bool PRE, int V, bool NT>
 __global__ __launch_bounds__(kBlock) void k_cg_search(int64_t n, T *__restrict__ x, int64_t ldx,
                                                       T *__restrict__ p, int64_t ldp, const T *__restrict__ r,
                                                       int64_t ldr, int kx, int kp, ColScalars s,
                                                       const T *__restrict__ dinv)
 {
     const int j = blockIdx.y;
+    const int64_t i = run_row<V>();
+    if (i >= n) return;
     const T al = (T)s.a[j], be = (T)s.b[j];
     T *xj = x + (int64_t)j * ldx;
     T *pj = p + (int64_t)j * ldp;
-    const T *rj = r + (int64_t)j * ldr;
-    const bool dx = j < kx, dp = j < kp;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    if (dx && dp) {
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) {
-            const T pv = pj[i];
-            xj[i] = axpby_el<T>(al, pv, T(1), xj[i]);
-            pj[i] = axpby_el<T>(T(1), PRE ? rj[i] * dinv[i] : rj[i], be, pv);
-        }
-    } else if (dx) {
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
-            xj[i] = axpby_el<T>(al, pj[i], T(1), xj[i]);
-    } else if (dp) {
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
-            pj[i] = axpby_el<T>(T(1), PRE ? rj[i] * dinv[i] : rj[i], be, pj[i]);
+    T pv[V], xv[V], rv[V], dv[V];
+    load_run<T, V, NT>(pj, i, n, pv);
+    if (j < kx) load_run<T, V, NT>(xj, i, n, xv);
+    if (j < kp) {
+        load_run<T, V, NT>(r + (int64_t)j * ldr, i, n, rv);
+        if (PRE) load_run<T, V, false>(dinv, i, n, dv);
+    }
+    if (j < kx) {
+#pragma unroll
+        for (int t = 0; t < V; t++) xv[t] = axpby_el<T>(al, pv[t], T(1), xv[t]);
+        store_run<T, V, NT>(xj, i, n, xv);
+    }
+    if (j < kp) {
+#pragma unroll
+        for (int t = 0; t < V; t++) pv[t] = axpby_el<T>(T(1), PRE ? rv[t] * dv[t] : rv[t], be, pv[t]);
+        store_run<T, V, NT>(pj, i, n, pv);
     }
 }
 
@@ -1344,19 +1449,61 @@ static ColScalars make_scalars(int k, const double *a, const double *b, const in
     return s;
 }
 
+// Every access of 16 bytes aligned: column starts and distances
+static bool wide_ok(int prec, std::initializer_list<const void *> ptrs, std::initializer_list<int64_t> lds)
+{
+    for (const void *p : ptrs)
+        if ((uintptr_t)p & 15u) return false;
+    for (int64_t ld : lds)
+        if (ld * (int64_t)elem_size(prec) % 16) return false;
+    return true;
+}
+
+// Grid of an element-wise kernel: every thread one run of V rows
+static dim3 run_grid(int64_t n, int V, int k) { return dim3((unsigned)((n + (int64_t)kBlock * V - 1) / (kBlock * V)), k); }
+
+// Calls f(V, NT) with constants: 16-byte accesses where aligned, past the
+// caches where more than kStreamBytes are touched
+template <typename T, typename F>
+static void run_variant(bool wide, double bytes, F f)
+{
+    using W = std::integral_constant<int, kWide<T>>;
+    if (!wide) f(std::integral_constant<int, 1>{}, std::false_type{});
+    else if (bytes > kStreamBytes) f(W{}, std::true_type{});
+    else f(W{}, std::false_type{});
+}
+
+// Calls f(U, NT) for the strided sums: 8 rows at a time past the caches; 4 at a
+// time where threads have many (2 columns of 4.1M rows in FP32, residual update
+// 23.9 -> 16.4 us), else one (16,384 rows, 20 columns: 2.7 us, 3.2 with 4)
+template <typename F>
+static void sum_variant(int64_t n, double bytes, F f)
+{
+    if (bytes > kStreamBytes) f(std::integral_constant<int, 8>{}, std::true_type{});
+    else if (n >= 1 << 20) f(std::integral_constant<int, 4>{}, std::false_type{});
+    else f(std::integral_constant<int, 1>{}, std::false_type{});
+}
+
+template <typename T>
+static void axpby_t(int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k, const ColScalars &s,
+                    bool wide, double bytes)
+{
+    run_variant<T>(wide, bytes, [&](auto V, auto NT) {
+        k_axpby<T, V(), NT()><<<run_grid(n, V(), k), kBlock, 0, ctx().stream>>>(n, (const T *)x, ldx, (T *)y, ldy, s);
+    });
+}
+
 void launch_axpby(int prec, int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k,
                   const double *a, const double *b, const int *xidx)
 {
     if (k <= 0 || n <= 0 || failed()) return;
     ColScalars s = make_scalars(k, a, b, xidx);
-    dim3 grid(grid_1d(n, 1024), k);
     double bytes = 0.0;
     for (int j = 0; j < k; j++) bytes += (double)n * elem_size(prec) * ((s.a[j] == 0.0 || s.b[j] == 0.0) ? 2 : 3);
     ProfScope ps(K_AXPBY, bytes, 0.0);
-    if (prec == GCGE_HIP_FP64)
-        k_axpby<double><<<grid, kBlock, 0, ctx().stream>>>(n, (const double *)x, ldx, (double *)y, ldy, s);
-    else
-        k_axpby<float><<<grid, kBlock, 0, ctx().stream>>>(n, (const float *)x, ldx, (float *)y, ldy, s);
+    const bool wide = wide_ok(prec, {x, y}, {ldx, ldy});
+    if (prec == GCGE_HIP_FP64) axpby_t<double>(n, x, ldx, y, ldy, k, s, wide, bytes);
+    else axpby_t<float>(n, x, ldx, y, ldy, k, s, wide, bytes);
     check(hipGetLastError(), "k_axpby");
 }
 
@@ -1376,11 +1523,15 @@ int dots_blocks(int64_t n) { return grid_1d(n, 256); }
 static void launch_dots(int prec, int64_t n, const void *x, int64_t ldx, const void *y, int64_t ldy, int k,
                         double *partial, int nb)
 {
-    dim3 grid(nb, k);
-    if (prec == GCGE_HIP_FP64)
-        k_dots<double><<<grid, kBlock, 0, ctx().stream>>>(n, (const double *)x, ldx, (const double *)y, ldy, partial);
-    else
-        k_dots<float><<<grid, kBlock, 0, ctx().stream>>>(n, (const float *)x, ldx, (const float *)y, ldy, partial);
+    const dim3 grid(nb, k);
+    sum_variant(n, 2.0 * k * (double)n * elem_size(prec), [&](auto U, auto NT) {
+        if (prec == GCGE_HIP_FP64)
+            k_dots<double, U(), NT()><<<grid, kBlock, 0, ctx().stream>>>(n, (const double *)x, ldx,
+                                                                         (const double *)y, ldy, partial);
+        else
+            k_dots<float, U(), NT()><<<grid, kBlock, 0, ctx().stream>>>(n, (const float *)x, ldx, (const float *)y,
+                                                                        ldy, partial);
+    });
 }
 
 bool dots(int prec, int64_t n, const void *x, int64_t ldx, const void *y, int64_t ldy, int k,
@@ -1418,20 +1569,30 @@ bool dots_with(int prec, int64_t n, const void *x, int64_t ldx, const void *y, i
     return check(hipStreamSynchronize(ctx().stream), "hipStreamSynchronize");
 }
 
+template <typename TX, typename TY>
+static void copy_t(int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k, bool wide, double bytes)
+{
+    // accesses of 16 bytes on the narrower side, 16 or 32 on the other
+    using T = std::conditional_t<(sizeof(TX) < sizeof(TY)), TX, TY>;
+    run_variant<T>(wide, bytes, [&](auto V, auto NT) {
+        k_copy<TX, TY, V(), NT()><<<run_grid(n, V(), k), kBlock, 0, ctx().stream>>>(n, (const TX *)x, ldx, (TY *)y,
+                                                                                    ldy);
+    });
+}
+
 void launch_copy(int xprec, const void *x, int64_t ldx, int yprec, void *y, int64_t ldy, int64_t n, int k)
 {
     if (k <= 0 || n <= 0 || failed()) return;
-    dim3 grid(grid_1d(n, 1024), k);
-    hipStream_t st = ctx().stream;
-    ProfScope ps(K_COPY, (double)k * n * (elem_size(xprec) + elem_size(yprec)), 0.0);
-    if (xprec == GCGE_HIP_FP64 && yprec == GCGE_HIP_FP64)
-        k_copy<double, double><<<grid, kBlock, 0, st>>>(n, (const double *)x, ldx, (double *)y, ldy);
-    else if (xprec == GCGE_HIP_FP64)
-        k_copy<double, float><<<grid, kBlock, 0, st>>>(n, (const double *)x, ldx, (float *)y, ldy);
-    else if (yprec == GCGE_HIP_FP64)
-        k_copy<float, double><<<grid, kBlock, 0, st>>>(n, (const float *)x, ldx, (double *)y, ldy);
-    else
-        k_copy<float, float><<<grid, kBlock, 0, st>>>(n, (const float *)x, ldx, (float *)y, ldy);
+    const double bytes = (double)k * n * (elem_size(xprec) + elem_size(yprec));
+    ProfScope ps(K_COPY, bytes, 0.0);
+    // a run of 4 rows in FP64 is one vector of 32 bytes
+    const bool mixed = xprec != yprec;
+    const bool wide = wide_ok(xprec, {x}, {ldx}) && wide_ok(yprec, {y}, {ldy}) &&
+                      (!mixed || ((((uintptr_t)x | (uintptr_t)y) & 31u) == 0 && ldx % 8 == 0 && ldy % 8 == 0));
+    if (xprec == GCGE_HIP_FP64 && yprec == GCGE_HIP_FP64) copy_t<double, double>(n, x, ldx, y, ldy, k, wide, bytes);
+    else if (xprec == GCGE_HIP_FP64) copy_t<double, float>(n, x, ldx, y, ldy, k, wide, bytes);
+    else if (yprec == GCGE_HIP_FP64) copy_t<float, double>(n, x, ldx, y, ldy, k, wide, bytes);
+    else copy_t<float, float>(n, x, ldx, y, ldy, k, wide, bytes);
     check(hipGetLastError(), "k_copy");
 }
 
@@ -1858,12 +2019,16 @@ bool cg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t 
         {
             ProfScope ps(prec == GCGE_HIP_FP64 ? K_CG_UPDATE_F64 : K_CG_UPDATE_F32,
                          3.0 * kc * (double)n * elem_size(prec), 4.0 * kc * (double)n);
-            if (prec == GCGE_HIP_FP64)
-                k_cg_resid<double><<<grid, kBlock, 0, ctx().stream>>>(
-                    n, (const double *)w + (int64_t)c0 * ldw, ldw, (double *)r + (int64_t)c0 * ldr, ldr, s, partial);
-            else
-                k_cg_resid<float><<<grid, kBlock, 0, ctx().stream>>>(
-                    n, (const float *)w + (int64_t)c0 * ldw, ldw, (float *)r + (int64_t)c0 * ldr, ldr, s, partial);
+            sum_variant(n, 2.0 * kc * (double)n * elem_size(prec), [&](auto U, auto NT) {
+                if (prec == GCGE_HIP_FP64)
+                    k_cg_resid<double, U(), NT()><<<grid, kBlock, 0, ctx().stream>>>(
+                        n, (const double *)w + (int64_t)c0 * ldw, ldw, (double *)r + (int64_t)c0 * ldr, ldr, s,
+                        partial);
+                else
+                    k_cg_resid<float, U(), NT()><<<grid, kBlock, 0, ctx().stream>>>(
+                        n, (const float *)w + (int64_t)c0 * ldw, ldw, (float *)r + (int64_t)c0 * ldr, ldr, s,
+                        partial);
+            });
         }
         if (!check(hipGetLastError(), "k_cg_resid")) return false;
         if (!reduce_to_host(partial, kc, nb, rr + c0)) return false;
@@ -1887,14 +2052,16 @@ bool pcg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t
         {
             ProfScope ps(prec == GCGE_HIP_FP64 ? K_CG_UPDATE_F64 : K_CG_UPDATE_F32,
                          3.0 * kc * (double)n * elem_size(prec) + (double)n * elem_size(prec), 6.0 * kc * (double)n);
-            if (prec == GCGE_HIP_FP64)
-                k_pcg_resid<double><<<grid, kBlock, 0, ctx().stream>>>(
-                    n, (const double *)w + (int64_t)c0 * ldw, ldw, (double *)r + (int64_t)c0 * ldr, ldr,
-                    (const double *)dinv, s, partial);
-            else
-                k_pcg_resid<float><<<grid, kBlock, 0, ctx().stream>>>(
-                    n, (const float *)w + (int64_t)c0 * ldw, ldw, (float *)r + (int64_t)c0 * ldr, ldr,
-                    (const float *)dinv, s, partial);
+            sum_variant(n, 2.0 * kc * (double)n * elem_size(prec), [&](auto U, auto NT) {
+                if (prec == GCGE_HIP_FP64)
+                    k_pcg_resid<double, U(), NT()><<<grid, kBlock, 0, ctx().stream>>>(
+                        n, (const double *)w + (int64_t)c0 * ldw, ldw, (double *)r + (int64_t)c0 * ldr, ldr,
+                        (const double *)dinv, s, partial);
+                else
+                    k_pcg_resid<float, U(), NT()><<<grid, kBlock, 0, ctx().stream>>>(
+                        n, (const float *)w + (int64_t)c0 * ldw, ldw, (float *)r + (int64_t)c0 * ldr, ldr,
+                        (const float *)dinv, s, partial);
+            });
         }
         if (!check(hipGetLastError(), "k_pcg_resid")) return false;
         if (!reduce_to_host(partial, 2 * kc, nb, tmp.data())) return false;
@@ -1918,7 +2085,7 @@ void launch_cg_search(int prec, int64_t n, void *x, int64_t ldx, void *p, int64_
 {
     const int k = std::max(kx, kp);
     if (k <= 0 || failed()) return;
-    const int nb = grid_1d(n, 1024);
+    const bool wide = wide_ok(prec, {x, p, r, dinv}, {ldx, ldp, ldr});
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         const int kxc = std::max(0, std::min(kc, kx - c0)), kpc = std::max(0, std::min(kc, kp - c0));
@@ -1926,17 +2093,18 @@ void launch_cg_search(int prec, int64_t n, void *x, int64_t ldx, void *p, int64_
         for (int j = 0; j < kxc; j++) aa[j] = alpha[c0 + j];
         for (int j = 0; j < kpc; j++) bb[j] = beta[c0 + j];
         ColScalars s = make_scalars(kc, aa.data(), bb.data(), nullptr);
-        dim3 grid(nb, kc);
         {
             ProfScope ps(prec == GCGE_HIP_FP64 ? K_CG_SEARCH_F64 : K_CG_SEARCH_F32,
                          (3.0 * kxc + 3.0 * kpc - 1.0 * std::min(kxc, kpc)) * (double)n * elem_size(prec) +
                              (dinv && kpc > 0 ? (double)n * elem_size(prec) : 0.0),
                          0.0);
+            const double held = (1.0 * kxc + kpc + kc) * (double)n * elem_size(prec);  // x, r and p
 #define GH_SEARCH(T_, PRE_)                                                                                     \
-    k_cg_search<T_, PRE_><<<grid, kBlock, 0, ctx().stream>>>(n, (T_ *)x + (int64_t)c0 * ldx, ldx,              \
-                                                              (T_ *)p + (int64_t)c0 * ldp, ldp,              \
-                                                              (const T_ *)r + (int64_t)c0 * ldr, ldr, kxc, kpc, \
-                                                              s, (const T_ *)dinv)
+    run_variant<T_>(wide, held, [&](auto V, auto NT) {                                                          \
+        k_cg_search<T_, PRE_, V(), NT()><<<run_grid(n, V(), kc), kBlock, 0, ctx().stream>>>(                    \
+            n, (T_ *)x + (int64_t)c0 * ldx, ldx, (T_ *)p + (int64_t)c0 * ldp, ldp,                              \
+            (const T_ *)r + (int64_t)c0 * ldr, ldr, kxc, kpc, s, (const T_ *)dinv);                             \
+    })
             if (prec == GCGE_HIP_FP64) {
                 if (dinv) GH_SEARCH(double, true);
                 else GH_SEARCH(double, false);

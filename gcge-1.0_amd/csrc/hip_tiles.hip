@@ -546,44 +546,61 @@ __global__ __launch_bounds__(kThreads) void k_sum_chunks(const double *__restric
 // column block; from L2 these reads cost as much as the products); X is
 // loaded one panel ahead into registers.  Bound by the matrix cores for large
 // p and q (a large library product reaches 67 TF here in FP64, 153 in FP32).
-// Over 4.1M rows, 300 x 100: FP64 6.73 -> 5.03 ms (49 TF), FP32 3.44 -> 2.76
-// (89 TF); 100 x 100: 2.86 -> 2.10 and 1.45 -> 1.33; 300 x 130 (two passes of
-// 5 blocks): 12.5 -> 7.3 and 6.5 -> 3.9.  Every sum runs over k in ascending
+// Over 4.1M rows, ms, C from L2 at first, then from LDS, then with the panels'
+// order pinned and Y's old values loaded ahead: FP32 300 x 100 3.44, 2.76, 2.58
+// (95 TF); 100 x 100 1.45, 1.28, 0.98; 200 x 100 added to Y 2.24 -> 1.97; 300 x
+// 130 (two passes of 5 blocks) 6.5, 3.8, 3.5; FP64 300 x 100 6.73, 5.19, 5.18
+// (47 TF, 53 with the padding); 100 x 100 2.86, 2.11, 2.00; 300 x 130 12.5, 7.2,
+// 7.0.  Every sum runs over k in ascending
 // blocks of 4, whatever RB and RN.
 
-// y[0..V) = beta y + alpha v with the branch rules of y = a x + b y, one
-// access of V elements
-template <typename T, int V>
-__device__ __forceinline__ void store_rows(T *y, const T (&v)[V], T al, T be, int64_t room)
-{
-    struct alignas(V * sizeof(T)) Vec {
-        T e[V];
-    };
-    if (room >= V) {
-        Vec out;
-        if (be == T(0)) {
-#pragma unroll
-            for (int t = 0; t < V; t++) out.e[t] = (al == T(1)) ? v[t] : al * v[t];
-        } else {
-            const Vec old = *reinterpret_cast<const Vec *>(y);
-#pragma unroll
-            for (int t = 0; t < V; t++) out.e[t] = be * old.e[t] + al * v[t];
-        }
-        *reinterpret_cast<Vec *>(y) = out;
-    } else {
-#pragma unroll
-        for (int t = 0; t < V; t++)
-            if (t < room) y[t] = (be == T(0)) ? ((al == T(1)) ? v[t] : al * v[t]) : be * y[t] + al * v[t];
-    }
-}
-
 // A wavefront's results to Y: slot t of lane group kk is operand row
-// drow(kk, t), column block r column 16 (g0 + r) + m
+// drow(kk, t), column block r column 16 (g0 + r) + m.  Where all rows exist,
+// the old values of a column block are loaded before the block in front of it
+// is stored: one access at a time, 28 of them in turn cost more than the
+// products.
 template <typename T, int RN, int RB>
 __device__ __forceinline__ void store_tile(const typename MT<T>::acc_t (&acc)[RB][RN], T *__restrict__ Y,
                                            int64_t ldy, int g0, int q, int64_t rw, int64_t n, T al, T be)
 {
+    typedef T vec __attribute__((ext_vector_type(RB)));
     const int m = threadIdx.x & 15, kk = (threadIdx.x & 63) >> 4;
+    if (rw + 16 * RB <= n) {
+        auto at = [&](int r, int t) {
+            const int j = min((g0 + r) * 16 + m, q - 1);
+            return reinterpret_cast<vec *>(Y + (int64_t)j * ldy + rw + MT<T>::spread(MT<T>::drow(kk, t)) * RB);
+        };
+        if (be == T(0)) {
+#pragma unroll
+            for (int r = 0; r < RN; r++)
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    vec v;
+#pragma unroll
+                    for (int h = 0; h < RB; h++) v[h] = (al == T(1)) ? (T)acc[h][r][t] : al * (T)acc[h][r][t];
+                    if ((g0 + r) * 16 + m < q) *at(r, t) = v;
+                }
+        } else {
+            vec old[2][4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) old[0][t] = *at(0, t);
+#pragma unroll
+            for (int r = 0; r < RN; r++) {
+                if (r + 1 < RN) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++) old[(r + 1) & 1][t] = *at(r + 1, t);
+                }
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    vec v;
+#pragma unroll
+                    for (int h = 0; h < RB; h++) v[h] = be * old[r & 1][t][h] + al * (T)acc[h][r][t];
+                    if ((g0 + r) * 16 + m < q) *at(r, t) = v;
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < RN; r++) {
         const int j = (g0 + r) * 16 + m;
@@ -592,10 +609,12 @@ __device__ __forceinline__ void store_tile(const typename MT<T>::acc_t (&acc)[RB
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const int64_t row = rw + MT<T>::spread(MT<T>::drow(kk, t)) * RB;
-            T v[RB];
 #pragma unroll
-            for (int h = 0; h < RB; h++) v[h] = (T)acc[h][r][t];
-            store_rows<T, RB>(yj + row, v, al, be, n - row);
+            for (int h = 0; h < RB; h++) {
+                const T v = (T)acc[h][r][t];
+                if (row + h < n)
+                    yj[row + h] = (be == T(0)) ? ((al == T(1)) ? v : al * v) : be * yj[row + h] + al * v;
+            }
         }
     }
 }
@@ -611,11 +630,17 @@ __global__ __launch_bounds__(kThreads, RN <= 2 ? 4 : RN <= 4 ? 3 : 2) void k_lin
     constexpr int E = 16 / (int)sizeof(T);       // elements of a 16-byte copy unit
     constexpr int UNITS = KP * RN * 64 / E;
     constexpr int UPT = (UNITS + kThreads - 1) / kThreads;
+    // The order of a panel's loads, LDS reads and products is pinned: left to
+    // the compiler the loads of X sink to the panel's end, where they are
+    // waited for.  FP64 of up to 4 column blocks has three wavefronts per SIMD
+    // to cover them and loses 4 - 6 % by it (100 x 50: 1.15 against 1.18 ms).
+    constexpr bool PIN = sizeof(T) == 4 || RN > 4;
+    constexpr int READS = (RN + 1) / 2;          // LDS reads of a k block's operands, two at a time
     typedef T u16 __attribute__((ext_vector_type(E)));
     struct alignas(RB * sizeof(T)) Rows {
         T e[RB];
     };
-    __shared__ __attribute__((aligned(16))) T sc[2][KP * RN * 64];
+    __shared__ __attribute__((aligned(16))) T sc[2][UPT * kThreads * E];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int m = lane & 15, kk = lane >> 4;
     // rows past n up to the next multiple of 64 RB <= 256 lie in the columns'
@@ -646,8 +671,9 @@ __global__ __launch_bounds__(kThreads, RN <= 2 ? 4 : RN <= 4 ? 3 : 2) void k_lin
         auto park = [&](int pan) {
 #pragma unroll
             for (int u = 0; u < UPT; u++) {
-                const int unit = threadIdx.x + u * kThreads;
-                if (UNITS % kThreads == 0 || unit < UNITS) *reinterpret_cast<u16 *>(&sc[pan & 1][unit * E]) = creg[u];
+                // units past UNITS fill the buffer's end: no branch, in which
+                // the load would be waited for
+                *reinterpret_cast<u16 *>(&sc[pan & 1][(threadIdx.x + u * kThreads) * E]) = creg[u];
             }
             const bool whole = (pan + 1) * KP * 4 <= p;
 #pragma unroll
@@ -661,29 +687,57 @@ __global__ __launch_bounds__(kThreads, RN <= 2 ? 4 : RN <= 4 ? 3 : 2) void k_lin
         for (int h = 0; h < RB; h++)
 #pragma unroll
             for (int r = 0; r < RN; r++) acc[h][r] = acc_t{};
-        auto products = [&](int i, const T *c) {
-            T bb[RN];
-#pragma unroll
-            for (int r = 0; r < RN; r++) bb[r] = c[(i * RN + r) * 64 + lane];
+        auto products = [&](int i, const T (&bb)[RN]) {
 #pragma unroll
             for (int r = 0; r < RN; r++)
 #pragma unroll
                 for (int h = 0; h < RB; h++) acc[h][r] = MT<T>::mma(a[i].e[h], bb[r], acc[h][r]);
+        };
+        auto read = [&](int i, const T *c, T (&bb)[RN]) {
+#pragma unroll
+            for (int r = 0; r < RN; r++) bb[r] = c[(i * RN + r) * 64 + lane];
         };
         fetch(0);
         park(0);
         __syncthreads();
         for (int pan = 0; pan + 1 < npan; pan++) {
             fetch(pan + 1);
+            if constexpr (!PIN) {
 #pragma unroll
-            for (int i = 0; i < KP; i++) products(i, sc[pan & 1]);
+                for (int i = 0; i < KP; i++) {
+                    T bb[RN];
+                    read(i, sc[pan & 1], bb);
+                    products(i, bb);
+                }
+            } else {
+                __builtin_amdgcn_sched_barrier(0);  // issued before the products, not where they are used
+                T bb[2][RN];
+                read(0, sc[pan & 1], bb[0]);
+#pragma unroll
+                for (int i = 0; i < KP; i++) {
+                    if (i + 1 < KP) read(i + 1, sc[pan & 1], bb[(i + 1) & 1]);
+                    products(i, bb[i & 1]);
+                }
+                // C's operands one k block ahead of the products
+                __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+#pragma unroll
+                for (int i = 0; i < KP; i++) {
+                    if (i + 1 < KP) __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, RN * RB, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // the loads are looked at after the products
+            }
             park(pan + 1);
             __syncthreads();
         }
         // the last panel: 1 .. KP k blocks
 #pragma unroll
         for (int i = 0; i < KP; i++)
-            if ((npan - 1) * KP + i < nkb) products(i, sc[(npan - 1) & 1]);
+            if ((npan - 1) * KP + i < nkb) {
+                T bb[RN];
+                read(i, sc[(npan - 1) & 1], bb);
+                products(i, bb);
+            }
         __syncthreads();  // the next pass overwrites sc
         store_tile<T, RN, RB>(acc, Y, ldy, g0, q, rw, n, al, be);
     }

@@ -281,6 +281,47 @@ bool wait_seq(size_t count, unsigned long long want)
     return i == count;
 }
 
+// A partial sum that is not there yet: a NaN that no arithmetic produces.  One
+// that carries just these bits all the same (from the caller's data) costs the
+// synchronization after 20 ms, no more.
+constexpr unsigned long long kNotYet = 0x7ffda3c96e1d8b47ull;
+
+double *host_partials(size_t count)
+{
+    if (!ensure_ctx()) return nullptr;
+    if (!g_ctx.hpart && !check(hipHostMalloc((void **)&g_ctx.hpart, sizeof(double) * kHostPartials,
+                                             hipHostMallocCoherent),
+                               "hipHostMalloc")) {
+        g_ctx.hpart = nullptr;
+        return nullptr;
+    }
+    auto *p = reinterpret_cast<unsigned long long *>(g_ctx.hpart);
+    for (size_t i = 0; i < count; i++) __atomic_store_n(p + i, kNotYet, __ATOMIC_RELAXED);
+    return g_ctx.hpart;
+}
+
+bool wait_partials(size_t count)
+{
+    const auto *p = reinterpret_cast<const unsigned long long *>(g_ctx.hpart);
+    size_t i = 0;
+    const auto arrived = [&] {
+        while (i < count && __atomic_load_n(p + i, __ATOMIC_ACQUIRE) != kNotYet) i++;
+        return i == count;
+    };
+    if (g_pending.empty()) {
+        const auto t0 = std::chrono::steady_clock::now();
+        for (unsigned spin = 1; !arrived(); spin++) {
+            __builtin_ia32_pause();
+            if (spin % 4096 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) break;
+        }
+        if (i == count) {
+            g_ctx.stage_off = 0;  // copies staged before the launch have completed
+            return true;
+        }
+    }
+    return sync();  // the launch has completed: what is there is the result
+}
+
 void *stage_to_device(const void *host, size_t bytes)
 {
     if (!ensure_ctx()) return nullptr;

@@ -22,6 +22,7 @@ constexpr uint32_t kMagicMat = 0x54414d48u;  // HIP_MAT
 
 constexpr int kMaxCols = 128;     // per-launch column batch for per-column scalars (2.5 KB of kernel arguments)
 constexpr int kMaxChunks = 512;   // split-n partial sums of reductions
+constexpr size_t kHostPartials = 2048;  // most partial sums that are added on the host
 
 struct MV;
 
@@ -111,6 +112,8 @@ struct Ctx {
     unsigned long long *hseq = nullptr;
     size_t hseq_count = 0;
     unsigned long long seq = 0;  // the last launch's
+    // partial sums of a small launch, in coherent host memory: the host adds them
+    double *hpart = nullptr;
     double dev_bytes = 0.0;
     int num_cu = 0;
     // host->device staging ring (pinned host side, device side)
@@ -134,6 +137,11 @@ unsigned long long *host_seq(size_t count, unsigned long long *next);
 // Waits until the first count numbers are all `want`, written by kernels
 // queued on the stream; false (latched) when it has drained without them.
 bool wait_seq(size_t count, unsigned long long want);
+// Host memory for `count` <= kHostPartials partial sums that the next launch
+// writes, marked as not yet written; null (latched) without memory.
+double *host_partials(size_t count);
+// Waits until the launch has written all of them; false (latched) on an error.
+bool wait_partials(size_t count);
 // Copy small host data (coefficients) to device memory without blocking:
 // the bytes go through a pinned ring whose slots are reused only after the
 // next stream synchronisation.  Returns the device address.

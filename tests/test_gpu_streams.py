@@ -80,3 +80,24 @@ def test_copy_converts_and_keeps_padding(ops):
     ops.copy(x, f, xs=1, ys=2, k=5)
     ops.copy(f, y, xs=2, ys=0, k=5)
     assert np.array_equal(y.get()[:, :5], H[:n, 1:6].astype(np.float32).astype(np.float64))
+
+
+def test_few_partial_sums(ops):
+    """8 columns of 256 blocks are added on the host, 9 on the device, in one
+    order; a NaN with the bits that mark a sum as not there yet ends in NaN."""
+    A = Matrix(P.lap2d(300)[0])
+    n, g = 90000, np.random.default_rng(3)
+    x, y = MultiVec(A, 9, F64), MultiVec(A, 9, F64)
+    X = np.asfortranarray(g.standard_normal((n, 9)))
+    x.set(X)
+    y.set(np.asfortranarray(g.standard_normal((n, 9))))
+    nine = ops.dots(x, y)
+    assert np.array_equal(ops.dots(x, y, 8), nine[:8])
+    assert np.array_equal(ops.dots(x, y, 1), nine[:1])
+    X[5, 3] = np.array([0x7ff5a3c96e1d8b47], dtype=np.uint64).view(np.float64)[0]
+    X[6, 4] = np.array([0x7ffda3c96e1d8b47], dtype=np.uint64).view(np.float64)[0]
+    x.set(X)
+    got = ops.dots(x, y, 8)
+    assert np.all(np.isnan(got) == [False] * 3 + [True] * 2 + [False] * 3)
+    got[3:5] = nine[3:5]
+    assert np.array_equal(got, nine[:8])

@@ -87,6 +87,7 @@ struct HIP_MAT_ {
     int *perm_h;              // n: new position -> the caller's row
     int *iperm_h;             // n: the caller's row -> new position
     int *nzmap_h;             // nnz: the caller's entry index -> stored entry index
+    int *perm_d, *nzmap_d;    // device copies of perm_h and nzmap_h (built on demand)
 };
 
 // largest LDS slot count per column of a k_spmm_halo row block
@@ -130,6 +131,7 @@ bool ensure_ctx();
 bool noalloc_setup(int device);
 void *scratch(size_t bytes);           // device scratch of at least bytes
 void *row_stage(size_t bytes);         // device staging of row-major X copies (SpMM), at least bytes
+void *try_row_stage(size_t bytes);     // the same, null without an error where memory is short
 double *host_buf(size_t count);        // pinned host doubles, writable by kernels
 // The first count numbers and the next launch's (one report at a time: the
 // launch, then wait_seq); null (latched) without memory.
@@ -187,6 +189,9 @@ size_t elem_size(int prec);
 void *col_ptr(MV *m, int64_t c);
 const float *mat_val32(HIP_MAT *A);
 const int *mat_rowidx(HIP_MAT *A);
+// device copies of the row order and of the entry order (built on first use)
+const int *mat_perm(HIP_MAT *A);
+const int *mat_nzmap(HIP_MAT *A);
 // 1 / diagonal of A in the given precision (built on first use)
 const void *mat_dinv(HIP_MAT *A, int prec);
 
@@ -238,9 +243,14 @@ bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, in
 // per-nonzero sampled outer product g_e = sum_i w_i x_i[row_e] x_i[col_e]
 bool sampled_outer(int prec, HIP_MAT *A, const void *X, int64_t ldx, int k, const double *w,
                    double *g_dev);
-// grad[p] = scale * sum_t jval[t] g[jnz[t]] over t in [jrowptr[p], jrowptr[p+1]),
-// added to grad[p] when accumulate
-void launch_csr_gather_sum(int nparam, const int *jrowptr, const int *jnz, const double *jval,
-                           const double *g, double *grad, double scale, bool accumulate);
+// grad[p] = scale * sum_t jval[t] g[map[jnz[t]]] over t in [jrowptr[p],
+// jrowptr[p+1]) (map null: g[jnz[t]]), added to grad[p] when accumulate; *bad
+// (host memory) becomes 1 when a jnz[t] lies outside [0, nnz)
+void launch_csr_gather_sum(int nparam, const int *jrowptr, const int *jnz, const double *jval, const int *map,
+                           int nnz, const double *g, double *grad, double scale, bool accumulate, double *bad);
+// y_j[i] = x_j[perm[i]] (perm null: x_j[i]), x in FP64 with distance ldx, and
+// the reverse x_j[perm[i]] = y_j[i]; j < k
+void launch_rows_in(int prec, int64_t n, const double *x, int64_t ldx, const int *perm, void *y, int64_t ldy, int k);
+void launch_rows_out(int prec, int64_t n, double *x, int64_t ldx, const int *perm, const void *y, int64_t ldy, int k);
 
 }  // namespace gh

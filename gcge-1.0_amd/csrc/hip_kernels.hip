@@ -1405,14 +1405,45 @@ __global__ __launch_bounds__(kBlock) void k_sampled_outer(int nnz, const int *__
 __global__ __launch_bounds__(kBlock) void k_csr_gather_sum(int nparam, const int *__restrict__ jrp,
                                                            const int *__restrict__ jnz,
                                                            const double *__restrict__ jval,
+                                                           const int *__restrict__ map, int nnz,
                                                            const double *__restrict__ g,
-                                                           double *__restrict__ grad, double scale, int accumulate)
+                                                           double *__restrict__ grad, double scale, int accumulate,
+                                                           double *__restrict__ bad)
 {
     const int p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= nparam) return;
     double acc = 0.0;
-    for (int t = jrp[p]; t < jrp[p + 1]; t++) acc = fma(jval[t], g[jnz[t]], acc);
+    bool out = false;
+    for (int t = jrp[p]; t < jrp[p + 1]; t++) {
+        const int e = jnz[t];
+        if (e < 0 || e >= nnz) {
+            out = true;
+            continue;
+        }
+        acc = fma(jval[t], g[map ? map[e] : e], acc);
+    }
+    if (out) *bad = 1.0;
     grad[p] = accumulate ? fma(scale, acc, grad[p]) : scale * acc;
+}
+
+// Host columns, as they lie in the staging buffer, into a multivector's row
+// order and precision, and back: the permutation of 16 columns of 262,144 rows
+// costs 30 us here and 1.7 ms on the host
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_rows_in(int64_t n, const double *__restrict__ x, int64_t ldx,
+                                                    const int *__restrict__ perm, T *__restrict__ y, int64_t ldy)
+{
+    const int64_t i = run_row<1>();
+    if (i < n) y[(int64_t)blockIdx.y * ldy + i] = (T)x[(int64_t)blockIdx.y * ldx + (perm ? (int64_t)perm[i] : i)];
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_rows_out(int64_t n, double *__restrict__ x, int64_t ldx,
+                                                     const int *__restrict__ perm, const T *__restrict__ y,
+                                                     int64_t ldy)
+{
+    const int64_t i = run_row<1>();
+    if (i < n) x[(int64_t)blockIdx.y * ldx + (perm ? (int64_t)perm[i] : i)] = (double)y[(int64_t)blockIdx.y * ldy + i];
 }
 
 __global__ __launch_bounds__(kBlock) void k_rowidx(int n, const int *__restrict__ rowptr,
@@ -2170,13 +2201,33 @@ bool sampled_outer(int prec, HIP_MAT *A, const void *X, int64_t ldx, int k, cons
     return true;
 }
 
-void launch_csr_gather_sum(int nparam, const int *jrowptr, const int *jnz, const double *jval, const double *g,
-                           double *grad, double scale, bool accumulate)
+void launch_csr_gather_sum(int nparam, const int *jrowptr, const int *jnz, const double *jval, const int *map,
+                           int nnz, const double *g, double *grad, double scale, bool accumulate, double *bad)
 {
     if (nparam <= 0 || failed()) return;
-    k_csr_gather_sum<<<(nparam + kBlock - 1) / kBlock, kBlock, 0, ctx().stream>>>(nparam, jrowptr, jnz, jval, g,
-                                                                                   grad, scale, accumulate ? 1 : 0);
+    k_csr_gather_sum<<<(nparam + kBlock - 1) / kBlock, kBlock, 0, ctx().stream>>>(
+        nparam, jrowptr, jnz, jval, map, nnz, g, grad, scale, accumulate ? 1 : 0, bad);
     check(hipGetLastError(), "k_csr_gather_sum");
+}
+
+void launch_rows_in(int prec, int64_t n, const double *x, int64_t ldx, const int *perm, void *y, int64_t ldy, int k)
+{
+    if (k <= 0 || n <= 0 || failed()) return;
+    if (prec == GCGE_HIP_FP64)
+        k_rows_in<double><<<run_grid(n, 1, k), kBlock, 0, ctx().stream>>>(n, x, ldx, perm, (double *)y, ldy);
+    else
+        k_rows_in<float><<<run_grid(n, 1, k), kBlock, 0, ctx().stream>>>(n, x, ldx, perm, (float *)y, ldy);
+    check(hipGetLastError(), "k_rows_in");
+}
+
+void launch_rows_out(int prec, int64_t n, double *x, int64_t ldx, const int *perm, const void *y, int64_t ldy, int k)
+{
+    if (k <= 0 || n <= 0 || failed()) return;
+    if (prec == GCGE_HIP_FP64)
+        k_rows_out<double><<<run_grid(n, 1, k), kBlock, 0, ctx().stream>>>(n, x, ldx, perm, (const double *)y, ldy);
+    else
+        k_rows_out<float><<<run_grid(n, 1, k), kBlock, 0, ctx().stream>>>(n, x, ldx, perm, (const float *)y, ldy);
+    check(hipGetLastError(), "k_rows_out");
 }
 
 // matrix helpers used by hip_backend.cpp

@@ -42,6 +42,7 @@ namespace {
 
 constexpr int kThreads = 256;       // 4 wavefronts per workgroup
 constexpr int kGramTargetWG = 2048; // workgroups a Gram launch aims for
+constexpr double kRowsBytes = 200e6;  // X and Y of k_lincomb_rows at most
 constexpr int kSlabThreads = 512;   // slab Gram: 8 wavefronts per workgroup
 constexpr int kSlabTiles = 28;      // most 16-column tiles of V and W together in its block (7 units per thread)
 constexpr int kSlabMaxNT = 17;      // most output tiles per wavefront
@@ -743,15 +744,19 @@ __global__ __launch_bounds__(kThreads, RN <= 2 ? 4 : RN <= 4 ? 3 : 2) void k_lin
     }
 }
 
-// The same products for few columns: a wavefront owns rows [rb, rb + 32) as
-// two 16-row blocks, walks the output in groups of RN 16-column blocks and
-// reads C from the caches; no LDS and no barriers, so more wavefronts are in
-// flight, which is what a memory-bound product needs.  FP32 over 4.1M rows,
-// this kernel against k_lincomb_mfma: 50 x 50 0.517 against 0.565 ms, 20 x 20
-// 0.228 against 0.250, but 150 x 50 1.087 against 0.999; FP64 20 x 20 0.419
-// against 0.433, but 50 x 50 1.080 against 0.840.  Over 16,384 rows, FP32:
-// 100 x 100 14.4 against 17.5 us, 200 x 100 23.5 against 25.5, but 300 x 100
-// 30.1 against 29.1.  slot t of lane l holds row drow(l / 16, t) of its block
+// The same products for few columns of few rows: a wavefront owns rows [rb, rb +
+// 32) as two 16-row blocks, walks the output in groups of RN 16-column blocks
+// and reads C from the caches; no LDS and no barriers, so more wavefronts are in
+// flight, which is what a memory-bound product needs while X and Y fit the
+// 256 MB cache (kRowsBytes, below it because other data is there too).  This
+// kernel against k_lincomb_mfma, us: FP32 20 x 20, 512,000 rows (82 MB) 21.5
+// against 25.0, 884,736 (142 MB) 32.1 against 37.7, 4.1M (655 MB) 159 against
+// 147; 40 x 40, 262,144 rows (84 MB) 26.7 against 26.9, 884,736 (283 MB) 91
+// against 72, 4.1M 374 against 285; FP64 20 x 20, 512,000 rows (164 MB) 37.4
+// against 40.7, 884,736 (283 MB) 71.0 against 69.8.  Where q or p are larger it
+// is the slower one at any size: FP32 150 x 50 over 4.1M rows 1.087 against 0.999
+// ms, 300 x 100 over 16,384 30.1 against 29.1 us (but 200 x 100 23.5 against
+// 25.5); FP64 50 x 50 over 4.1M rows 1.080 against 0.840.  slot t of lane l holds row drow(l / 16, t) of its block
 // and column l % 16.
 // Result rows of one lane after regrouping: lane (g = l / 16, m) returns
 // rows 4 g .. 4 g + 3 of column m of the 16 x 16 block.  For FP32 these are
@@ -1286,10 +1291,12 @@ bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, in
         latch(171, "lincomb: operands are not aligned or padded");
         return false;
     }
+    const size_t es = elem_size(prec);
     // column blocks per pass (RN, at most 8) so that the passes are equal;
     // k_lincomb_rows: 1, 2 or 4, beyond 4 by two wavefronts (WC)
     const int nkb = (p + 3) / 4, nqb0 = (q + 15) / 16;
-    const bool rows = prec == GCGE_HIP_FP64 ? q <= 32 && p < 64 : q <= 64 ? p < 128 : n < 65536 && p < 256;
+    const bool rows = (double)n * (p + q) * es <= kRowsBytes &&
+                      (prec == GCGE_HIP_FP64 ? q <= 32 && p < 64 : q <= 64 ? p < 128 : n < 65536 && p < 256);
     const int wc = rows && nqb0 > 4 ? 2 : 1;
     const int groups = (nqb0 + 7) / 8;
     const int rn = rows ? (nqb0 <= 2 ? nqb0 : 4) : (nqb0 + groups - 1) / groups;

@@ -127,7 +127,8 @@ void *try_row_stage(size_t bytes)
         (void)hipGetLastError();
         return nullptr;
     }
-    return room > bytes + ((size_t)64 << 20) ? row_stage(bytes) : nullptr;
+    // room for a row order's device copy beside it
+    return room > 2 * bytes + ((size_t)64 << 20) ? row_stage(bytes) : nullptr;
 }
 
 double *host_buf(size_t count)
@@ -1173,7 +1174,7 @@ static const int *mv_perm_d(const MV *m) { return mv_perm(m) ? mat_perm(m->mat) 
 template <typename F>
 static bool staged_columns_through(MV *m, int start, int ncols, F f)
 {
-    const size_t column = sizeof(double) * (size_t)m->n;
+    const size_t column = sizeof(double) * (size_t)std::max<int64_t>(m->n, 1);
     const int some = (int)std::min<size_t>(std::max(ncols, 1), std::max<size_t>(1, ((size_t)64 << 20) / column));
     double *stage = (double *)try_row_stage(column * some);
     if (!stage || (mv_perm(m) && !mv_perm_d(m))) return false;

@@ -251,6 +251,9 @@ void launch_csr_gather_sum(int nparam, const int *jrowptr, const int *jnz, const
 // y_j[i] = x_j[perm[i]] (perm null: x_j[i]), x in FP64 with distance ldx, and
 // the reverse x_j[perm[i]] = y_j[i]; j < k
 void launch_rows_in(int prec, int64_t n, const double *x, int64_t ldx, const int *perm, void *y, int64_t ldy, int k);
+// bytes (rounded up to 16) from coherent host memory to device memory, both
+// 16-byte aligned
+void launch_fetch(const void *host, void *dev, size_t bytes);
 void launch_rows_out(int prec, int64_t n, double *x, int64_t ldx, const int *perm, const void *y, int64_t ldy, int k);
 
 }  // namespace gh

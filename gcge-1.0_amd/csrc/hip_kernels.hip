@@ -1438,6 +1438,13 @@ __global__ __launch_bounds__(kBlock) void k_rows_in(int64_t n, const double *__r
     if (i < n) y[(int64_t)blockIdx.y * ldy + i] = (T)x[(int64_t)blockIdx.y * ldx + (perm ? (int64_t)perm[i] : i)];
 }
 
+// 16-byte units over the host link: as many reads in flight as there are
+__global__ __launch_bounds__(kBlock) void k_fetch(const int4 *__restrict__ host, int4 *__restrict__ dev, size_t units)
+{
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < units) dev[i] = host[i];
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_rows_out(int64_t n, double *__restrict__ x, int64_t ldx,
                                                      const int *__restrict__ perm, const T *__restrict__ y,
@@ -2219,6 +2226,15 @@ void launch_rows_in(int prec, int64_t n, const double *x, int64_t ldx, const int
     else
         k_rows_in<float><<<run_grid(n, 1, k), kBlock, 0, ctx().stream>>>(n, x, ldx, perm, (float *)y, ldy);
     check(hipGetLastError(), "k_rows_in");
+}
+
+void launch_fetch(const void *host, void *dev, size_t bytes)
+{
+    if (bytes == 0 || failed()) return;
+    const size_t units = (bytes + 15) / 16;
+    k_fetch<<<(unsigned)((units + kBlock - 1) / kBlock), kBlock, 0, ctx().stream>>>((const int4 *)host, (int4 *)dev,
+                                                                                    units);
+    check(hipGetLastError(), "k_fetch");
 }
 
 void launch_rows_out(int prec, int64_t n, double *x, int64_t ldx, const int *perm, const void *y, int64_t ldy, int k)

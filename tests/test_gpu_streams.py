@@ -101,3 +101,20 @@ def test_few_partial_sums(ops):
     assert np.all(np.isnan(got) == [False] * 3 + [True] * 2 + [False] * 3)
     got[3:5] = nine[3:5]
     assert np.array_equal(got, nine[:8])
+
+
+@pytest.mark.parametrize("p,q", [(16, 126), (64, 32), (65, 33), (9, 9), (331, 129)])
+def test_staged_coefficients(ops, p, q):
+    """Coefficients on both sides of the size from which a kernel fetches them,
+    several launches in flight over one staging ring: Y = X C with X a part of
+    the identity shows C itself."""
+    n = 37 * 37
+    A, g = Matrix(P.lap2d(37)[0]), np.random.default_rng(p)
+    x = MultiVec(A, p, F64)
+    x.set(np.asfortranarray(np.eye(n, p)))
+    cs = [g.standard_normal((p, q)) for _ in range(4)]
+    ys = [MultiVec(A, q, F64) for _ in cs]
+    for c, y in zip(cs, ys):
+        ops.lincomb(x, y, c)
+    for c, y in zip(cs, ys):
+        assert np.array_equal(y.get()[:p], c)

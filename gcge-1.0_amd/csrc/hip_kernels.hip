@@ -1550,11 +1550,16 @@ void launch_axpby(int prec, int64_t n, const void *x, int64_t ldx, void *y, int6
 // host memory, where the host adds them in k_reduce_rows_host's order: a launch
 // less and its wait.  us a call, FP64 dots of 1 column of 16,384 rows (64
 // partial sums) 14.6 -> 11.1, of 20 columns (1280) 15.9 -> 14.7, of 8 columns of
-// 90,000 rows (2048) 15.8 -> 15.6, where the line is drawn.
-static double *partial_buf(size_t rows, size_t nb)
+// 90,000 rows (2048) 15.8 -> 15.6, where the line is drawn.  Not where the launch
+// also `writes` columns: the host would have the sums while stores of the same
+// launch may still lie in one XCD's L2, out of sight of other streams.  The
+// launch that reduces comes after those stores (residual update of 1 column of
+// 16,384 rows 16.6 us, 12.6 without; of 20 columns 18.1 and 16.0; with a
+// system-scope release by every workgroup instead 29).
+static double *partial_buf(size_t rows, size_t nb, bool writes)
 {
-    return rows * nb <= kHostPartials ? host_partials(rows * nb)
-                                      : (double *)scratch(sizeof(double) * rows * nb);
+    return !writes && rows * nb <= kHostPartials ? host_partials(rows * nb)
+                                                 : (double *)scratch(sizeof(double) * rows * nb);
 }
 
 // sum_row and block_sum on the host
@@ -1608,7 +1613,7 @@ bool dots(int prec, int64_t n, const void *x, int64_t ldx, const void *y, int64_
     if (k <= 0) return true;
     if (failed()) return false;
     const int nb = dots_blocks(n);
-    double *partial = partial_buf((size_t)k, nb);
+    double *partial = partial_buf((size_t)k, nb, false);
     if (!partial) return false;
     {
         ProfScope ps(K_DOTS, 2.0 * k * (double)n * elem_size(prec), 2.0 * k * (double)n);
@@ -1707,7 +1712,7 @@ static bool spmm_rows_g(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColS
     const int pstride = nblk + (DOT ? nlong : 0);
     double *partial = nullptr;
     if (DOT) {
-        partial = partial_buf((size_t)kc, pstride);
+        partial = partial_buf((size_t)kc, pstride, true);
         if (!partial) return false;
     }
     {
@@ -1797,7 +1802,7 @@ static bool spmm_halo(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColSca
     const int pstride = nblk + (DOT ? nlong : 0);
     double *partial = nullptr;
     if (DOT) {
-        partial = partial_buf((size_t)kc, pstride);
+        partial = partial_buf((size_t)kc, pstride, true);
         if (!partial) return false;
     }
     {
@@ -1845,7 +1850,7 @@ static bool spmm_t(HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy,
         const int pstride = nblk + (DOT ? nlong : 0);
         double *partial = nullptr;
         if (DOT) {
-            partial = partial_buf((size_t)kc, pstride);
+            partial = partial_buf((size_t)kc, pstride, true);
             if (!partial) return false;
         }
         {
@@ -1900,7 +1905,7 @@ static bool residual_rows_g(HIP_MAT *A, HIP_MAT *B, const T *X, int64_t ldx, Col
     const int RWG = rows_per_wg(G);
     const int nblk = (n + RWG - 1) / RWG, nlong = A->nlong, nlb = (nlong + 3) / 4;
     const int pstride = nblk + nlong;
-    double *partial = partial_buf((size_t)3 * kc, pstride);
+    double *partial = partial_buf((size_t)3 * kc, pstride, false);
     if (!partial) return false;
     {
         ProfScope ps(K_RESIDUAL,
@@ -2005,7 +2010,7 @@ static bool residual_t(HIP_MAT *A, HIP_MAT *B, const void *X, int64_t ldx, const
             }
             continue;
         }
-        double *partial = partial_buf((size_t)3 * kc, nblk);
+        double *partial = partial_buf((size_t)3 * kc, nblk, false);
         if (!partial) return false;
         const double rbytes = 12.0 * A->nnz + 4.0 * (A->n + 1) + (B ? 12.0 * B->nnz + 4.0 * (B->n + 1) : 0.0) +
                               (double)kc * A->n * sizeof(T);
@@ -2051,7 +2056,7 @@ bool cg_update(int prec, int64_t n, void *x, int64_t ldx, const void *p, int64_t
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars s = make_scalars(kc, alpha + c0, nullptr, nullptr);
-        double *partial = partial_buf((size_t)kc, nb);
+        double *partial = partial_buf((size_t)kc, nb, true);
         if (!partial) return false;
         dim3 grid(nb, kc);
         {
@@ -2081,7 +2086,7 @@ bool cg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t 
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars s = make_scalars(kc, alpha + c0, nullptr, nullptr);
-        double *partial = partial_buf((size_t)kc, nb);
+        double *partial = partial_buf((size_t)kc, nb, true);
         if (!partial) return false;
         dim3 grid(nb, kc);
         {
@@ -2114,7 +2119,7 @@ bool pcg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars s = make_scalars(kc, alpha + c0, nullptr, nullptr);
-        double *partial = partial_buf((size_t)2 * kc, nb);
+        double *partial = partial_buf((size_t)2 * kc, nb, true);
         if (!partial) return false;
         dim3 grid(nb, kc);
         {

@@ -222,6 +222,10 @@ GCGE_INT GCGE_HIP_MultiVecInnerProdDiagNoAlloc(void **x, void **y, GCGE_DOUBLE *
 /* Returns the latched error code (0 = none) and copies its message. */
 GCGE_INT GCGE_HIP_GetLastError(char *msg, GCGE_INT len);
 void GCGE_HIP_ClearError(void);
+/* Waits for all queued work.  A call that returns numbers (dots, Gram
+ * products, residual norms, CG scalars) returns when they are in host memory:
+ * earlier work and the columns it writes itself are complete, for other
+ * streams too.  Other calls only queue their work. */
 GCGE_INT GCGE_HIP_Synchronize(void);
 /* Device memory currently held by the backend, in bytes. */
 double GCGE_HIP_DeviceBytes(void);

@@ -1,0 +1,71 @@
+"""The library's host code -- which kernels a call launches, in which order,
+what it keeps of the memory it takes, what it does where there is none --
+against a HIP runtime of host memory (hostrt/hostrt.cpp), where no GPU is
+needed.  Each test's script runs in a process of its own, because that runtime
+has to be loaded before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, sys
+rt = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+rt.hostrt_launches.restype = C.c_char_p
+rt.hostrt_live.restype = C.c_size_t
+rt.hostrt_limit.argtypes = [C.c_size_t]
+sys.path[:0] = sys.argv[2:]
+import numpy as np
+from gcge_hip import Matrix, MultiVec, Ops, capi, eig_gradient
+from gcge_hip import problems as P
+F64, F32 = capi.GCGE_HIP_FP64, capi.GCGE_HIP_FP32
+ops = Ops()
+
+def launched(f):
+    '''names of the kernels that f() launches'''
+    rt.hostrt_launches()
+    f()
+    out = []
+    for name in rt.hostrt_launches().decode().split():
+        i = name.index("k_")
+        out.append(name[i:i + int(name[:i].split("_1")[-1])])
+    return out
+"""
+
+
+@pytest.fixture(scope="session")
+def hostrt(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hostrt") / "hostrt.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Werror",
+                    os.path.join(HERE, "hostrt", "hostrt.cpp"), "-o", so], check=True)
+
+    def run(script, **env):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + script, so, os.path.join(ROOT, "gcge-1.0_amd")],
+                           capture_output=True, text=True, timeout=300, env={**os.environ, **env})
+        assert p.returncode == 0, p.stdout + p.stderr
+
+    return run
+
+
+def test_columns_are_written_before_the_call_returns(hostrt):
+    """A call that writes columns and returns sums of them reads the sums from
+    a later launch, so the columns are complete, for every stream, when the
+    host has the sums."""
+    hostrt("""
+A, M = P.lap3d_mass(8)
+G = P.chung_lu(20000)[0]
+for M, prec in ((P.lap2d(24)[0], F64), (P.lap2d(24)[0], F32), (M, F64), (G, F32)):
+    A = Matrix(M)
+    for k in (1, 2, 20):
+        x, r, w, p = (MultiVec(A, k, prec) for _ in range(4))
+        a = np.ones(k)
+        for f in (lambda: ops.matdot_dot(A, x, w), lambda: ops.cg_update(x, 0, p, w, r, k, a),
+                  lambda: ops.cg_residual_update(w, r, k, a), lambda: ops.pcg_residual_update(A, w, r, k, a)):
+            names = launched(f)
+            assert len(names) >= 2 and names[-1] == "k_reduce_rows_host", names
+        assert launched(lambda: ops.dots(x, w))[0] == "k_dots"
+""")

@@ -127,7 +127,6 @@ void *try_row_stage(size_t bytes)
         (void)hipGetLastError();
         return nullptr;
     }
-    // room for a row order's device copy beside it
     return room > 2 * bytes + ((size_t)64 << 20) ? row_stage(bytes) : nullptr;
 }
 
@@ -409,11 +408,15 @@ const int *mat_rowidx(HIP_MAT *A)
     return failed() ? nullptr : A->rowidx;
 }
 
+// Null without an error where there is no memory: callers have a host path.
 static const int *device_ints(int **dev, const int *host, int n)
 {
     if (*dev || !host) return *dev;
     int *d = nullptr;
-    if (!check(hipMalloc((void **)&d, sizeof(int) * std::max(1, n)), "hipMalloc row order")) return nullptr;
+    if (hipMalloc((void **)&d, sizeof(int) * std::max(1, n)) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     if (!check(hipMemcpy(d, host, sizeof(int) * (size_t)n, hipMemcpyHostToDevice), "H2D row order")) {
         (void)hipFree(d);
         return nullptr;
@@ -1972,7 +1975,7 @@ bool jacobian_ok(const HIP_MAT *M, GCGE_INT nparam, const GCGE_INT *jrowptr, con
 }
 
 // every jnz a stored-entry index of the matrix (asked where the device found
-// that one is not)
+// that one is not, or does not look)
 void latch_bad_entry(const HIP_MAT *M, GCGE_INT nparam, const GCGE_INT *jrowptr, const GCGE_INT *jnz, const char *which)
 {
     for (int t = 0; t < jrowptr[nparam]; t++)
@@ -2000,9 +2003,19 @@ bool gradient_term(HIP_MAT *M, MV *mx, GCGE_INT k, const double *wgt, GCGE_INT n
     const int nj = jrowptr[nparam];
     double *g = (double *)mem, *dval = g + std::max(1, M->nnz);
     int *dnz = (int *)(dval + nj), *drp = dnz + nj;
+    // what cannot be done without takes device memory first
+    if (!mat_rowidx(M)) return false;
     const int *map = mat_nzmap(M);  // the caller's entry indices -> the stored order
+    std::vector<int> mapped;
+    if (M->nzmap_h && !map && !failed()) {  // no device memory for it: here
+        latch_bad_entry(M, nparam, jrowptr, jnz, which);
+        if (failed()) return false;
+        mapped.resize((size_t)nj);
+        for (int t = 0; t < nj; t++) mapped[t] = M->nzmap_h[jnz[t]];
+        jnz = mapped.data();
+    }
     double *bad = host_buf(1);
-    if ((M->nzmap_h && !map) || !bad) return false;
+    if (!bad || failed()) return false;
     *bad = 0.0;
     const bool ok = check(hipMemcpy(drp, jrowptr, sizeof(int) * (nparam + 1), hipMemcpyHostToDevice), "H2D") &&
                     (nj == 0 || check(hipMemcpy(dnz, jnz, sizeof(int) * nj, hipMemcpyHostToDevice), "H2D")) &&

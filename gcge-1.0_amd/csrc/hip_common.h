@@ -189,7 +189,8 @@ size_t elem_size(int prec);
 void *col_ptr(MV *m, int64_t c);
 const float *mat_val32(HIP_MAT *A);
 const int *mat_rowidx(HIP_MAT *A);
-// device copies of the row order and of the entry order (built on first use)
+// device copies of the row order and of the entry order (built on first use;
+// null without an error where there is no memory for them)
 const int *mat_perm(HIP_MAT *A);
 const int *mat_nzmap(HIP_MAT *A);
 // 1 / diagonal of A in the given precision (built on first use)

@@ -20,10 +20,11 @@ rt.hostrt_live.restype = C.c_size_t
 rt.hostrt_limit.argtypes = [C.c_size_t]
 sys.path[:0] = sys.argv[2:]
 import numpy as np
-from gcge_hip import Matrix, MultiVec, Ops, capi, eig_gradient
+from gcge_hip import Matrix, MultiVec, Ops, capi
 from gcge_hip import problems as P
 F64, F32 = capi.GCGE_HIP_FP64, capi.GCGE_HIP_FP32
 ops = Ops()
+Hook = C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_void_p))
 
 def launched(f):
     '''names of the kernels that f() launches'''
@@ -68,4 +69,60 @@ for M, prec in ((P.lap2d(24)[0], F64), (P.lap2d(24)[0], F32), (M, F64), (G, F32)
             names = launched(f)
             assert len(names) >= 2 and names[-1] == "k_reduce_rows_host", names
         assert launched(lambda: ops.dots(x, w))[0] == "k_dots"
+""")
+
+
+def test_host_columns_without_memory_for_the_row_order(hostrt):
+    """Columns of an ordered matrix move and gradients map their entries on the
+    host where the device has no room for the order, without an error."""
+    hostrt("""
+M = P.lap2d(300)[0]
+n, k, g = M.shape[0], 4, np.random.default_rng(0)
+X = np.asfortranarray(g.standard_normal((n, k)))
+order = g.permutation(n).astype(np.int32)
+plain, ordered = Matrix(M), Matrix(M, order=order)
+stage = MultiVec(plain, k, F32)
+stage.set(X)  # the staging buffer is there
+jrp = np.arange(n + 1, dtype=np.int32)
+jnz = g.integers(0, M.nnz, n).astype(np.int32)
+jval, w, grad = g.standard_normal(n), np.ones(k), np.zeros(n)
+px = MultiVec(plain, k, F64)
+
+def gradient(A, mv):
+    capi.load().GCGE_HIP_EigGradient(A.ptr, mv.ptr, k, w.ctypes.data_as(capi.DP), n, jrp.ctypes.data_as(capi.IP),
+                                     jnz.ctypes.data_as(capi.IP), jval.ctypes.data_as(capi.DP),
+                                     grad.ctypes.data_as(capi.DP))
+    capi.raise_on_error("gradient")
+
+entries = []
+
+def note(name, args):
+    if b"k_csr_gather_sum" in name:
+        at = lambda i: C.c_void_p.from_address(args[i]).value
+        e = np.ctypeslib.as_array((C.c_int * n).from_address(at(2))).copy()
+        if at(4):
+            e = np.ctypeslib.as_array((C.c_int * M.nnz).from_address(at(4)))[e]
+        entries.append(e)
+
+hook = Hook(note)
+rt.hostrt_hook(hook)
+gradient(plain, px)
+room = MultiVec(ordered, k, F64)
+gradient(ordered, room)
+room.close()
+fresh = Matrix(M, order=order)  # no order on the device yet
+d, f = MultiVec(fresh, k, F64), MultiVec(fresh, k, F32)
+rt.hostrt_limit(rt.hostrt_live())
+for mv in (d, f):
+    mv.set(X)
+    assert np.array_equal(mv.get(), X if mv is d else X.astype(np.float32).astype(np.float64))
+rt.hostrt_limit(rt.hostrt_live() + 4 * M.nnz)  # the rows of the entries, and no more
+gradient(fresh, d)
+assert np.array_equal(entries[0], jnz) and np.array_equal(entries[2], entries[1])
+jnz[7] = M.nnz
+try:
+    gradient(fresh, d)
+    raise SystemExit("a bad entry was taken")
+except RuntimeError as e:
+    assert "jnz[7]" in str(e), e
 """)

@@ -80,6 +80,80 @@ bool ensure_ctx()
     return true;
 }
 
+// Live matrices, for the device copies of their orders
+static std::vector<HIP_MAT *> g_mats;
+
+// Gives back what is kept for speed alone: the buffer of TmpDev and the
+// matrices' orders.  Calls fetch an order after their last allocation.
+static void release_kept()
+{
+    (void)hipStreamSynchronize(g_ctx.stream);
+    if (g_ctx.tmp && !g_ctx.tmp_used) {
+        (void)hipFree(g_ctx.tmp);
+        g_ctx.dev_bytes -= (double)g_ctx.tmp_bytes;
+        g_ctx.tmp = nullptr;
+        g_ctx.tmp_bytes = 0;
+    }
+    for (HIP_MAT *A : g_mats) {
+        if (A->perm_d) g_ctx.dev_bytes -= 4.0 * A->n;
+        if (A->nzmap_d) g_ctx.dev_bytes -= 4.0 * A->nnz;
+        for (int **p : {&A->perm_d, &A->nzmap_d}) {
+            if (*p) (void)hipFree(*p);
+            *p = nullptr;
+        }
+    }
+}
+
+// hipMalloc, once more without what is kept where memory is short
+static hipError_t dev_malloc(void *p, size_t bytes)
+{
+    hipError_t e = hipMalloc((void **)p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    release_kept();
+    return hipMalloc((void **)p, bytes);
+}
+
+// Device memory for the duration of a call, p null without an error where there
+// is none.  Up to kTmpKept it stays with the context for the next such call.
+constexpr size_t kTmpKept = (size_t)128 << 20;
+
+struct TmpDev {
+    void *p = nullptr;
+    explicit TmpDev(size_t bytes)
+    {
+        const bool keep = bytes <= kTmpKept && !g_ctx.tmp_used;
+        if (keep && bytes <= g_ctx.tmp_bytes) p = g_ctx.tmp;
+        else if (sync()) {
+            if (keep && g_ctx.tmp) {
+                (void)hipFree(g_ctx.tmp);
+                g_ctx.dev_bytes -= (double)g_ctx.tmp_bytes;
+                g_ctx.tmp = nullptr;
+                g_ctx.tmp_bytes = 0;
+            }
+            if (dev_malloc(&p, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                p = nullptr;
+            } else if (keep) {
+                g_ctx.tmp = p;
+                g_ctx.tmp_bytes = bytes;
+                g_ctx.dev_bytes += (double)bytes;
+            }
+        }
+        if (p && p == g_ctx.tmp) g_ctx.tmp_used = true;
+    }
+    ~TmpDev()
+    {
+        if (!p) return;
+        if (p == g_ctx.tmp) g_ctx.tmp_used = false;
+        else {
+            sync();
+            (void)hipFree(p);
+        }
+    }
+    TmpDev(const TmpDev &) = delete;
+};
+
 void *scratch(size_t bytes)
 {
     if (!ensure_ctx()) return nullptr;
@@ -94,7 +168,7 @@ void *scratch(size_t bytes)
     }
     size_t want = std::max(bytes, (size_t)(8u << 20));
     want = (want + 4095) & ~(size_t)4095;
-    if (!check(hipMalloc(&g_ctx.scratch, want), "hipMalloc scratch")) return nullptr;
+    if (!check(dev_malloc(&g_ctx.scratch, want), "hipMalloc scratch")) return nullptr;
     g_ctx.scratch_bytes = want;
     g_ctx.dev_bytes += (double)want;
     return g_ctx.scratch;
@@ -112,22 +186,10 @@ void *row_stage(size_t bytes)
         g_ctx.rows_bytes = 0;
     }
     const size_t want = (bytes + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
-    if (!check(hipMalloc(&g_ctx.rows, want), "hipMalloc row staging")) return nullptr;
+    if (!check(dev_malloc(&g_ctx.rows, want), "hipMalloc row staging")) return nullptr;
     g_ctx.rows_bytes = want;
     g_ctx.dev_bytes += (double)want;
     return g_ctx.rows;
-}
-
-void *try_row_stage(size_t bytes)
-{
-    if (!ensure_ctx()) return nullptr;
-    if (bytes <= g_ctx.rows_bytes) return g_ctx.rows;
-    size_t room = 0, total = 0;
-    if (hipMemGetInfo(&room, &total) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return room > 2 * bytes + ((size_t)64 << 20) ? row_stage(bytes) : nullptr;
 }
 
 double *host_buf(size_t count)
@@ -349,7 +411,7 @@ void *stage_to_device(const void *host, size_t bytes)
         g_ctx.stage_d = nullptr;
         const size_t cap = std::max(need, (size_t)(8u << 20));
         if (!check(hipHostMalloc((void **)&g_ctx.stage_h, cap, hipHostMallocCoherent), "hipHostMalloc stage") ||
-            !check(hipMalloc((void **)&g_ctx.stage_d, cap), "hipMalloc stage")) {
+            !check(dev_malloc((void **)&g_ctx.stage_d, cap), "hipMalloc stage")) {
             g_ctx.stage_cap = 0;
             return nullptr;
         }
@@ -378,7 +440,7 @@ void *col_ptr(MV *m, int64_t c) { return (char *)m->data + (size_t)c * (size_t)m
 const float *mat_val32(HIP_MAT *A)
 {
     if (A->val32) return A->val32;
-    if (!check(hipMalloc((void **)&A->val32, sizeof(float) * std::max(1, A->nnz)), "hipMalloc val32"))
+    if (!check(dev_malloc((void **)&A->val32, sizeof(float) * std::max(1, A->nnz)), "hipMalloc val32"))
         return nullptr;
     g_ctx.dev_bytes += sizeof(float) * (double)A->nnz;
     launch_to_f32(A->nnz, A->val64, A->val32);
@@ -389,8 +451,8 @@ const void *mat_dinv(HIP_MAT *A, int prec)
 {
     if (!A->dinv64) {
         const size_t n = (size_t)std::max(1, A->n);
-        if (!check(hipMalloc((void **)&A->dinv64, sizeof(double) * n), "hipMalloc dinv64")) return nullptr;
-        if (!check(hipMalloc((void **)&A->dinv32, sizeof(float) * n), "hipMalloc dinv32")) return nullptr;
+        if (!check(dev_malloc((void **)&A->dinv64, sizeof(double) * n), "hipMalloc dinv64")) return nullptr;
+        if (!check(dev_malloc((void **)&A->dinv32, sizeof(float) * n), "hipMalloc dinv32")) return nullptr;
         g_ctx.dev_bytes += 12.0 * (double)n;
         launch_diag_inv(A);
         if (failed()) return nullptr;
@@ -401,7 +463,7 @@ const void *mat_dinv(HIP_MAT *A, int prec)
 const int *mat_rowidx(HIP_MAT *A)
 {
     if (A->rowidx) return A->rowidx;
-    if (!check(hipMalloc((void **)&A->rowidx, sizeof(int) * std::max(1, A->nnz)), "hipMalloc rowidx"))
+    if (!check(dev_malloc((void **)&A->rowidx, sizeof(int) * std::max(1, A->nnz)), "hipMalloc rowidx"))
         return nullptr;
     g_ctx.dev_bytes += sizeof(int) * (double)A->nnz;
     launch_rowidx(A);
@@ -452,7 +514,7 @@ static MV *mv_new(int64_t n, int ncols, int prec, HIP_MAT *mat)
     m->mat = mat;
     m->data = nullptr;
     size_t bytes = (size_t)m->ld * (size_t)std::max(ncols, 1) * elem_size(prec);
-    if (!check(hipMalloc(&m->data, bytes), "hipMalloc multivector")) {
+    if (!check(dev_malloc(&m->data, bytes), "hipMalloc multivector")) {
         delete m;
         return nullptr;
     }
@@ -580,16 +642,16 @@ extern "C" HIP_MAT *HIP_MatCreateFromCSR(GCGE_INT nrows, GCGE_INT ncols, GCGE_IN
         if (rowptr[i + 1] - rowptr[i] > kLongRow) longs.push_back(i);
     A->nlong = (int)longs.size();
     A->gather_rows = pick_gather_rows(nrows, rowptr, col);
-    bool ok = check(hipMalloc((void **)&A->rowptr, sizeof(int) * (nrows + 1)), "hipMalloc rowptr") &&
-              check(hipMalloc((void **)&A->col, sizeof(int) * std::max(1, nnz)), "hipMalloc col") &&
-              check(hipMalloc((void **)&A->val64, sizeof(double) * std::max(1, nnz)), "hipMalloc val");
+    bool ok = check(dev_malloc((void **)&A->rowptr, sizeof(int) * (nrows + 1)), "hipMalloc rowptr") &&
+              check(dev_malloc((void **)&A->col, sizeof(int) * std::max(1, nnz)), "hipMalloc col") &&
+              check(dev_malloc((void **)&A->val64, sizeof(double) * std::max(1, nnz)), "hipMalloc val");
     if (ok) {
         ok = check(hipMemcpy(A->rowptr, rowptr, sizeof(int) * (nrows + 1), hipMemcpyHostToDevice), "H2D rowptr") &&
              (nnz == 0 || check(hipMemcpy(A->col, col, sizeof(int) * nnz, hipMemcpyHostToDevice), "H2D col")) &&
              (nnz == 0 || check(hipMemcpy(A->val64, val, sizeof(double) * nnz, hipMemcpyHostToDevice), "H2D val"));
     }
     if (ok && A->nlong > 0)
-        ok = check(hipMalloc((void **)&A->long_rows, sizeof(int) * A->nlong), "hipMalloc long_rows") &&
+        ok = check(dev_malloc((void **)&A->long_rows, sizeof(int) * A->nlong), "hipMalloc long_rows") &&
              check(hipMemcpy(A->long_rows, longs.data(), sizeof(int) * A->nlong, hipMemcpyHostToDevice),
                    "H2D long_rows");
     if (ok && A->gather_rows != 1) ok = build_halo(A, rowptr, col);
@@ -599,6 +661,7 @@ extern "C" HIP_MAT *HIP_MatCreateFromCSR(GCGE_INT nrows, GCGE_INT ncols, GCGE_IN
         return nullptr;
     }
     g_ctx.dev_bytes += sizeof(int) * (double)(nrows + 1) + 12.0 * nnz;
+    g_mats.push_back(A);
     return A;
 }
 
@@ -772,9 +835,9 @@ static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col)
     hcol.reserve((size_t)total);
     for (const std::vector<int> &l : lists) hcol.insert(hcol.end(), l.begin(), l.end());
     const size_t nh = std::max<size_t>(1, hcol.size());
-    bool ok = check(hipMalloc((void **)&A->halo_ptr, sizeof(int) * hptr.size()), "hipMalloc halo_ptr") &&
-              check(hipMalloc((void **)&A->halo_col, sizeof(int) * nh), "hipMalloc halo_col") &&
-              check(hipMalloc((void **)&A->lcol, sizeof(unsigned short) * lcol.size()), "hipMalloc lcol");
+    bool ok = check(dev_malloc((void **)&A->halo_ptr, sizeof(int) * hptr.size()), "hipMalloc halo_ptr") &&
+              check(dev_malloc((void **)&A->halo_col, sizeof(int) * nh), "hipMalloc halo_col") &&
+              check(dev_malloc((void **)&A->lcol, sizeof(unsigned short) * lcol.size()), "hipMalloc lcol");
     if (!ok) return false;
     ok = check(hipMemcpy(A->halo_ptr, hptr.data(), sizeof(int) * hptr.size(), hipMemcpyHostToDevice), "H2D halo") &&
          (hcol.empty() ||
@@ -783,7 +846,7 @@ static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col)
                "H2D lcol");
     if (!ok) return false;
     if (br.order) {
-        ok = check(hipMalloc((void **)&A->brick_rows, sizeof(int) * order.size()), "hipMalloc brick_rows") &&
+        ok = check(dev_malloc((void **)&A->brick_rows, sizeof(int) * order.size()), "hipMalloc brick_rows") &&
              check(hipMemcpy(A->brick_rows, br.order, sizeof(int) * order.size(), hipMemcpyHostToDevice), "H2D bricks");
         if (!ok) return false;
     }
@@ -1066,6 +1129,8 @@ extern "C" void HIP_MatDestroy(HIP_MAT **mat)
     HIP_MAT *A = *mat;
     if (A->magic == kMagicMat) {
         sync();
+        g_mats.erase(std::remove(g_mats.begin(), g_mats.end(), A), g_mats.end());
+        if (g_mats.empty()) release_kept();
         if (A->rowptr) (void)hipFree(A->rowptr);
         if (A->col) (void)hipFree(A->col);
         if (A->val64) (void)hipFree(A->val64);
@@ -1184,9 +1249,9 @@ static bool staged_columns_through(MV *m, int start, int ncols, F f)
 {
     const size_t column = sizeof(double) * (size_t)std::max<int64_t>(m->n, 1);
     const int some = (int)std::min<size_t>(std::max(ncols, 1), std::max<size_t>(1, ((size_t)64 << 20) / column));
-    double *stage = (double *)try_row_stage(column * some);
-    if (!stage || (mv_perm(m) && !mv_perm_d(m))) return false;
-    for (int c = 0; c < ncols && !failed(); c += some) f(stage, c, std::min(some, ncols - c));
+    const TmpDev stage(column * some);
+    if (!stage.p || (mv_perm(m) && !mv_perm_d(m))) return false;
+    for (int c = 0; c < ncols && !failed(); c += some) f((double *)stage.p, c, std::min(some, ncols - c));
     return true;
 }
 
@@ -1987,7 +2052,7 @@ void latch_bad_entry(const HIP_MAT *M, GCGE_INT nparam, const GCGE_INT *jrowptr,
 
 // grad (device, nparam) = scale * J^T g_M + (accumulate ? grad : 0), where g_M[e] =
 // sum_i wgt_i x_i[row_e] x_i[col_e] over the stored entries of M.  mem: device
-// memory of gradient_bytes, kept by the context; 16 pairs of a 512^2 grid with
+// memory of gradient_bytes; 16 pairs of a 512^2 grid with
 // 3.4M entries in J take 3.2 ms, 75 MB of host data at 31 GB/s most of it (with
 // allocations, index checks and orders on the host 4.6, ordered matrix 7.8)
 size_t gradient_bytes(const HIP_MAT *M, GCGE_INT nparam, const GCGE_INT *jrowptr)
@@ -2003,8 +2068,7 @@ bool gradient_term(HIP_MAT *M, MV *mx, GCGE_INT k, const double *wgt, GCGE_INT n
     const int nj = jrowptr[nparam];
     double *g = (double *)mem, *dval = g + std::max(1, M->nnz);
     int *dnz = (int *)(dval + nj), *drp = dnz + nj;
-    // what cannot be done without takes device memory first
-    if (!mat_rowidx(M)) return false;
+    if (!sampled_outer(mx->prec, M, mx->data, mx->ld, k, wgt, g)) return false;
     const int *map = mat_nzmap(M);  // the caller's entry indices -> the stored order
     std::vector<int> mapped;
     if (M->nzmap_h && !map && !failed()) {  // no device memory for it: here
@@ -2019,8 +2083,7 @@ bool gradient_term(HIP_MAT *M, MV *mx, GCGE_INT k, const double *wgt, GCGE_INT n
     *bad = 0.0;
     const bool ok = check(hipMemcpy(drp, jrowptr, sizeof(int) * (nparam + 1), hipMemcpyHostToDevice), "H2D") &&
                     (nj == 0 || check(hipMemcpy(dnz, jnz, sizeof(int) * nj, hipMemcpyHostToDevice), "H2D")) &&
-                    (nj == 0 || check(hipMemcpy(dval, jval, sizeof(double) * nj, hipMemcpyHostToDevice), "H2D")) &&
-                    sampled_outer(mx->prec, M, mx->data, mx->ld, k, wgt, g);
+                    (nj == 0 || check(hipMemcpy(dval, jval, sizeof(double) * nj, hipMemcpyHostToDevice), "H2D"));
     if (ok) launch_csr_gather_sum(nparam, drp, dnz, dval, map, M->nnz, g, dgrad, scale, accumulate, bad);
     if (!sync() || !ok || failed()) return false;
     if (*(volatile double *)bad != 0.0) latch_bad_entry(M, nparam, jrowptr, jnz, which);
@@ -2048,8 +2111,13 @@ extern "C" GCGE_INT GCGE_HIP_EigGradientGeneralized(HIP_MAT *A, HIP_MAT *B, void
     if (!sync()) return g_err;
     size_t bytes = gradient_bytes(A, nparam, ja_rowptr);
     if (bterm) bytes = std::max(bytes, gradient_bytes(B, nparam, jb_rowptr));
-    double *dgrad = (double *)scratch(sizeof(double) * std::max(1, nparam) + bytes);
-    if (!dgrad) return g_err;
+    bytes += sizeof(double) * std::max(1, nparam);
+    const TmpDev tmp(bytes);
+    double *dgrad = (double *)tmp.p;
+    if (!dgrad) {
+        if (!failed()) latch((int)hipErrorOutOfMemory, "GCGE_HIP_EigGradient: no device memory for %zu bytes", bytes);
+        return g_err;
+    }
     void *mem = dgrad + std::max(1, nparam);
     // x_i^T (dA/dtheta) x_i weighted by w_i, then - lambda_i x_i^T (dB/dtheta) x_i
     bool ok = gradient_term(A, mx, k, w, nparam, ja_rowptr, ja_nz, ja_val, 1.0, false, dgrad, mem, "A");

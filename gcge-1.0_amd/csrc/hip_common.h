@@ -104,6 +104,11 @@ struct Ctx {
     size_t scratch_bytes = 0;
     void *rows = nullptr;  // row-major X staging of the SpMM gather path
     size_t rows_bytes = 0;
+    // memory of TmpDev between calls, given back where memory is short and with
+    // the last matrix
+    void *tmp = nullptr;
+    size_t tmp_bytes = 0;
+    bool tmp_used = false;
     // pinned host buffer for results that kernels write and the host reads
     double *hbuf = nullptr;
     size_t hbuf_bytes = 0;
@@ -131,7 +136,6 @@ bool ensure_ctx();
 bool noalloc_setup(int device);
 void *scratch(size_t bytes);           // device scratch of at least bytes
 void *row_stage(size_t bytes);         // device staging of row-major X copies (SpMM), at least bytes
-void *try_row_stage(size_t bytes);     // the same, null without an error where memory is short
 double *host_buf(size_t count);        // pinned host doubles, writable by kernels
 // The first count numbers and the next launch's (one report at a time: the
 // launch, then wait_seq); null (latched) without memory.

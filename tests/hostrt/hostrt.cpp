@@ -46,7 +46,8 @@ int hipMalloc(void **p, size_t n)
 {
     *p = nullptr;
     if (g_live + n > g_limit) return kNoMemory;
-    if (!(*p = calloc(n ? n : 1, 1))) return kNoMemory;
+    if (posix_memalign(p, 4096, n ? n : 1)) return kNoMemory;
+    memset(*p, 0, n);
     g_blocks[*p] = n;
     g_live += n;
     return 0;

@@ -126,3 +126,51 @@ try:
 except RuntimeError as e:
     assert "jnz[7]" in str(e), e
 """)
+
+
+def test_memory_of_gradients_and_host_columns_is_given_back(hostrt):
+    """A large gradient keeps no more than 128 MiB and the entry order; what is
+    kept makes room for an allocation that needs it, and goes with the last
+    matrix."""
+    hostrt("""
+M = P.lap2d(300)[0]
+n, k, g = M.shape[0], 3, np.random.default_rng(0)
+plain, ordered = Matrix(M), Matrix(M, order=g.permutation(n).astype(np.int32))
+x, y = MultiVec(ordered, k, F64), MultiVec(plain, k, F64)
+X = np.asfortranarray(g.standard_normal((n, k)))
+y.set(X)
+ops.gram(y, y)  # scratch and coefficient staging are there
+ops.lincomb(y, MultiVec(plain, 40, F64), np.ones((3, 40)))
+
+def gradient(nj):
+    jrp = np.linspace(0, nj, n + 1).astype(np.int32)
+    jnz, jval = np.zeros(nj, np.int32), np.ones(nj)
+    w, grad = np.ones(k), np.zeros(n)
+    capi.load().GCGE_HIP_EigGradient(ordered.ptr, x.ptr, k, w.ctypes.data_as(capi.DP), n,
+                                     jrp.ctypes.data_as(capi.IP), jnz.ctypes.data_as(capi.IP),
+                                     jval.ctypes.data_as(capi.DP), grad.ctypes.data_as(capi.DP))
+    capi.raise_on_error("gradient")
+
+live = rt.hostrt_live()
+held = capi.load().GCGE_HIP_DeviceBytes()
+gradient(12_000_000)
+fixed = 2 * 4 * M.nnz + 4 * n  # rows and order of the entries, row order
+assert rt.hostrt_live() <= live + fixed, rt.hostrt_live() - live
+gradient(5_000_000)
+x.set(X)
+x.get()
+grown = rt.hostrt_live() - live
+assert 0 < grown <= (128 << 20) + fixed
+assert capi.load().GCGE_HIP_DeviceBytes() - held == grown
+rt.hostrt_limit(rt.hostrt_live())
+rows = 4 * M.nnz  # what no call gives back: the rows of the entries
+cols = (grown - rows) // (8 * (n // 256 + 1 | 1) * 256)
+big = MultiVec(plain, cols, F64)
+big.close()
+rt.hostrt_limit(1 << 40)
+gradient(5_000_000)
+for o in (x, y, ordered, plain):
+    o.close()
+assert rt.hostrt_live() < live, (rt.hostrt_live(), live)
+assert rt.hostrt_live() <= 20 << 20, rt.hostrt_live()
+""")

@@ -1998,9 +1998,11 @@ static bool residual_t(HIP_MAT *A, HIP_MAT *B, const void *X, int64_t ldx, const
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars g = make_scalars(kc, lambda + c0, nullptr, idx + c0);
-        // row gather for scattered or long rows that cannot be staged (B's
-        // rows must all be short)
-        const bool rows = A->gather_rows || long_average(A) || (B && (B->gather_rows || long_average(B)));
+        // row gather for scattered rows, and for long ones staged for SpMM but
+        // not here (B's rows must all be short); a matrix with neither was
+        // created with the direct gather asked for
+        const auto by_rows = [](const HIP_MAT *M) { return M->gather_rows || (M->halo && long_average(M)); };
+        const bool rows = by_rows(A) || (B && by_rows(B));
         if (!cap && rows && (!B || B->nlong == 0) && kc >= 2) {
             if (!residual_rows<T>(A, B, (const T *)X, ldx, g, kc, tmp.data())) return false;
             for (int j = 0; j < kc; j++) {

@@ -174,3 +174,19 @@ for o in (x, y, ordered, plain):
 assert rt.hostrt_live() < live, (rt.hostrt_live(), live)
 assert rt.hostrt_live() <= 20 << 20, rt.hostrt_live()
 """)
+
+
+@pytest.mark.parametrize("layout,kernel", [("columns", "k_residual"), ("rows", "k_residual_rows"),
+                                           ("halo", "k_residual_halo")])
+def test_layout_override_holds_for_the_residual_check(hostrt, layout, kernel):
+    """GCGE_HIP_SPMM_GATHER decides the residual check's kernel too, for rows of
+    more than 8 entries on average in A, B or both."""
+    hostrt(f"""
+A, B = (Matrix(M) for M in P.lap3d_mass(12))
+lam, idx = np.ones(5), np.arange(5, dtype=np.int32)
+for prec in (F64, F32):
+    x = MultiVec(A, 5, prec)
+    for a, b in ((A, B), (B, None), (B, A), (B, B), (A, None)):
+        names = launched(lambda: ops.residual_norms(a, b, x, idx, lam))
+        assert "{kernel}" in names, (names, prec)
+""", GCGE_HIP_SPMM_GATHER=layout)

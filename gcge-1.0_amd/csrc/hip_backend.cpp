@@ -1120,7 +1120,7 @@ extern "C" GCGE_INT HIP_MatGetOrder(const HIP_MAT *mat, GCGE_INT *perm)
 extern "C" GCGE_INT HIP_MatGatherKind(const HIP_MAT *mat)
 {
     if (!mat || mat->magic != kMagicMat) return -1;
-    return mat->gather_rows ? 1 : mat->halo ? 2 : 0;
+    return mat->gather_rows ? 1 : mat->halo && (mat->prec == GCGE_HIP_FP64 || mat->halo_f32) ? 2 : 0;
 }
 
 extern "C" void HIP_MatDestroy(HIP_MAT **mat)

@@ -67,9 +67,11 @@ HIP_MAT *HIP_MatCreateFromCSROrdered(GCGE_INT nrows, GCGE_INT ncols, GCGE_INT nn
 /* Writes the matrix's row order into perm[n] and returns 1, or returns 0
  * (natural order, perm untouched); -1 for a bad matrix. */
 GCGE_INT HIP_MatGetOrder(const HIP_MAT *mat, GCGE_INT *perm);
-/* The SpMM layout chosen at creation: 0 direct column gather (k_spmm),
- * 1 row-major gather (k_spmm_rows), 2 staged row blocks (k_spmm_halo);
- * -1 for a bad matrix.  No counterpart in the reference (a query of this
+/* The SpMM layout chosen at creation, for products in the precision of
+ * HIP_MatSetPrecision (a large 3-D grid in its natural order may be staged in
+ * FP64 only): 0 direct column gather (k_spmm), 1 row-major gather
+ * (k_spmm_rows; single columns k_spmm), 2 staged row blocks (k_spmm_halo); -1
+ * for a bad matrix.  No counterpart in the reference (a query of this
  * backend's layout choice). */
 GCGE_INT HIP_MatGatherKind(const HIP_MAT *mat);
 /* Write CSR arrays (host) in the text format (binary = 0; values with 17

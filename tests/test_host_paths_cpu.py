@@ -190,3 +190,24 @@ for prec in (F64, F32):
         names = launched(lambda: ops.residual_norms(a, b, x, idx, lam))
         assert "{kernel}" in names, (names, prec)
 """, GCGE_HIP_SPMM_GATHER=layout)
+
+
+def test_gather_kind_is_that_of_the_products(hostrt):
+    """HIP_MatGatherKind names the kernel that products run with in the
+    matrix's present precision: a grid's natural order may be staged in FP64 only."""
+    hostrt("""
+KERNELS = ["k_spmm", "k_spmm_rows", "k_spmm_halo"]
+mats = [P.lap2d(40)[0], P.lap3d_mass(20)[1], P.chung_lu(20000)[0], P.lap3d_mass(85)[0]]
+kinds = []
+for M in mats:
+    A = Matrix(M)
+    kinds.append([])
+    for prec in (F64, F32):
+        A.set_precision(prec)
+        kind = capi.load().HIP_MatGatherKind(A.ptr)
+        kinds[-1].append(kind)
+        A.set_precision(F64)
+        x, y = MultiVec(A, 3, prec), MultiVec(A, 3, prec)
+        assert KERNELS[kind] in launched(lambda: ops.matdot(A, x, y)), (kind, prec, A.n)
+assert kinds == [[2, 2], [2, 2], [1, 1], [2, 0]], kinds
+""")

@@ -1227,19 +1227,38 @@ static const int *mv_perm(const MV *m) { return (m->mat && m->mat->perm_h) ? m->
 template <typename T>
 static void host_to_dev_cols(MV *m, int start, int ncols, const double *host, int ldh)
 {
-    std::vector<T> buf((size_t)m->n);
+    const int64_t n = m->n;
+    std::vector<T> buf((size_t)n);
+    T *__restrict__ b = buf.data();
     const int *perm = mv_perm(m);
     for (int j = 0; j < ncols && !failed(); j++) {
         const double *hc = host + (size_t)j * ldh;
         if (perm)
-            for (int64_t i = 0; i < m->n; i++) buf[i] = (T)hc[perm[i]];
+            for (int64_t i = 0; i < n; i++) b[i] = (T)hc[perm[i]];
         else
-            for (int64_t i = 0; i < m->n; i++) buf[i] = (T)hc[i];
+            for (int64_t i = 0; i < n; i++) b[i] = (T)hc[i];
         check(hipMemcpy(col_ptr(m, start + j), buf.data(), sizeof(T) * m->n, hipMemcpyHostToDevice), "H2D column");
     }
 }
 
 static const int *mv_perm_d(const MV *m) { return mv_perm(m) ? mat_perm(m->mat) : nullptr; }
+
+// Whether host columns go through the device.  A launch and its wait, 12 us, and
+// in FP32 twice the bytes on the link stand against ordering and converting one
+// column after the other here (us, here / through the device):
+//   ordered FP64, 16,384 rows: 1 column up 16 / 27, 4 columns up 62 / 61 and down
+//   71 / 62; 90,000 rows: 1 column up 54 / 47; 400 rows: 16 columns up 184 / 159, 8
+//   columns down 94 / 69; 4,096 rows: 8 columns up 79 / 93, down 80 / 82
+//   ordered FP32, 16,384 rows: 8 columns up 108 / 110; 40,000: 4 up 84 / 79
+//   unordered FP32, 262,144 rows: 2 columns up 142 / 150, 4 up 279 / 262, 8 down
+//   725 / 903, 32 down 3974 / 3707
+static bool through_device(const MV *m, int ncols, bool upload)
+{
+    const double entries = (double)m->n * ncols;
+    const bool f64 = m->prec == GCGE_HIP_FP64;
+    if (mv_perm(m)) return ncols >= (upload ? 16 : 8) || entries >= (f64 ? 6e4 : 1.6e5);
+    return !f64 && entries >= (upload ? 1e6 : 4e6);
+}
 
 // Calls f(stage, c, k) for the columns c .. c + k - 1 of ncols, a few at a time
 // so that the device staging buffer stays below 64 MiB (or one column); false,
@@ -1266,7 +1285,7 @@ extern "C" GCGE_INT HIP_MultiVecSetFromHost(void **mv, GCGE_INT start, GCGE_INT 
     }
     if (!sync()) return g_err;
     if (mv_perm(m) || m->prec != GCGE_HIP_FP64) {
-        if (staged_columns_through(m, start, ncols, [&](double *stage, int c, int k) {
+        if (through_device(m, ncols, true) && staged_columns_through(m, start, ncols, [&](double *stage, int c, int k) {
                 if (!check(hipMemcpy2D(stage, sizeof(double) * m->n, host + (size_t)c * ldh, sizeof(double) * ldh,
                                        sizeof(double) * m->n, k, hipMemcpyHostToDevice),
                            "H2D 2D"))
@@ -1301,7 +1320,7 @@ extern "C" GCGE_INT HIP_MultiVecGetToHost(void **mv, GCGE_INT start, GCGE_INT nc
     }
     if (!sync()) return g_err;
     const int *perm = mv_perm(m);
-    if ((perm || m->prec != GCGE_HIP_FP64) &&
+    if (through_device(m, ncols, false) &&
         staged_columns_through(m, start, ncols, [&](double *stage, int c, int k) {
             launch_rows_out(m->prec, m->n, stage, m->n, mv_perm_d(m), col_ptr(m, start + c), m->ld, k);
             if (sync())

@@ -211,3 +211,26 @@ for M in mats:
         assert KERNELS[kind] in launched(lambda: ops.matdot(A, x, y)), (kind, prec, A.n)
 assert kinds == [[2, 2], [2, 2], [1, 1], [2, 0]], kinds
 """)
+
+
+def test_small_host_columns_are_ordered_and_converted_on_the_host(hostrt):
+    """Where a launch, its wait and FP32's doubled bytes on the link cost more
+    than the host's own work, no kernel runs; the columns are the same."""
+    hostrt("""
+M = P.lap2d(128)[0]
+n, g = M.shape[0], np.random.default_rng(0)
+plain, ordered = Matrix(M), Matrix(M, order=g.permutation(n).astype(np.int32))
+# matrix, precision, columns, kernels of an upload and a download
+UP, DOWN = ["k_rows_in"], ["k_rows_out"]
+for A, prec, k, up, down in ((ordered, F64, 1, [], []), (ordered, F64, 3, [], []), (ordered, F64, 4, UP, DOWN),
+                             (ordered, F32, 7, [], []), (ordered, F32, 9, [], DOWN), (ordered, F32, 10, UP, DOWN),
+                             (plain, F32, 1, [], []), (plain, F32, 61, [], []), (plain, F32, 62, UP, []),
+                             (plain, F32, 244, UP, []), (plain, F32, 245, UP, DOWN), (plain, F64, 100, [], [])):
+    x = MultiVec(A, k, prec)
+    X = np.asfortranarray(g.standard_normal((n, k)))
+    assert launched(lambda: x.set(X)) == up, (prec, k)
+    got = []
+    assert launched(lambda: got.append(x.get())) == down, (prec, k)
+    if not up and not down:
+        assert np.array_equal(got[0], X if prec == F64 else X.astype(np.float32).astype(np.float64))
+""")

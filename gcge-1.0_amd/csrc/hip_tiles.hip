@@ -34,6 +34,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "gram_shape.h"
 #include "hip_common.h"
 
 namespace gh {
@@ -44,8 +45,6 @@ constexpr int kThreads = 256;       // 4 wavefronts per workgroup
 constexpr int kGramTargetWG = 2048; // workgroups a Gram launch aims for
 constexpr double kRowsBytes = 200e6;  // X and Y of k_lincomb_rows at most
 constexpr int kSlabThreads = 512;   // slab Gram: 8 wavefronts per workgroup
-constexpr int kSlabTiles = 28;      // most 16-column tiles of V and W together in its block (7 units per thread)
-constexpr int kSlabMaxNT = 17;      // most output tiles per wavefront
 
 typedef double dx4 __attribute__((ext_vector_type(4)));
 typedef float fx4 __attribute__((ext_vector_type(4)));
@@ -1071,49 +1070,6 @@ void launch_gram_mfma(const GramShape &g, int grid, int64_t n, const void *V, in
     GH_GRAM(1, 2, 1, 2)
     GH_GRAM(2, 2, 2, 2)
 #undef GH_GRAM
-}
-
-// Blocks of a slab Gram launch: p16 x q16 tiles cut into bp x bq blocks of
-// MB x NB tiles, NT of them per wavefront
-struct SlabShape {
-    int bp, bq, MB, NB, NT;
-};
-
-// Most tiles that a block computes
-int slab_live(int p16, int q16, int MB, int NB, bool upper)
-{
-    if (!upper) return std::min(MB, p16) * std::min(NB, q16);
-    int most = 0;
-    for (int i = 0; i < p16; i += MB)
-        for (int j = 0; j < q16; j += NB) {
-            int live = 0;
-            for (int y = j; y < std::min(q16, j + NB); y++)
-                live += std::max(0, std::min(std::min(MB, p16 - i), y - i + 1));
-            most = std::max(most, live);
-        }
-    return most;
-}
-
-// The cheapest cut: per row, a tile of products costs about 1, a tile's 16
-// columns 3.5 to load (67 TF and 5 TB/s in FP64, 153 TF in FP32).
-SlabShape slab_shape(int p16, int q16, bool upper)
-{
-    SlabShape best{0, 0, 0, 0, 0};
-    double least = 0.0;
-    for (int bp = 1; bp <= p16; bp++)
-        for (int bq = 1; bq <= q16; bq++) {
-            // many more blocks than some cut needs only load more
-            if (best.bp > 0 && bp * bq > 4 * best.bp * best.bq) break;
-            const int MB = (p16 + bp - 1) / bp, NB = (q16 + bq - 1) / bq;
-            const int NT = (slab_live(p16, q16, MB, NB, upper) + 7) / 8;
-            if (MB + NB > kSlabTiles || NT > kSlabMaxNT) continue;
-            const double cost = (double)bp * bq * (8.0 * NT + 3.5 * (MB + NB));
-            if (best.bp == 0 || cost < least) {
-                least = cost;
-                best = {(p16 + MB - 1) / MB, (q16 + NB - 1) / NB, MB, NB, NT};
-            }
-        }
-    return best;
 }
 
 // Blocks of up to 16 columns of tiles (74 KiB of LDS, at most 8 tiles per

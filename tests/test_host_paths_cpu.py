@@ -234,3 +234,13 @@ for A, prec, k, up, down in ((ordered, F64, 1, [], []), (ordered, F64, 3, [], []
     if not up and not down:
         assert np.array_equal(got[0], X if prec == F64 else X.astype(np.float32).astype(np.float64))
 """)
+
+
+def test_cut_of_the_slab_gram_kernel(tmp_path):
+    """Every block's tiles fit its wavefronts, and the choice is cheap for many
+    columns too."""
+    exe = str(tmp_path / "gram_shape")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "gcge-1.0_amd", "csrc"),
+                    os.path.join(HERE, "hostrt", "gram_shape.cpp"), "-o", exe], check=True)
+    p = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout

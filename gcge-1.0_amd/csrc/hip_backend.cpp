@@ -18,6 +18,7 @@
 #include <cstdlib>
 #include <cstddef>
 #include <cstring>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -772,7 +773,7 @@ static void host_parallel(int parts, F f)
 // consecutive rows whenever they fit, =columns or =rows never.  Rows longer
 // than kLongRow (k_spmm_long) are left out.
 static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col)
-{
+try {
     const char *e = getenv("GCGE_HIP_SPMM_GATHER");
     const bool forced = e && !strcmp(e, "halo");
     if (e && !forced) return true;
@@ -857,6 +858,8 @@ static bool build_halo(HIP_MAT *A, const int *rowptr, const int *col)
     A->halo_bytes = 4.0 * (double)(hptr.size() + nh + (br.order ? order.size() : 0)) + 2.0 * (double)lcol.size();
     g_ctx.dev_bytes += A->halo_bytes;
     return true;
+} catch (const std::bad_alloc &) {
+    return true;  // out of host memory, before any of the device's: keep the other layouts
 }
 
 // Gather layout of the SpMM.  The row-major path is used when

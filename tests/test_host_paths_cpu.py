@@ -244,3 +244,24 @@ def test_cut_of_the_slab_gram_kernel(tmp_path):
                     os.path.join(HERE, "hostrt", "gram_shape.cpp"), "-o", exe], check=True)
     p = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, p.stdout
+
+
+def test_matrix_without_host_memory_for_staged_blocks(hostrt):
+    """A matrix whose staged blocks do not fit host memory takes another layout;
+    nothing is thrown through the C entry."""
+    hostrt("""
+import resource
+M = P.lap3d_mass(90)[1]
+rowptr, col, val = M.indptr.astype(np.int32), M.indices.astype(np.int32), np.ascontiguousarray(M.data)
+L = capi.load()
+small = Matrix(P.lap3d_mass(12)[1])
+with open("/proc/self/statm") as f:
+    now = int(f.read().split()[0]) * resource.getpagesize()
+device = 12 * M.nnz + 4 * M.shape[0]
+resource.setrlimit(resource.RLIMIT_AS, (now + device + 24 * 1024 * 1024,) * 2)
+A = L.HIP_MatCreateFromCSR(M.shape[0], M.shape[0], M.nnz, rowptr.ctypes.data_as(capi.IP),
+                           col.ctypes.data_as(capi.IP), val.ctypes.data_as(capi.DP))
+capi.raise_on_error("create")
+assert L.HIP_MatGatherKind(A) == 1, L.HIP_MatGatherKind(A)
+assert L.HIP_MatGatherKind(small.ptr) == 2
+""")

@@ -13,7 +13,6 @@
 #include <cmath>
 #include <cstring>
 #include <climits>
-#include <initializer_list>
 #include <type_traits>
 #include <vector>
 
@@ -1488,27 +1487,17 @@ static ColScalars make_scalars(int k, const double *a, const double *b, const in
     return s;
 }
 
-// Every access of 16 bytes aligned: column starts and distances
-static bool wide_ok(int prec, std::initializer_list<const void *> ptrs, std::initializer_list<int64_t> lds)
-{
-    for (const void *p : ptrs)
-        if ((uintptr_t)p & 15u) return false;
-    for (int64_t ld : lds)
-        if (ld * (int64_t)elem_size(prec) % 16) return false;
-    return true;
-}
-
 // Grid of an element-wise kernel: every thread one run of V rows
 static dim3 run_grid(int64_t n, int V, int k) { return dim3((unsigned)((n + (int64_t)kBlock * V - 1) / (kBlock * V)), k); }
 
-// Calls f(V, NT) with constants: 16-byte accesses where aligned, past the
-// caches where more than kStreamBytes are touched
+// Calls f(V, NT) with constants: 16-byte accesses (a multivector's columns
+// start on 1 KiB or 2 KiB boundaries), past the caches where more than
+// kStreamBytes are touched
 template <typename T, typename F>
-static void run_variant(bool wide, double bytes, F f)
+static void run_variant(double bytes, F f)
 {
     using W = std::integral_constant<int, kWide<T>>;
-    if (!wide) f(std::integral_constant<int, 1>{}, std::false_type{});
-    else if (bytes > kStreamBytes) f(W{}, std::true_type{});
+    if (bytes > kStreamBytes) f(W{}, std::true_type{});
     else f(W{}, std::false_type{});
 }
 
@@ -1525,9 +1514,9 @@ static void sum_variant(int64_t n, double bytes, F f)
 
 template <typename T>
 static void axpby_t(int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k, const ColScalars &s,
-                    bool wide, double bytes)
+                    double bytes)
 {
-    run_variant<T>(wide, bytes, [&](auto V, auto NT) {
+    run_variant<T>(bytes, [&](auto V, auto NT) {
         k_axpby<T, V(), NT()><<<run_grid(n, V(), k), kBlock, 0, ctx().stream>>>(n, (const T *)x, ldx, (T *)y, ldy, s);
     });
 }
@@ -1540,9 +1529,8 @@ void launch_axpby(int prec, int64_t n, const void *x, int64_t ldx, void *y, int6
     double bytes = 0.0;
     for (int j = 0; j < k; j++) bytes += (double)n * elem_size(prec) * ((s.a[j] == 0.0 || s.b[j] == 0.0) ? 2 : 3);
     ProfScope ps(K_AXPBY, bytes, 0.0);
-    const bool wide = wide_ok(prec, {x, y}, {ldx, ldy});
-    if (prec == GCGE_HIP_FP64) axpby_t<double>(n, x, ldx, y, ldy, k, s, wide, bytes);
-    else axpby_t<float>(n, x, ldx, y, ldy, k, s, wide, bytes);
+    if (prec == GCGE_HIP_FP64) axpby_t<double>(n, x, ldx, y, ldy, k, s, bytes);
+    else axpby_t<float>(n, x, ldx, y, ldy, k, s, bytes);
     check(hipGetLastError(), "k_axpby");
 }
 
@@ -1643,11 +1631,12 @@ bool dots_with(int prec, int64_t n, const void *x, int64_t ldx, const void *y, i
 }
 
 template <typename TX, typename TY>
-static void copy_t(int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k, bool wide, double bytes)
+static void copy_t(int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k, double bytes)
 {
-    // accesses of 16 bytes on the narrower side, 16 or 32 on the other
+    // accesses of 16 bytes on the narrower side, 16 or 32 on the other (a run of 4
+    // rows in FP64 is one vector of 32 bytes)
     using T = std::conditional_t<(sizeof(TX) < sizeof(TY)), TX, TY>;
-    run_variant<T>(wide, bytes, [&](auto V, auto NT) {
+    run_variant<T>(bytes, [&](auto V, auto NT) {
         k_copy<TX, TY, V(), NT()><<<run_grid(n, V(), k), kBlock, 0, ctx().stream>>>(n, (const TX *)x, ldx, (TY *)y,
                                                                                     ldy);
     });
@@ -1658,14 +1647,10 @@ void launch_copy(int xprec, const void *x, int64_t ldx, int yprec, void *y, int6
     if (k <= 0 || n <= 0 || failed()) return;
     const double bytes = (double)k * n * (elem_size(xprec) + elem_size(yprec));
     ProfScope ps(K_COPY, bytes, 0.0);
-    // a run of 4 rows in FP64 is one vector of 32 bytes
-    const bool mixed = xprec != yprec;
-    const bool wide = wide_ok(xprec, {x}, {ldx}) && wide_ok(yprec, {y}, {ldy}) &&
-                      (!mixed || ((((uintptr_t)x | (uintptr_t)y) & 31u) == 0 && ldx % 8 == 0 && ldy % 8 == 0));
-    if (xprec == GCGE_HIP_FP64 && yprec == GCGE_HIP_FP64) copy_t<double, double>(n, x, ldx, y, ldy, k, wide, bytes);
-    else if (xprec == GCGE_HIP_FP64) copy_t<double, float>(n, x, ldx, y, ldy, k, wide, bytes);
-    else if (yprec == GCGE_HIP_FP64) copy_t<float, double>(n, x, ldx, y, ldy, k, wide, bytes);
-    else copy_t<float, float>(n, x, ldx, y, ldy, k, wide, bytes);
+    if (xprec == GCGE_HIP_FP64 && yprec == GCGE_HIP_FP64) copy_t<double, double>(n, x, ldx, y, ldy, k, bytes);
+    else if (xprec == GCGE_HIP_FP64) copy_t<double, float>(n, x, ldx, y, ldy, k, bytes);
+    else if (yprec == GCGE_HIP_FP64) copy_t<float, double>(n, x, ldx, y, ldy, k, bytes);
+    else copy_t<float, float>(n, x, ldx, y, ldy, k, bytes);
     check(hipGetLastError(), "k_copy");
 }
 
@@ -2160,7 +2145,6 @@ void launch_cg_search(int prec, int64_t n, void *x, int64_t ldx, void *p, int64_
 {
     const int k = std::max(kx, kp);
     if (k <= 0 || failed()) return;
-    const bool wide = wide_ok(prec, {x, p, r, dinv}, {ldx, ldp, ldr});
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         const int kxc = std::max(0, std::min(kc, kx - c0)), kpc = std::max(0, std::min(kc, kp - c0));
@@ -2175,7 +2159,7 @@ void launch_cg_search(int prec, int64_t n, void *x, int64_t ldx, void *p, int64_
                          0.0);
             const double held = (1.0 * kxc + kpc + kc) * (double)n * elem_size(prec);  // x, r and p
 #define GH_SEARCH(T_, PRE_)                                                                                     \
-    run_variant<T_>(wide, held, [&](auto V, auto NT) {                                                          \
+    run_variant<T_>(held, [&](auto V, auto NT) {                                                          \
         k_cg_search<T_, PRE_, V(), NT()><<<run_grid(n, V(), kc), kBlock, 0, ctx().stream>>>(                    \
             n, (T_ *)x + (int64_t)c0 * ldx, ldx, (T_ *)p + (int64_t)c0 * ldp, ldp,                              \
             (const T_ *)r + (int64_t)c0 * ldr, ldr, kxc, kpc, s, (const T_ *)dinv);                             \

@@ -149,8 +149,10 @@ double *host_partials(size_t count);
 // Waits until the launch has written all of them; false (latched) on an error.
 bool wait_partials(size_t count);
 // Copy small host data (coefficients) to device memory without blocking:
-// the bytes go through a pinned ring whose slots are reused only after the
-// next stream synchronisation.  Returns the device address.
+// the bytes go through a pinned ring whose slots are reused only after the next
+// stream synchronisation, or after the results of a later launch have reached
+// the host (wait_seq, wait_partials): the copies and the launches that read them
+// come before it on the stream.  Returns the device address.
 void *stage_to_device(const void *host, size_t bytes);
 bool sync();                           // stream synchronize + error check
 

@@ -22,8 +22,8 @@
 // Very thin products (p <= 4, q <= 8 or the transpose) take a vector kernel
 // that keeps the whole p x q block in registers and reads V and W once.
 //
-// LinComb: a wavefront owns 32 (FP64) or 64 (FP32) rows of Y and all its
-// columns up to 128; X supplies the A operand straight from HBM, C the B
+// LinComb: a wavefront owns 16, 32 or (FP32) 64 rows of Y, as leave workgroups
+// enough, and all its columns up to 128; X supplies the A operand straight from HBM, C the B
 // operand from a copy packed on the host in operand order and staged through
 // LDS for the workgroup.  Thin combinations (p, q <= 8) take a vector kernel
 // with C in the kernel arguments and 16-byte row vectors.
@@ -275,9 +275,14 @@ __global__ __launch_bounds__(kThreads) void k_gram_mfma(int64_t n, const T *__re
 // whatever MB and NB: every SIMD has the same number of products.
 // UPT: 16-byte units that a thread copies per slab, at least (MB + NB) / 4.
 // Product t = 0 .. E - 1 of step 0 or 1, E = 16 / sizeof(T), takes row
-// 4 E step + 4 t + l / 16  of the slab for both operands, or with RUN (up to 64
-// x 64 columns, as in k_gram_mfma, and past 256)  2 E (l / 16) + E step + t,
-// which a lane reads at once: 4 % faster.
+// 4 E step + 4 t + l / 16  of the slab for both operands, or with RUN
+// 2 E (l / 16) + E step + t, which a lane reads at once: 4 - 8 % faster at every
+// size.  The two add the rows in different orders.  From 65 to 256 columns the
+// slower one stays, because its sums keep the bits they had before this kernel
+// and with them the course of solves whose pairs lie at the tolerance (the other
+// order moved residuals of a power-law graph's locked pairs to 1.04e-8, above
+// their 1e-8); up to 64 columns k_gram_mfma's order is RUN's, and past 256 the chunks
+// changed anyway.
 // Bound by memory for few columns (4.0 - 4.6 TB/s: each visit of a column
 // reads 128 bytes of another page), by the matrix cores for many (67 TF in
 // FP64 and 153 in FP32 for a large library product here; 46 and 84 reached, 53
@@ -743,20 +748,6 @@ __global__ __launch_bounds__(kThreads, RN <= 2 ? 4 : RN <= 4 ? 3 : 2) void k_lin
     }
 }
 
-// The same products for few columns of few rows: a wavefront owns rows [rb, rb +
-// 32) as two 16-row blocks, walks the output in groups of RN 16-column blocks
-// and reads C from the caches; no LDS and no barriers, so more wavefronts are in
-// flight, which is what a memory-bound product needs while X and Y fit the
-// 256 MB cache (kRowsBytes, below it because other data is there too).  This
-// kernel against k_lincomb_mfma, us: FP32 20 x 20, 512,000 rows (82 MB) 21.5
-// against 25.0, 884,736 (142 MB) 32.1 against 37.7, 4.1M (655 MB) 159 against
-// 147; 40 x 40, 262,144 rows (84 MB) 26.7 against 26.9, 884,736 (283 MB) 91
-// against 72, 4.1M 374 against 285; FP64 20 x 20, 512,000 rows (164 MB) 37.4
-// against 40.7, 884,736 (283 MB) 71.0 against 69.8.  Where q or p are larger it
-// is the slower one at any size: FP32 150 x 50 over 4.1M rows 1.087 against 0.999
-// ms, 300 x 100 over 16,384 30.1 against 29.1 us (but 200 x 100 23.5 against
-// 25.5); FP64 50 x 50 over 4.1M rows 1.080 against 0.840.  slot t of lane l holds row drow(l / 16, t) of its block
-// and column l % 16.
 // Result rows of one lane after regrouping: lane (g = l / 16, m) returns
 // rows 4 g .. 4 g + 3 of column m of the 16 x 16 block.  For FP32 these are
 // already its four slots; for FP64 (slot t holds row 4 t + g) the four lanes
@@ -811,6 +802,20 @@ __device__ __forceinline__ void store_rows4(T *y, typename MT<T>::acc_t v, T al,
     *reinterpret_cast<v4 *>(y) = out;
 }
 
+// The products of k_lincomb_mfma for few columns of few rows: a wavefront owns
+// rows [rb, rb + 32) as two 16-row blocks (slot t of lane l holds row drow(l /
+// 16, t) of its block and column l % 16), walks the output in groups of RN
+// 16-column blocks and reads C from the caches; no LDS and no barriers, so more
+// wavefronts are in flight, which is what a memory-bound product needs while X
+// and Y fit the 256 MB cache (kRowsBytes, below it because other data is there
+// too).  This kernel against k_lincomb_mfma, us: FP32 20 x 20, 512,000 rows (82
+// MB) 21.5 against 25.0, 884,736 (142 MB) 32.1 against 37.7, 4.1M (655 MB) 159
+// against 147; 40 x 40, 262,144 rows (84 MB) 26.7 against 26.9, 884,736 (283 MB)
+// 91 against 72, 4.1M 374 against 285; FP64 20 x 20, 512,000 rows (164 MB) 37.4
+// against 40.7, 884,736 (283 MB) 71.0 against 69.8.  Where q or p are larger it
+// is the slower one at any size: FP32 150 x 50 over 4.1M rows 1.087 against
+// 0.999 ms, 300 x 100 over 16,384 30.1 against 29.1 us (but 200 x 100 23.5
+// against 25.5); FP64 50 x 50 over 4.1M rows 1.080 against 0.840.
 template <typename T, int RN, int WC>
 __global__ __launch_bounds__(kThreads) void k_lincomb_rows(int64_t n, const T *__restrict__ X, int64_t ldx, int p,
                                                            T *__restrict__ Y, int64_t ldy, int q,
@@ -1082,6 +1087,7 @@ template <typename T>
 void launch_gram_slab(const SlabShape &s, int grid, int64_t n, const void *V, int64_t ldv, int p, const void *W,
                       int64_t ldw, int q, int nchunk, int64_t rpc, int upper, double *partial)
 {
+    // run: by the bits to keep, not by speed (k_gram_slab)
     const bool small = p <= 64 && q <= 64, run = small || ((p > 256 || q > 256) && !slab_narrow(s));
     const int upt = small ? 2 : slab_narrow(s) ? 4 : 7;
 #define GH_SLAB(NT_, UPT_, RUN_)                                                                                \

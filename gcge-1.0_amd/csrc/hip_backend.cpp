@@ -51,6 +51,7 @@ bool failed() { return g_err != 0; }
 bool check(hipError_t e, const char *what)
 {
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // the runtime keeps it for the next launch's check
         latch((int)e, "%s: %s", what, hipGetErrorString(e));
         return false;
     }
@@ -81,8 +82,9 @@ bool ensure_ctx()
     return true;
 }
 
-// Live matrices, for the device copies of their orders
-static std::vector<HIP_MAT *> g_mats;
+// Live matrices, for the device copies of their orders (never destroyed: a
+// program may destroy matrices in its own static destructors)
+static std::vector<HIP_MAT *> &g_mats = *new std::vector<HIP_MAT *>;
 
 // Gives back what is kept for speed alone: the buffer of TmpDev and the
 // matrices' orders.  Calls fetch an order after their last allocation.

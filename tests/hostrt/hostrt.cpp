@@ -24,6 +24,7 @@ struct Call {
     void *stream;
 } g_call;
 constexpr int kNoMemory = 2;
+int g_last = 0;  // the last error, until it is asked for
 }  // namespace
 
 extern "C" {
@@ -45,7 +46,7 @@ const char *hostrt_launches()
 int hipMalloc(void **p, size_t n)
 {
     *p = nullptr;
-    if (g_live + n > g_limit) return kNoMemory;
+    if (g_live + n > g_limit) return g_last = kNoMemory;
     if (posix_memalign(p, 4096, n ? n : 1)) return kNoMemory;
     memset(*p, 0, n);
     g_blocks[*p] = n;
@@ -125,7 +126,12 @@ int hipEventElapsedTime(float *ms, void *, void *)
     *ms = 0.0f;
     return 0;
 }
-int hipGetLastError() { return 0; }
+int hipGetLastError()
+{
+    const int e = g_last;
+    g_last = 0;
+    return e;
+}
 const char *hipGetErrorString(int e) { return e == kNoMemory ? "out of memory" : "error"; }
 
 // ---- launches

@@ -265,3 +265,21 @@ capi.raise_on_error("create")
 assert L.HIP_MatGatherKind(A) == 1, L.HIP_MatGatherKind(A)
 assert L.HIP_MatGatherKind(small.ptr) == 2
 """)
+
+
+def test_cleared_error_does_not_come_back(hostrt):
+    """An allocation that failed is no error of the launches after
+    GCGE_HIP_ClearError."""
+    hostrt("""
+A = Matrix(P.lap2d(40)[0])
+x, y = MultiVec(A, 3, F64), MultiVec(A, 3, F64)
+rt.hostrt_limit(rt.hostrt_live())
+try:
+    MultiVec(A, 3, F64)
+    raise SystemExit("no error")
+except RuntimeError as e:
+    assert "out of memory" in str(e), e
+rt.hostrt_limit(1 << 40)
+ops.copy(x, y)
+ops.dots(x, y)
+""")

@@ -1220,6 +1220,28 @@ bool gram(int prec, int64_t n, const void *V, int64_t ldv, int p, const void *W,
     return true;
 }
 
+// Whether k_lincomb_rows is the faster kernel while X and Y fit the cache
+// (blocks: the column blocks that k_lincomb_mfma multiplies).  Few input columns
+// make a product of stores, which its many small wavefronts keep in flight;
+// against it stand the blocks that it multiplies for nothing, as it takes 4 or 8
+// at a time.  k_lincomb_mfma has enough workgroups from 65,536 rows on in FP64
+// (16,384 rows are one per CU) and from 262,144 in FP32.  us, this kernel / that
+// one:
+//   FP32, 110,592 rows: 3 x 200 20.1 / 34.6, 20 x 128 19.2 / 29.4, 20 x 65 15.7 /
+//   19.2, 64 x 65 29.0 / 27.7; 262,144: 12 x 128 31.1 / 31.6, 32 x 128 39.6 / 42.0
+//   FP64, 65,025 rows: 3 x 300 34.1 / 50.8, 48 x 64 18.3 / 23.0, 20 x 65 19.3 /
+//   19.8, 48 x 65 28.2 / 25.7; 16,384: 3 x 200 12.7 / 14.9, 48 x 48 12.3 / 11.6;
+//   125,316: 12 x 65 27.2 / 21.6
+static bool lincomb_by_rows(int prec, int64_t n, int p, int q, int blocks)
+{
+    const int nqb = (q + 15) / 16, mine = nqb <= 2 ? nqb : nqb <= 4 ? 4 : (nqb + 7) / 8 * 8;
+    const double pad = (double)mine / blocks, weight = p * pad * pad;
+    if (prec == GCGE_HIP_FP64)
+        return q <= 32 ? p <= 64 : n < 65536 && (n >= 24576 || q > 96) && weight < 64;
+    if (q <= 64) return p < 128 || weight <= 128;
+    return n < 262144 && weight < (n < 65536 ? 256 : 100);
+}
+
 bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, int64_t ldy, int q, const double *C,
              int ldc, double alpha, double beta)
 {
@@ -1257,11 +1279,10 @@ bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, in
     // column blocks per pass (RN, at most 8) so that the passes are equal;
     // k_lincomb_rows: 1, 2 or 4, beyond 4 by two wavefronts (WC)
     const int nkb = (p + 3) / 4, nqb0 = (q + 15) / 16;
-    const bool rows = (double)n * (p + q) * es <= kRowsBytes &&
-                      (prec == GCGE_HIP_FP64 ? q <= 32 && p < 64 : q <= 64 ? p < 128 : n < 65536 && p < 256);
+    const int groups = (nqb0 + 7) / 8, even = (nqb0 + groups - 1) / groups;
+    const bool rows = (double)n * (p + q) * es <= kRowsBytes && lincomb_by_rows(prec, n, p, q, even * groups);
     const int wc = rows && nqb0 > 4 ? 2 : 1;
-    const int groups = (nqb0 + 7) / 8;
-    const int rn = rows ? (nqb0 <= 2 ? nqb0 : 4) : (nqb0 + groups - 1) / groups;
+    const int rn = rows ? (nqb0 <= 2 ? nqb0 : 4) : even;
     const int nqb = ((nqb0 + rn * wc - 1) / (rn * wc)) * rn * wc;  // zero blocks pad the last pass
     const size_t ncp = (size_t)nkb * nqb * 64;
     const void *dC = nullptr;
@@ -1294,8 +1315,10 @@ bool lincomb(int prec, int64_t n, const void *X, int64_t ldx, int p, void *Y, in
         // k_lincomb_mfma: as many 16-row blocks per wavefront as leave 512 workgroups
         const int want = (int)std::min<int64_t>(4, n / (64 * 512));
         if (rows && prec == GCGE_HIP_FP64) {
-            if (rn == 1) GH_LR(double, 1, 1);
-            else GH_LR(double, 2, 1);
+            if (wc == 2) GH_LR(double, 4, 2);
+            else if (rn == 1) GH_LR(double, 1, 1);
+            else if (rn == 2) GH_LR(double, 2, 1);
+            else GH_LR(double, 4, 1);
         } else if (rows) {
             if (wc == 2) GH_LR(float, 4, 2);
             else if (rn == 1) GH_LR(float, 1, 1);

@@ -14,7 +14,7 @@ from test_gpu_raw import padded
 pytestmark = pytest.mark.gpu
 
 F64, F32 = capi.GCGE_HIP_FP64, capi.GCGE_HIP_FP32
-ROWS = {1: 1, 1369: 37, 16900: 130, 99856: 316, 140625: 375}  # rows: side of the 2-D grid
+ROWS = {1: 1, 1369: 37, 16900: 130, 39601: 199, 99856: 316, 140625: 375}  # rows: side of the 2-D grid
 
 
 @pytest.fixture(scope="module")
@@ -54,6 +54,15 @@ def test_lincomb_exact(ops, mats, prec, n, p, q, beta):
     x, y = padded(mats[n], X, prec), padded(mats[n], Y, prec)
     ops.lincomb(x, y, C, alpha=-1.0, beta=beta)
     assert np.array_equal(y.get(), -(X @ C) + (beta * Y if beta else 0.0))
+
+
+@pytest.mark.parametrize("prec", [F64, F32])
+@pytest.mark.parametrize("n", [1, 1369, 39601, 99856])
+# few columns into many, on both sides of the choice between the two kernels
+@pytest.mark.parametrize("p,q,beta", [(1, 300, 0.0), (3, 200, 1.0), (12, 128, -1.0), (20, 48, 1.0), (25, 65, 0.0),
+                                      (64, 64, 1.0), (20, 120, 0.0), (99, 113, 2.0)])
+def test_lincomb_of_few_into_many(ops, mats, prec, n, p, q, beta):
+    test_lincomb_exact(ops, mats, prec, n, p, q, beta)
 
 
 @pytest.mark.parametrize("prec", [F64, F32])

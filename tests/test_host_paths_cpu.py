@@ -283,3 +283,22 @@ rt.hostrt_limit(1 << 40)
 ops.copy(x, y)
 ops.dots(x, y)
 """)
+
+
+def test_kernel_of_a_combination(hostrt):
+    """Few columns into many take the kernel without LDS while the blocks fit the
+    cache and the other one does not fill the chip."""
+    hostrt("""
+for side, prec, p, q, rows in ((128, F64, 3, 200, 1), (128, F64, 12, 48, 0), (255, F64, 3, 300, 1), (255, F64, 20, 64, 1),
+                               (255, F64, 48, 65, 0), (257, F64, 3, 300, 0), (128, F64, 64, 32, 1), (128, F64, 65, 32, 0),
+                               (333, F32, 3, 200, 1), (333, F32, 20, 120, 1), (333, F32, 64, 65, 0),
+                               (200, F32, 99, 65, 1), (200, F32, 128, 64, 1), (200, F32, 129, 64, 0),
+                               (200, F32, 127, 33, 1), (200, F32, 128, 33, 0), (512, F32, 3, 65, 0),
+                               (512, F32, 3, 64, 1), (800, F32, 12, 128, 0)):
+    A = Matrix(P.lap2d(side)[0])
+    x, y = MultiVec(A, p, prec), MultiVec(A, q, prec)
+    names = launched(lambda: ops.lincomb(x, y, np.ones((p, q))))
+    assert names[-1] == ("k_lincomb_rows" if rows else "k_lincomb_mfma"), (side, prec, p, q, names)
+    for o in (x, y, A):
+        o.close()
+""")

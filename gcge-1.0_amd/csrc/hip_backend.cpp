@@ -453,9 +453,13 @@ const float *mat_val32(HIP_MAT *A)
 const void *mat_dinv(HIP_MAT *A, int prec)
 {
     if (!A->dinv64) {
-        const size_t n = (size_t)std::max(1, A->n);
+        const size_t n = (size_t)((std::max(1, A->n) + 3) / 4 * 4);  // whole runs of 4 rows (load_run)
         if (!check(dev_malloc((void **)&A->dinv64, sizeof(double) * n), "hipMalloc dinv64")) return nullptr;
-        if (!check(dev_malloc((void **)&A->dinv32, sizeof(float) * n), "hipMalloc dinv32")) return nullptr;
+        if (!check(dev_malloc((void **)&A->dinv32, sizeof(float) * n), "hipMalloc dinv32")) {
+            (void)hipFree(A->dinv64);
+            A->dinv64 = nullptr;
+            return nullptr;
+        }
         g_ctx.dev_bytes += 12.0 * (double)n;
         launch_diag_inv(A);
         if (failed()) return nullptr;

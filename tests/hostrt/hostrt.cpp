@@ -33,7 +33,7 @@ size_t hostrt_live() { return g_live; }
 void hostrt_limit(size_t bytes) { g_limit = bytes; }
 // called with the name and the arguments' addresses of every launch
 void hostrt_hook(void (*f)(const char *, void **)) { g_hook = f; }
-// names of the kernels launched since the last call, one a line
+// the kernels launched since the last call, one a line: mangled name and grid
 const char *hostrt_launches()
 {
     static std::string out;
@@ -163,7 +163,7 @@ int __hipPopCallConfiguration(Dim *grid, Dim *block, size_t *lds, void **stream)
 int hipLaunchKernel(const void *f, Dim grid, Dim, void **args, size_t, void *)
 {
     const std::string &name = g_names[f];
-    g_log += name + "\n";
+    g_log += name + " " + std::to_string(grid.x) + " " + std::to_string(grid.y) + "\n";
     if (g_hook) g_hook(name.c_str(), args);
     // arguments (..., numbers, number) of the two kernels that report
     const int at = name.find("k_reduce_rows_host") != std::string::npos ? 3

@@ -26,15 +26,21 @@ F64, F32 = capi.GCGE_HIP_FP64, capi.GCGE_HIP_FP32
 ops = Ops()
 Hook = C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_void_p))
 
-def launched(f):
-    '''names of the kernels that f() launches'''
+def launches(f):
+    '''kernels that f() launches: [name, mangled template arguments and
+    parameters, grid x, grid y]'''
     rt.hostrt_launches()
     f()
     out = []
-    for name in rt.hostrt_launches().decode().split():
+    for line in rt.hostrt_launches().decode().splitlines():
+        name, gx, gy = line.split()
         i = name.index("k_")
-        out.append(name[i:i + int(name[:i].split("_1")[-1])])
+        j = i + int(name[:i].split("_1")[-1])
+        out.append([name[i:j], name[j:], int(gx), int(gy)])
     return out
+
+def launched(f):
+    return [x[0] for x in launches(f)]
 """
 
 
@@ -301,4 +307,22 @@ for side, prec, p, q, rows in ((128, F64, 3, 200, 1), (128, F64, 12, 48, 0), (25
     assert names[-1] == ("k_lincomb_rows" if rows else "k_lincomb_mfma"), (side, prec, p, q, names)
     for o in (x, y, A):
         o.close()
+""")
+
+
+def test_columns_of_a_search_update_meet_on_one_xcd(hostrt):
+    """Workgroups go to the 8 XCDs in turn: with a multiple of 8 per column the
+    same rows of every column, and the diagonal's, lie in one XCD's L2."""
+    hostrt("""
+for side in (3, 37, 300, 512, 1015):
+    A = Matrix(P.lap2d(side)[0])
+    for prec in (F64, F32):
+        x, p, r = (MultiVec(A, 3, prec) for _ in range(3))
+        (name, _, gx, gy), = [k for k in launches(lambda: ops.pcg_search_update(A, x, 0, p, r, 3, 3, np.ones(3),
+                                                                                np.ones(3))) if "search" in k[0]]
+        rows = 256 * (2 if prec == F64 else 4)
+        assert gx % 8 == 0 and gy == 3 and gx * rows >= side * side, (side, prec, gx, gy)
+        for o in (x, p, r):
+            o.close()
+    A.close()
 """)

@@ -326,3 +326,14 @@ for side in (3, 37, 300, 512, 1015):
             o.close()
     A.close()
 """)
+
+
+def test_accesses_of_the_element_wise_kernels(hostrt):
+    """Copies store 16 bytes per thread in either direction of a conversion."""
+    hostrt("""
+A = Matrix(P.lap2d(40)[0])
+v = {(p, i): MultiVec(A, 3, p) for p in (F64, F32) for i in (0, 1)}
+for a, b, types in ((F64, F64, "IddLi2E"), (F64, F32, "IdfLi4E"), (F32, F64, "IfdLi2E"), (F32, F32, "IffLi4E")):
+    (name, rest, _, _), = launches(lambda: ops.copy(v[a, 0], v[b, 1]))
+    assert name == "k_copy" and rest.startswith(types), (name, rest)
+""")

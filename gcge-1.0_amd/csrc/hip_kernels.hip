@@ -1526,10 +1526,10 @@ static dim3 run_grid(int64_t n, int V, int k)
 // start on 1 KiB or 2 KiB boundaries), past the caches where more than
 // kStreamBytes are touched
 template <typename T, typename F>
-static void run_variant(double bytes, F f)
+static void run_variant(double held, F f)
 {
     using W = std::integral_constant<int, kWide<T>>;
-    if (bytes > kStreamBytes) f(W{}, std::true_type{});
+    if (held > kStreamBytes) f(W{}, std::true_type{});
     else f(W{}, std::false_type{});
 }
 
@@ -1546,9 +1546,9 @@ static void sum_variant(int64_t n, double bytes, F f)
 
 template <typename T>
 static void axpby_t(int64_t n, const void *x, int64_t ldx, void *y, int64_t ldy, int k, const ColScalars &s,
-                    double bytes)
+                    double held)
 {
-    run_variant<T>(bytes, [&](auto V, auto NT) {
+    run_variant<T>(held, [&](auto V, auto NT) {
         k_axpby<T, V(), NT()><<<run_grid(n, V(), k), kBlock, 0, ctx().stream>>>(n, (const T *)x, ldx, (T *)y, ldy, s);
     });
 }
@@ -1558,11 +1558,14 @@ void launch_axpby(int prec, int64_t n, const void *x, int64_t ldx, void *y, int6
 {
     if (k <= 0 || n <= 0 || failed()) return;
     ColScalars s = make_scalars(k, a, b, xidx);
-    double bytes = 0.0;
-    for (int j = 0; j < k; j++) bytes += (double)n * elem_size(prec) * ((s.a[j] == 0.0 || s.b[j] == 0.0) ? 2 : 3);
+    double bytes = 0.0, held = 0.0;  // moved; y is read and written but held once
+    for (int j = 0; j < k; j++) {
+        bytes += (double)n * elem_size(prec) * ((s.a[j] == 0.0 || s.b[j] == 0.0) ? 2 : 3);
+        held += (double)n * elem_size(prec) * (s.a[j] == 0.0 ? 1 : 2);
+    }
     ProfScope ps(K_AXPBY, bytes, 0.0);
-    if (prec == GCGE_HIP_FP64) axpby_t<double>(n, x, ldx, y, ldy, k, s, bytes);
-    else axpby_t<float>(n, x, ldx, y, ldy, k, s, bytes);
+    if (prec == GCGE_HIP_FP64) axpby_t<double>(n, x, ldx, y, ldy, k, s, held);
+    else axpby_t<float>(n, x, ldx, y, ldy, k, s, held);
     check(hipGetLastError(), "k_axpby");
 }
 

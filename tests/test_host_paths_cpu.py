@@ -329,11 +329,18 @@ for side in (3, 37, 300, 512, 1015):
 
 
 def test_accesses_of_the_element_wise_kernels(hostrt):
-    """Copies store 16 bytes per thread in either direction of a conversion."""
+    """Copies store 16 bytes per thread in either direction of a conversion; the
+    caches are passed by where the columns, each counted once, exceed 384 MB."""
     hostrt("""
 A = Matrix(P.lap2d(40)[0])
 v = {(p, i): MultiVec(A, 3, p) for p in (F64, F32) for i in (0, 1)}
 for a, b, types in ((F64, F64, "IddLi2E"), (F64, F32, "IdfLi4E"), (F32, F64, "IfdLi2E"), (F32, F32, "IffLi4E")):
     (name, rest, _, _), = launches(lambda: ops.copy(v[a, 0], v[b, 1]))
     assert name == "k_copy" and rest.startswith(types), (name, rest)
+
+B = Matrix(P.lap2d(1015)[0])
+x, y = MultiVec(B, 24, F64), MultiVec(B, 24, F64)
+for a, b, k, past in ((0.5, 0.5, 16, 0), (0.0, 0.5, 24, 0), (0.5, 0.5, 23, 0), (0.5, 0.5, 24, 1), (1.0, 0.0, 24, 1)):
+    (name, rest, _, _), = launches(lambda: ops.axpby(a, x, b, y, k=k))
+    assert name == "k_axpby" and rest.startswith("IdLi2ELb%dE" % past), (a, b, k, rest)
 """)

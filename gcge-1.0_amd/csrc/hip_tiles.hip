@@ -278,11 +278,12 @@ __global__ __launch_bounds__(kThreads) void k_gram_mfma(int64_t n, const T *__re
 // 4 E step + 4 t + l / 16  of the slab for both operands, or with RUN
 // 2 E (l / 16) + E step + t, which a lane reads at once: 4 - 8 % faster at every
 // size.  The two add the rows in different orders.  From 65 to 256 columns the
-// slower one stays, because its sums keep the bits they had before this kernel
-// and with them the course of solves whose pairs lie at the tolerance (the other
-// order moved residuals of a power-law graph's locked pairs to 1.04e-8, above
-// their 1e-8); up to 64 columns k_gram_mfma's order is RUN's, and past 256 the chunks
-// changed anyway.
+// slower one stays: with up to 128 columns on one side its sums keep the bits
+// they had before this kernel, and with them the course of solves whose pairs lie
+// at the tolerance (the other order moved residuals of a power-law graph's locked
+// pairs to 1.04e-8, above their 1e-8).  Up to 64 columns k_gram_mfma's order is
+// RUN's; with more than 128 on both sides, and past 256, the chunks changed
+// anyway.
 // Bound by memory for few columns (4.0 - 4.6 TB/s: each visit of a column
 // reads 128 bytes of another page), by the matrix cores for many (67 TF in
 // FP64 and 153 in FP32 for a large library product here; 46 and 84 reached, 53

@@ -1361,6 +1361,8 @@ __global__ __launch_bounds__(kBlock) void k_diag_inv(int n, const int *__restric
 // p = r + beta p (MultiVecAxpbyDiag(1, r, beta, p)) for the columns j < kp
 // With PRE, the search direction is built from z = dinv .* r (the Jacobi-
 // preconditioned residual, formed here rather than stored).
+constexpr int kLoadsDone = 0x0f70;  // s_waitcnt vmcnt(0), nothing else
+
 template <typename T, bool PRE, int V, bool NT>
 __global__ __launch_bounds__(kBlock) void k_cg_search(int64_t n, T *__restrict__ x, int64_t ldx,
                                                       T *__restrict__ p, int64_t ldp, const T *__restrict__ r,
@@ -1390,10 +1392,18 @@ __global__ __launch_bounds__(kBlock) void k_cg_search(int64_t n, T *__restrict__
         store_run<T, V, NT>(pj, i, n, pv);
     };
     if (j < kx && j < kp) {
+        // Past the caches the three streams are better read one after the other
+        // (40 columns of 4.1M rows, us, together / in turn: FP32 528 / 515, FP64 1052
+        // / 1017; with the diagonal FP32 513 / 517, 24 columns 311 / 305, FP64 1102 /
+        // 1085, where the last wait gains nothing)
         load_run<T, V, NT>(pj, i, pv);
+        if constexpr (NT) __builtin_amdgcn_s_waitcnt(kLoadsDone);
         load_run<T, V, NT>(xj, i, xv);
+        if constexpr (NT) __builtin_amdgcn_s_waitcnt(kLoadsDone);
         load_r();
+        if constexpr (NT && !PRE) __builtin_amdgcn_s_waitcnt(kLoadsDone);
         put_x();
+        if constexpr (NT) __builtin_amdgcn_s_waitcnt(kLoadsDone);
         put_p();
     } else if (j < kx) {
         load_run<T, V, NT>(pj, i, pv);

@@ -125,6 +125,7 @@ struct TmpDev {
     void *p = nullptr;
     explicit TmpDev(size_t bytes)
     {
+        bytes = (bytes + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
         const bool keep = bytes <= kTmpKept && !g_ctx.tmp_used;
         if (keep && bytes <= g_ctx.tmp_bytes) p = g_ctx.tmp;
         else if (sync()) {
@@ -1233,40 +1234,88 @@ extern "C" void HIP_MultiVecDestroy(void ***mv)
 // the caller's row order of a multivector: that of the matrix it was created from
 static const int *mv_perm(const MV *m) { return (m->mat && m->mat->perm_h) ? m->mat->perm_h : nullptr; }
 
+// Columns ordered and converted here, as many per copy as fit 1 MiB with their
+// padding rows (a copy costs about 11 us whatever its size up to there)
+template <typename T>
+static int cols_per_copy(const MV *m, int ncols)
+{
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ncols, ((int64_t)1 << 20) / (m->ld * (int64_t)sizeof(T))));
+}
+
 template <typename T>
 static void host_to_dev_cols(MV *m, int start, int ncols, const double *host, int ldh)
 {
-    const int64_t n = m->n;
-    std::vector<T> buf((size_t)n);
-    T *__restrict__ b = buf.data();
+    const int64_t n = m->n, ld = m->ld;
+    const int some = cols_per_copy<T>(m, ncols);
+    std::vector<T> buf((size_t)(some * ld), T(0));
     const int *perm = mv_perm(m);
-    for (int j = 0; j < ncols && !failed(); j++) {
-        const double *hc = host + (size_t)j * ldh;
-        if (perm)
-            for (int64_t i = 0; i < n; i++) b[i] = (T)hc[perm[i]];
-        else
-            for (int64_t i = 0; i < n; i++) b[i] = (T)hc[i];
-        check(hipMemcpy(col_ptr(m, start + j), buf.data(), sizeof(T) * m->n, hipMemcpyHostToDevice), "H2D column");
+    for (int c = 0; c < ncols && !failed(); c += some) {
+        const int k = std::min(some, ncols - c);
+        for (int j = 0; j < k; j++) {
+            const double *hc = host + (size_t)(c + j) * ldh;
+            T *__restrict__ b = buf.data() + j * ld;
+            if (perm)
+                for (int64_t i = 0; i < n; i++) b[i] = (T)hc[perm[i]];
+            else
+                for (int64_t i = 0; i < n; i++) b[i] = (T)hc[i];
+        }
+        check(hipMemcpy(col_ptr(m, start + c), buf.data(), sizeof(T) * ((k - 1) * ld + n), hipMemcpyHostToDevice),
+              "H2D columns");
+    }
+}
+
+template <typename T>
+static void dev_to_host_cols(MV *m, int start, int ncols, double *host, int ldh)
+{
+    const int64_t n = m->n, ld = m->ld;
+    const int some = cols_per_copy<T>(m, ncols);
+    std::vector<T> buf((size_t)(some * ld));
+    const int *perm = mv_perm(m);
+    for (int c = 0; c < ncols; c += some) {
+        const int k = std::min(some, ncols - c);
+        if (failed() || !check(hipMemcpy(buf.data(), col_ptr(m, start + c), sizeof(T) * ((k - 1) * ld + n),
+                                         hipMemcpyDeviceToHost),
+                               "D2H columns"))
+            return;
+        for (int j = 0; j < k; j++) {
+            const T *b = buf.data() + j * ld;
+            double *__restrict__ hc = host + (size_t)(c + j) * ldh;
+            if (perm)
+                for (int64_t i = 0; i < n; i++) hc[perm[i]] = b[i];
+            else
+                for (int64_t i = 0; i < n; i++) hc[i] = b[i];
+        }
     }
 }
 
 static const int *mv_perm_d(const MV *m) { return mv_perm(m) ? mat_perm(m->mat) : nullptr; }
 
 // Whether host columns go through the device.  A launch and its wait, 12 us, and
-// in FP32 twice the bytes on the link stand against ordering and converting one
-// column after the other here (us, here / through the device):
-//   ordered FP64, 16,384 rows: 1 column up 16 / 27, 4 columns up 62 / 61 and down
-//   71 / 62; 90,000 rows: 1 column up 54 / 47; 400 rows: 16 columns up 184 / 159, 8
-//   columns down 94 / 69; 4,096 rows: 8 columns up 79 / 93, down 80 / 82
-//   ordered FP32, 16,384 rows: 8 columns up 108 / 110; 40,000: 4 up 84 / 79
-//   unordered FP32, 262,144 rows: 2 columns up 142 / 150, 4 up 279 / 262, 8 down
-//   725 / 903, 32 down 3974 / 3707
+// in FP32 twice the bytes on the link stand against ordering and converting them
+// here (us, here / through the device):
+//   ordered FP64, 16,384 rows: 1 column up 16 / 26, 4 columns up 42 / 38 and down
+//   48 / 42, 32 down 340 / 239; 90,000 rows: 1 column up 55 / 43
+//   ordered FP32, 16,384 rows: 8 columns up 55 / 66, 16 up 113 / 94, 32 down 232 /
+//   242; 90,000: 2 up 76 / 73, 8 down 323 / 301
+//   unordered FP32, 262,144 rows: 2 columns up 141 / 139, 4 up 281 / 256, 16 down
+//   1799 / 1856, 32 down 3919 / 3718
 static bool through_device(const MV *m, int ncols, bool upload)
 {
     const double entries = (double)m->n * ncols;
     const bool f64 = m->prec == GCGE_HIP_FP64;
-    if (mv_perm(m)) return ncols >= (upload ? 16 : 8) || entries >= (f64 ? 6e4 : 1.6e5);
-    return !f64 && entries >= (upload ? 1e6 : 4e6);
+    if (mv_perm(m)) return entries >= (f64 ? 4.5e4 : upload ? 1.6e5 : 3.2e5);
+    return !f64 && entries >= (upload ? 1e6 : 6e6);
+}
+
+// ncols columns of n rows.  Short ones in one piece where they lie so: the 2-D copy
+// is a copy per column of about 9 us (32 columns of 400 rows down 235 us, 25 in one
+// piece); from 64 Ki rows on it is the faster one (16 of 110,592 rows 687, 796).
+static bool copy_columns(double *dst, int64_t ldd, const double *src, int64_t lds, int64_t n, int ncols,
+                         hipMemcpyKind kind)
+{
+    if (n < 65536 && ldd == n && lds == n) return check(hipMemcpy(dst, src, sizeof(double) * n * ncols, kind), "columns");
+    return check(hipMemcpy2D(dst, sizeof(double) * ldd, src, sizeof(double) * lds, sizeof(double) * n, ncols, kind),
+                 "columns 2D");
 }
 
 // Calls f(stage, c, k) for the columns c .. c + k - 1 of ncols, a few at a time
@@ -1295,10 +1344,7 @@ extern "C" GCGE_INT HIP_MultiVecSetFromHost(void **mv, GCGE_INT start, GCGE_INT 
     if (!sync()) return g_err;
     if (mv_perm(m) || m->prec != GCGE_HIP_FP64) {
         if (through_device(m, ncols, true) && staged_columns_through(m, start, ncols, [&](double *stage, int c, int k) {
-                if (!check(hipMemcpy2D(stage, sizeof(double) * m->n, host + (size_t)c * ldh, sizeof(double) * ldh,
-                                       sizeof(double) * m->n, k, hipMemcpyHostToDevice),
-                           "H2D 2D"))
-                    return;
+                if (!copy_columns(stage, m->n, host + (size_t)c * ldh, ldh, m->n, k, hipMemcpyHostToDevice)) return;
                 launch_rows_in(m->prec, m->n, stage, m->n, mv_perm_d(m), col_ptr(m, start + c), m->ld, k);
                 sync();
             }))
@@ -1332,10 +1378,7 @@ extern "C" GCGE_INT HIP_MultiVecGetToHost(void **mv, GCGE_INT start, GCGE_INT nc
     if (through_device(m, ncols, false) &&
         staged_columns_through(m, start, ncols, [&](double *stage, int c, int k) {
             launch_rows_out(m->prec, m->n, stage, m->n, mv_perm_d(m), col_ptr(m, start + c), m->ld, k);
-            if (sync())
-                check(hipMemcpy2D(host + (size_t)c * ldh, sizeof(double) * ldh, stage, sizeof(double) * m->n,
-                                  sizeof(double) * m->n, k, hipMemcpyDeviceToHost),
-                      "D2H 2D");
+            if (sync()) copy_columns(host + (size_t)c * ldh, ldh, stage, m->n, m->n, k, hipMemcpyDeviceToHost);
         }))
         return g_err;
     if (m->prec == GCGE_HIP_FP64 && !perm) {
@@ -1343,26 +1386,9 @@ extern "C" GCGE_INT HIP_MultiVecGetToHost(void **mv, GCGE_INT start, GCGE_INT nc
                           sizeof(double) * m->n, ncols, hipMemcpyDeviceToHost),
               "D2H 2D");
     } else if (m->prec == GCGE_HIP_FP64) {
-        std::vector<double> buf((size_t)m->n);
-        for (int j = 0; j < ncols && !failed(); j++) {
-            if (!check(hipMemcpy(buf.data(), col_ptr(m, start + j), sizeof(double) * m->n, hipMemcpyDeviceToHost),
-                       "D2H column"))
-                break;
-            double *hc = host + (size_t)j * ldh;
-            for (int64_t i = 0; i < m->n; i++) hc[perm[i]] = buf[i];
-        }
+        dev_to_host_cols<double>(m, start, ncols, host, ldh);
     } else {
-        std::vector<float> buf((size_t)m->n);
-        for (int j = 0; j < ncols && !failed(); j++) {
-            if (!check(hipMemcpy(buf.data(), col_ptr(m, start + j), sizeof(float) * m->n, hipMemcpyDeviceToHost),
-                       "D2H column"))
-                break;
-            double *hc = host + (size_t)j * ldh;
-            if (perm)
-                for (int64_t i = 0; i < m->n; i++) hc[perm[i]] = buf[i];
-            else
-                for (int64_t i = 0; i < m->n; i++) hc[i] = buf[i];
-        }
+        dev_to_host_cols<float>(m, start, ncols, host, ldh);
     }
     return g_err;
 }

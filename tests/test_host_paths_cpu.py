@@ -228,10 +228,10 @@ n, g = M.shape[0], np.random.default_rng(0)
 plain, ordered = Matrix(M), Matrix(M, order=g.permutation(n).astype(np.int32))
 # matrix, precision, columns, kernels of an upload and a download
 UP, DOWN = ["k_rows_in"], ["k_rows_out"]
-for A, prec, k, up, down in ((ordered, F64, 1, [], []), (ordered, F64, 3, [], []), (ordered, F64, 4, UP, DOWN),
-                             (ordered, F32, 7, [], []), (ordered, F32, 9, [], DOWN), (ordered, F32, 10, UP, DOWN),
+for A, prec, k, up, down in ((ordered, F64, 1, [], []), (ordered, F64, 2, [], []), (ordered, F64, 3, UP, DOWN),
+                             (ordered, F32, 9, [], []), (ordered, F32, 10, UP, []), (ordered, F32, 20, UP, DOWN),
                              (plain, F32, 1, [], []), (plain, F32, 61, [], []), (plain, F32, 62, UP, []),
-                             (plain, F32, 244, UP, []), (plain, F32, 245, UP, DOWN), (plain, F64, 100, [], [])):
+                             (plain, F32, 366, UP, []), (plain, F32, 367, UP, DOWN), (plain, F64, 100, [], [])):
     x = MultiVec(A, k, prec)
     X = np.asfortranarray(g.standard_normal((n, k)))
     assert launched(lambda: x.set(X)) == up, (prec, k)

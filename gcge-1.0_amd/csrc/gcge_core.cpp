@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "gcge.h"
+#include "stream_slots.h"
 
 // error latch of the library (hip_backend.cpp): read by GCGE_HIP_GetLastError
 namespace gh {
@@ -938,6 +939,9 @@ void bcg(void *A, void **RHS, void **V, int x_start, int x_length, GCGE_OPS *ops
 {
     if (x_length <= 0) return;
     const bool pre = para->bcg_precond != 0;
+    // between these calls come only calls that queue their work, and a search
+    // update comes last: whoever reads columns elsewhere has to wait for that
+    const gh::StreamSlots slots = gh::stream_slots(ops);
     std::vector<double> e2(pre ? x_length : 0);
     double *rho1 = dtmp, *rho2 = rho1 + x_length, *error = rho2 + x_length;
     double *last_error = error + x_length, *ptw = last_error + x_length;
@@ -989,20 +993,20 @@ void bcg(void *A, void **RHS, void **V, int x_start, int x_length, GCGE_OPS *ops
             if (pre) ops->BlockPCGSearchUpdate(A, V, x_start, CG_P, RHS, na_prev, na, alpha.data(), b.data(), ops);
             else ops->BlockCGSearchUpdate(V, x_start, CG_P, RHS, na_prev, na, alpha.data(), b.data(), ops);
         }
-        ops->MatDotMultiVecInnerProdDiag(A, CG_P, CG_W, ms, me, ptw, ops);
+        slots.MatDotMultiVecInnerProdDiag(A, CG_P, CG_W, ms, me, ptw, ops);
         for (int id = 0; id < na; id++) {
             alpha[id] = rho2[id] / ptw[id];
             rho1[id] = rho2[id];
         }
         if (pre) {
             std::vector<double> rz(na);
-            ops->BlockPCGResidualUpdate(A, CG_W, RHS, na, alpha.data(), rz.data(), rr.data(), ops);
+            slots.BlockPCGResidualUpdate(A, CG_W, RHS, na, alpha.data(), rz.data(), rr.data(), ops);
             for (int id = 0; id < na; id++) {
                 rho2[id] = rz[id];
                 e2[id] = rr[id];
             }
         } else {
-            ops->BlockCGResidualUpdate(CG_W, RHS, na, alpha.data(), rr.data(), ops);
+            slots.BlockCGResidualUpdate(CG_W, RHS, na, alpha.data(), rr.data(), ops);
             for (int id = 0; id < na; id++) rho2[id] = rr[id];
         }
         na_prev = na;

@@ -24,6 +24,7 @@
 
 #include "gcge_app_hip.h"
 #include "hip_common.h"
+#include "stream_slots.h"
 
 namespace gh {
 void launch_rowidx(HIP_MAT *A);
@@ -1748,6 +1749,7 @@ void s_MultiVecLinearCombAxpby(void **x, void **y, GCGE_INT *start, GCGE_INT *en
     lincomb_impl(x, y, start, end, a, lda, alpha, beta, "MultiVecLinearCombAxpby");
 }
 
+template <Seen seen>
 void s_MatDotMultiVecInnerProdDiag(void *mat, void **x, void **y, GCGE_INT *start, GCGE_INT *end, GCGE_DOUBLE *out,
                                    GCGE_OPS *)
 {
@@ -1758,7 +1760,8 @@ void s_MatDotMultiVecInnerProdDiag(void *mat, void **x, void **y, GCGE_INT *star
         !same_rows(mx, my, "MatDotMultiVecInnerProdDiag") || !same_prec(mx, my, "MatDotMultiVecInnerProdDiag") ||
         !mat_ok((HIP_MAT *)mat, mx, "MatDotMultiVecInnerProdDiag"))
         return;
-    if (!spmm_dot(mx->prec, (HIP_MAT *)mat, col_ptr(mx, start[0]), mx->ld, col_ptr(my, start[1]), my->ld, k, out))
+    if (!spmm_dot(mx->prec, (HIP_MAT *)mat, col_ptr(mx, start[0]), mx->ld, col_ptr(my, start[1]), my->ld, k, out,
+                  seen))
         for (int j = 0; j < k; j++) out[j] = NAN;
 }
 
@@ -1777,16 +1780,18 @@ void s_BlockCGUpdate(void **x, GCGE_INT sx, void **p, void **w, void **r, GCGE_I
         for (int j = 0; j < k; j++) rr[j] = NAN;
 }
 
+template <Seen seen>
 void s_BlockCGResidualUpdate(void **w, void **r, GCGE_INT k, const GCGE_DOUBLE *alpha, GCGE_DOUBLE *rr, GCGE_OPS *)
 {
     MV *mw = as_mv(w), *mr = as_mv(r);
     if (!range_ok(mw, 0, k, "BlockCGResidualUpdate") || !range_ok(mr, 0, k, "BlockCGResidualUpdate") ||
         !same_rows(mw, mr, "BlockCGResidualUpdate") || !same_prec(mw, mr, "BlockCGResidualUpdate"))
         return;
-    if (!cg_resid(mr->prec, mr->n, mw->data, mw->ld, mr->data, mr->ld, k, alpha, rr))
+    if (!cg_resid(mr->prec, mr->n, mw->data, mw->ld, mr->data, mr->ld, k, alpha, rr, seen))
         for (int j = 0; j < k; j++) rr[j] = NAN;
 }
 
+template <Seen seen>
 void s_BlockPCGResidualUpdate(void *Mat, void **w, void **r, GCGE_INT k, const GCGE_DOUBLE *alpha, GCGE_DOUBLE *rz,
                               GCGE_DOUBLE *rr, GCGE_OPS *)
 {
@@ -1797,7 +1802,7 @@ void s_BlockPCGResidualUpdate(void *Mat, void **w, void **r, GCGE_INT k, const G
         !mat_ok(A, mr, who))
         return;
     const void *dinv = mat_dinv(A, mr->prec);
-    if (!dinv || !pcg_resid(mr->prec, mr->n, mw->data, mw->ld, mr->data, mr->ld, dinv, k, alpha, rz, rr))
+    if (!dinv || !pcg_resid(mr->prec, mr->n, mw->data, mw->ld, mr->data, mr->ld, dinv, k, alpha, rz, rr, seen))
         for (int j = 0; j < k; j++) rz[j] = rr[j] = NAN;
 }
 
@@ -1920,6 +1925,18 @@ GCGE_INT s_MultiVecNumRows(void **x)
 // dense slots live in the host core (gcge_dense.cpp)
 extern "C" void GCGE_SetDenseOps(GCGE_OPS *ops);
 
+gh::StreamSlots gh::stream_slots(const GCGE_OPS *ops)
+{
+    StreamSlots r{ops->MatDotMultiVecInnerProdDiag, ops->BlockCGResidualUpdate, ops->BlockPCGResidualUpdate};
+    if (r.MatDotMultiVecInnerProdDiag == s_MatDotMultiVecInnerProdDiag<Seen::everywhere>)
+        r.MatDotMultiVecInnerProdDiag = s_MatDotMultiVecInnerProdDiag<Seen::in_stream>;
+    if (r.BlockCGResidualUpdate == s_BlockCGResidualUpdate<Seen::everywhere>)
+        r.BlockCGResidualUpdate = s_BlockCGResidualUpdate<Seen::in_stream>;
+    if (r.BlockPCGResidualUpdate == s_BlockPCGResidualUpdate<Seen::everywhere>)
+        r.BlockPCGResidualUpdate = s_BlockPCGResidualUpdate<Seen::in_stream>;
+    return r;
+}
+
 extern "C" void GCGE_HIP_SetOps(GCGE_OPS *ops)
 {
     ensure_ctx();
@@ -1949,11 +1966,11 @@ extern "C" void GCGE_HIP_SetOps(GCGE_OPS *ops)
     ops->MultiVecAxpbyDiag = s_MultiVecAxpbyDiag;
     ops->MultiVecInnerProdDiag = s_MultiVecInnerProdDiag;
     ops->MultiVecLinearCombAxpby = s_MultiVecLinearCombAxpby;
-    ops->MatDotMultiVecInnerProdDiag = s_MatDotMultiVecInnerProdDiag;
+    ops->MatDotMultiVecInnerProdDiag = s_MatDotMultiVecInnerProdDiag<Seen::everywhere>;
     ops->BlockCGUpdate = s_BlockCGUpdate;
-    ops->BlockCGResidualUpdate = s_BlockCGResidualUpdate;
+    ops->BlockCGResidualUpdate = s_BlockCGResidualUpdate<Seen::everywhere>;
     ops->BlockCGSearchUpdate = s_BlockCGSearchUpdate;
-    ops->BlockPCGResidualUpdate = s_BlockPCGResidualUpdate;
+    ops->BlockPCGResidualUpdate = s_BlockPCGResidualUpdate<Seen::everywhere>;
     ops->BlockPCGSearchUpdate = s_BlockPCGSearchUpdate;
     ops->MultiVecResidualNorms = s_MultiVecResidualNorms;
     ops->MultiVecGather = s_MultiVecGather;

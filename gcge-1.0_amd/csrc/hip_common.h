@@ -220,9 +220,12 @@ void launch_zero_rows(int prec, void *x, int64_t ldx, int64_t n, int k, const un
 // Y_j = A X_j (xidx: optional gather of X columns, k <= kMaxCols when given)
 void launch_spmm(int prec, HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy, int k,
                  const int *xidx);
+// Where the columns that a launch writes beside its sums are complete when the
+// host has the sums: for later launches of the stream, or for other streams too
+enum class Seen { in_stream, everywhere };
 // Y_j = A X_j and out_j = <X_j, Y_j>
 bool spmm_dot(int prec, HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy, int k,
-              double *out);
+              double *out, Seen seen);
 // rnorm/xnorm/bxnorm of A x_j - lambda_j B x_j, x_j = X(:, idx[j])
 bool residual_norms(int prec, HIP_MAT *A, HIP_MAT *B, const void *X, int64_t ldx, const int *idx,
                     int k, const double *lambda, double *rnorm, double *xnorm, double *bxnorm);
@@ -231,10 +234,10 @@ bool cg_update(int prec, int64_t n, void *x, int64_t ldx, const void *p, int64_t
                int64_t ldw, void *r, int64_t ldr, int k, const double *alpha, double *rr);
 // r_j -= alpha_j w_j ; rr_j = <r_j, r_j>
 bool cg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t ldr, int k, const double *alpha,
-              double *rr);
+              double *rr, Seen seen);
 // r_j -= alpha_j w_j ; rz_j = <r_j, dinv .* r_j> ; rr_j = <r_j, r_j>
 bool pcg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t ldr, const void *dinv, int k,
-               const double *alpha, double *rz, double *rr);
+               const double *alpha, double *rz, double *rr, Seen seen);
 // dinv64[i] = 1 / a_ii (1 where a_ii is 0 or absent), dinv32 its FP32 rounding
 void launch_diag_inv(HIP_MAT *A);
 // x_j += alpha_j p_j (j < kx), then p_j = r_j + beta_j p_j (j < kp); with

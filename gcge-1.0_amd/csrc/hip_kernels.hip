@@ -1584,15 +1584,16 @@ void launch_axpby(int prec, int64_t n, const void *x, int64_t ldx, void *y, int6
 // less and its wait.  us a call, FP64 dots of 1 column of 16,384 rows (64
 // partial sums) 14.6 -> 11.1, of 20 columns (1280) 15.9 -> 14.7, of 8 columns of
 // 90,000 rows (2048) 15.8 -> 15.6, where the line is drawn.  Not where the launch
-// also `writes` columns: the host would have the sums while stores of the same
-// launch may still lie in one XCD's L2, out of sight of other streams.  The
-// launch that reduces comes after those stores (residual update of 1 column of
+// also writes columns that are to be seen everywhere when the call returns: the
+// host would have the sums while stores of the same launch may still lie in one
+// XCD's L2, out of sight of other streams.  The launch that reduces comes after
+// those stores (residual update of 1 column of
 // 16,384 rows 16.6 us, 12.6 without; of 20 columns 18.1 and 16.0; with a
 // system-scope release by every workgroup instead 29).
-static double *partial_buf(size_t rows, size_t nb, bool writes)
+static double *partial_buf(size_t rows, size_t nb, Seen seen)
 {
-    return !writes && rows * nb <= kHostPartials ? host_partials(rows * nb)
-                                                 : (double *)scratch(sizeof(double) * rows * nb);
+    return seen == Seen::in_stream && rows * nb <= kHostPartials ? host_partials(rows * nb)
+                                                                 : (double *)scratch(sizeof(double) * rows * nb);
 }
 
 // sum_row and block_sum on the host
@@ -1646,7 +1647,7 @@ bool dots(int prec, int64_t n, const void *x, int64_t ldx, const void *y, int64_
     if (k <= 0) return true;
     if (failed()) return false;
     const int nb = dots_blocks(n);
-    double *partial = partial_buf((size_t)k, nb, false);
+    double *partial = partial_buf((size_t)k, nb, Seen::in_stream);
     if (!partial) return false;
     {
         ProfScope ps(K_DOTS, 2.0 * k * (double)n * elem_size(prec), 2.0 * k * (double)n);
@@ -1732,7 +1733,7 @@ const float *mat_vals<float>(HIP_MAT *A) { return mat_val32(A); }
 // Row-major gather path (see k_spmm_rows) for kc <= kMaxCols columns.
 template <typename T, bool DOT, int G>
 static bool spmm_rows_g(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColScalars g, T *Yc, int64_t ldy,
-                        int kc, double *out)
+                        int kc, double *out, Seen seen)
 {
     const int n = A->n, kp = G < 64 ? G : ((kc + 63) / 64) * 64;
     T *Xt = (T *)row_stage(sizeof(T) * (size_t)n * kp);
@@ -1742,7 +1743,7 @@ static bool spmm_rows_g(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColS
     const int pstride = nblk + (DOT ? nlong : 0);
     double *partial = nullptr;
     if (DOT) {
-        partial = partial_buf((size_t)kc, pstride, true);
+        partial = partial_buf((size_t)kc, pstride, seen);
         if (!partial) return false;
     }
     {
@@ -1762,14 +1763,14 @@ static bool spmm_rows_g(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColS
 
 template <typename T, bool DOT>
 static bool spmm_rows(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColScalars g, T *Yc, int64_t ldy,
-                      int kc, double *out)
+                      int kc, double *out, Seen seen)
 {
-    if (kc > 32) return spmm_rows_g<T, DOT, 64>(A, val, Xc, ldx, g, Yc, ldy, kc, out);
-    if (kc > 16) return spmm_rows_g<T, DOT, 32>(A, val, Xc, ldx, g, Yc, ldy, kc, out);
-    if (kc > 8) return spmm_rows_g<T, DOT, 16>(A, val, Xc, ldx, g, Yc, ldy, kc, out);
-    if (kc > 4) return spmm_rows_g<T, DOT, 8>(A, val, Xc, ldx, g, Yc, ldy, kc, out);
-    if (kc > 2) return spmm_rows_g<T, DOT, 4>(A, val, Xc, ldx, g, Yc, ldy, kc, out);
-    return spmm_rows_g<T, DOT, 2>(A, val, Xc, ldx, g, Yc, ldy, kc, out);
+    if (kc > 32) return spmm_rows_g<T, DOT, 64>(A, val, Xc, ldx, g, Yc, ldy, kc, out, seen);
+    if (kc > 16) return spmm_rows_g<T, DOT, 32>(A, val, Xc, ldx, g, Yc, ldy, kc, out, seen);
+    if (kc > 8) return spmm_rows_g<T, DOT, 16>(A, val, Xc, ldx, g, Yc, ldy, kc, out, seen);
+    if (kc > 4) return spmm_rows_g<T, DOT, 8>(A, val, Xc, ldx, g, Yc, ldy, kc, out, seen);
+    if (kc > 2) return spmm_rows_g<T, DOT, 4>(A, val, Xc, ldx, g, Yc, ldy, kc, out, seen);
+    return spmm_rows_g<T, DOT, 2>(A, val, Xc, ldx, g, Yc, ldy, kc, out, seen);
 }
 
 // Columns per LDS pass of k_spmm_halo: 4, or GCGE_HIP_HALO_KC (1, 2, 4 or
@@ -1825,14 +1826,14 @@ static void spmm_halo_kc(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, Col
 
 template <typename T, bool DOT>
 static bool spmm_halo(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColScalars g, T *Yc, int64_t ldy,
-                      int kc, double *out)
+                      int kc, double *out, Seen seen)
 {
     const int nblk = A->halo_blocks;
     const int nlong = A->nlong, long_thr = nlong > 0 ? kLongRow : INT_MAX;
     const int pstride = nblk + (DOT ? nlong : 0);
     double *partial = nullptr;
     if (DOT) {
-        partial = partial_buf((size_t)kc, pstride, true);
+        partial = partial_buf((size_t)kc, pstride, seen);
         if (!partial) return false;
     }
     {
@@ -1856,7 +1857,7 @@ static bool spmm_halo(HIP_MAT *A, const T *val, const T *Xc, int64_t ldx, ColSca
 
 template <typename T, bool DOT>
 static bool spmm_t(HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy, int k, const int *xidx,
-                   double *out)
+                   double *out, Seen seen)
 {
     const int nblk = (A->n + kSpmmRows - 1) / kSpmmRows;
     const T *val = mat_vals<T>(A);
@@ -1867,11 +1868,11 @@ static bool spmm_t(HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy,
         const T *Xc = (const T *)X + (xidx ? 0 : (int64_t)c0 * ldx);
         T *Yc = (T *)Y + (int64_t)c0 * ldy;
         if (A->gather_rows && kc >= 2) {  // one column gathers a line per entry either way
-            if (!spmm_rows<T, DOT>(A, val, Xc, ldx, g, Yc, ldy, kc, DOT ? out + c0 : nullptr)) return false;
+            if (!spmm_rows<T, DOT>(A, val, Xc, ldx, g, Yc, ldy, kc, DOT ? out + c0 : nullptr, seen)) return false;
             continue;
         }
         if (A->halo && (sizeof(T) == 8 || A->halo_f32)) {
-            if (!spmm_halo<T, DOT>(A, val, Xc, ldx, g, Yc, ldy, kc, DOT ? out + c0 : nullptr)) return false;
+            if (!spmm_halo<T, DOT>(A, val, Xc, ldx, g, Yc, ldy, kc, DOT ? out + c0 : nullptr, seen)) return false;
             continue;
         }
         // long rows (power-law graphs) go to k_spmm_long; their dot partials
@@ -1880,7 +1881,7 @@ static bool spmm_t(HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy,
         const int pstride = nblk + (DOT ? nlong : 0);
         double *partial = nullptr;
         if (DOT) {
-            partial = partial_buf((size_t)kc, pstride, true);
+            partial = partial_buf((size_t)kc, pstride, seen);
             if (!partial) return false;
         }
         {
@@ -1911,16 +1912,16 @@ static bool spmm_t(HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy,
 void launch_spmm(int prec, HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy, int k, const int *xidx)
 {
     if (k <= 0 || failed()) return;
-    if (prec == GCGE_HIP_FP64) spmm_t<double, false>(A, X, ldx, Y, ldy, k, xidx, nullptr);
-    else spmm_t<float, false>(A, X, ldx, Y, ldy, k, xidx, nullptr);
+    if (prec == GCGE_HIP_FP64) spmm_t<double, false>(A, X, ldx, Y, ldy, k, xidx, nullptr, Seen::in_stream);
+    else spmm_t<float, false>(A, X, ldx, Y, ldy, k, xidx, nullptr, Seen::in_stream);
 }
 
-bool spmm_dot(int prec, HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy, int k, double *out)
+bool spmm_dot(int prec, HIP_MAT *A, const void *X, int64_t ldx, void *Y, int64_t ldy, int k, double *out, Seen seen)
 {
     if (k <= 0) return true;
     if (failed()) return false;
-    if (prec == GCGE_HIP_FP64) return spmm_t<double, true>(A, X, ldx, Y, ldy, k, nullptr, out);
-    return spmm_t<float, true>(A, X, ldx, Y, ldy, k, nullptr, out);
+    if (prec == GCGE_HIP_FP64) return spmm_t<double, true>(A, X, ldx, Y, ldy, k, nullptr, out, seen);
+    return spmm_t<float, true>(A, X, ldx, Y, ldy, k, nullptr, out, seen);
 }
 
 // Residual sums of kc <= kMaxCols columns on the row-major gather path;
@@ -1935,7 +1936,7 @@ static bool residual_rows_g(HIP_MAT *A, HIP_MAT *B, const T *X, int64_t ldx, Col
     const int RWG = rows_per_wg(G);
     const int nblk = (n + RWG - 1) / RWG, nlong = A->nlong, nlb = (nlong + 3) / 4;
     const int pstride = nblk + nlong;
-    double *partial = partial_buf((size_t)3 * kc, pstride, false);
+    double *partial = partial_buf((size_t)3 * kc, pstride, Seen::in_stream);
     if (!partial) return false;
     {
         ProfScope ps(K_RESIDUAL,
@@ -2042,7 +2043,7 @@ static bool residual_t(HIP_MAT *A, HIP_MAT *B, const void *X, int64_t ldx, const
             }
             continue;
         }
-        double *partial = partial_buf((size_t)3 * kc, nblk, false);
+        double *partial = partial_buf((size_t)3 * kc, nblk, Seen::in_stream);
         if (!partial) return false;
         const double rbytes = 12.0 * A->nnz + 4.0 * (A->n + 1) + (B ? 12.0 * B->nnz + 4.0 * (B->n + 1) : 0.0) +
                               (double)kc * A->n * sizeof(T);
@@ -2088,7 +2089,7 @@ bool cg_update(int prec, int64_t n, void *x, int64_t ldx, const void *p, int64_t
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars s = make_scalars(kc, alpha + c0, nullptr, nullptr);
-        double *partial = partial_buf((size_t)kc, nb, true);
+        double *partial = partial_buf((size_t)kc, nb, Seen::everywhere);
         if (!partial) return false;
         dim3 grid(nb, kc);
         {
@@ -2110,7 +2111,7 @@ bool cg_update(int prec, int64_t n, void *x, int64_t ldx, const void *p, int64_t
 }
 
 bool cg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t ldr, int k, const double *alpha,
-              double *rr)
+              double *rr, Seen seen)
 {
     if (k <= 0) return true;
     if (failed()) return false;
@@ -2118,7 +2119,7 @@ bool cg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t 
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars s = make_scalars(kc, alpha + c0, nullptr, nullptr);
-        double *partial = partial_buf((size_t)kc, nb, true);
+        double *partial = partial_buf((size_t)kc, nb, seen);
         if (!partial) return false;
         dim3 grid(nb, kc);
         {
@@ -2142,7 +2143,7 @@ bool cg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t 
 }
 
 bool pcg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t ldr, const void *dinv, int k,
-               const double *alpha, double *rz, double *rr)
+               const double *alpha, double *rz, double *rr, Seen seen)
 {
     if (k <= 0) return true;
     if (failed()) return false;
@@ -2151,7 +2152,7 @@ bool pcg_resid(int prec, int64_t n, const void *w, int64_t ldw, void *r, int64_t
     for (int c0 = 0; c0 < k; c0 += kMaxCols) {
         const int kc = std::min(kMaxCols, k - c0);
         ColScalars s = make_scalars(kc, alpha + c0, nullptr, nullptr);
-        double *partial = partial_buf((size_t)2 * kc, nb, true);
+        double *partial = partial_buf((size_t)2 * kc, nb, seen);
         if (!partial) return false;
         dim3 grid(nb, kc);
         {
